@@ -9,8 +9,8 @@
 // column accumulator and no carry has to be propagated until the column is
 // finished (18 products of < 2^60 plus a 2^35 carry stay below 2^64).  On
 // gfx950 the 32x32->64 mad issues at full rate, so the instruction count of
-// the multiply is what matters; this layout needs 162 mads and 42 other ops
-// (a square 126 and 50) against ~560 instructions for a compiler-lowered
+// the multiply is what matters; this layout needs 169 mads and 22 other ops
+// (a square 133 and 30) against ~560 instructions for a compiler-lowered
 // 8x32-bit CIOS.
 //
 // At the memory boundary elements are the reference's 32-byte little-endian
@@ -25,8 +25,7 @@
 
 #if defined(__HIPCC__)
 #include <hip/hip_runtime.h>
-#include <utility>
-#include "mad_chain.hpp"
+#include "mont_asm.hpp"
 #define ZK_HD __host__ __device__ __forceinline__
 #else
 #define ZK_HD static inline
@@ -53,6 +52,8 @@ struct FqP {
   static constexpr uint32_t MOD8[9] = {0x03e7ea38u, 0x082305b6u, 0x03951a78u, 0x16a91687u, 0x0c2ecbc0u,
                                        0x16da0605u, 0x05370a08u, 0x12e131a0u, 0x01832273u};
   static constexpr uint32_t INV = 0x04866389u;  // -q^-1 mod 2^29
+  static constexpr uint32_t EDIG[9] = {0x02e38790u, 0x0d1e68dcu, 0x148e556bu, 0x10c54699u, 0x0f93f7a8u,
+                                       0x02d6db27u, 0x05f64f9au, 0x1010b67bu, 0x015995e9u};  // (q k + 1) / 2^29, k = -q^-1 mod 2^32
   static constexpr uint32_t ONE[9] = {0x157ccc21u, 0x141c2758u, 0x185230d3u, 0x014c0419u, 0x0aa36fb9u,
                                       0x1d4240ceu, 0x11d54c07u, 0x052ac7a8u, 0x000dc836u};  // 2^261 mod q
   static constexpr uint32_t R2[9] = {0x059bac10u, 0x0d1503a3u, 0x018016b8u, 0x10ab0ca8u, 0x02632639u,
@@ -79,6 +80,8 @@ struct FrP {
   static constexpr uint32_t MOD8[9] = {0x00000008u, 0x187d64fcu, 0x12e12287u, 0x1e84879bu, 0x0c2e9419u,
                                        0x16da0605u, 0x05370a08u, 0x12e131a0u, 0x01832273u};
   static constexpr uint32_t INV = 0x0fffffffu;  // -r^-1 mod 2^29
+  static constexpr uint32_t EDIG[9] = {0x08f05368u, 0x1a996a5bu, 0x13e27f6bu, 0x15166c9eu, 0x1e906a17u,
+                                       0x04c58463u, 0x16877334u, 0x0b82ba37u, 0x016af04cu};  // (r k + 1) / 2^29, k = -r^-1 mod 2^32
   static constexpr uint32_t ONE[9] = {0x0fffff57u, 0x1ea70ab4u, 0x052c068bu, 0x17504f49u, 0x0aa8075bu,
                                       0x1d4240ceu, 0x11d54c07u, 0x052ac7a8u, 0x000dc836u};  // 2^261 mod r
   static constexpr uint32_t R2[9] = {0x05b69bd4u, 0x06170a5au, 0x020cddceu, 0x1db6310bu, 0x0e54d0ffu,
@@ -118,177 +121,114 @@ ZK_HD fe<P> fe_one() {
   return fe_const<P>(P::ONE);
 }
 
-#if defined(__HIP_DEVICE_COMPILE__)
-// Device columns of the Montgomery products below: the same terms in the
-// same columns, each column one serial multiply-add chain seeded with the
-// incoming carry (mad_chain.hpp).  Every partial sum is a prefix of the
-// column's sum, so the bounds stated for the products hold at every step.
-//
-// Reduction part of column K: q_i m_(K-i) for i < K, 1 <= K - i <= 8, then
-// the column's own quotient (K < 9) or output limb (K >= 9), then the carry.
-template <class P, int K>
-__device__ __forceinline__ void mont_col_reduce(uint64_t& acc, uint32_t* q, fe<P>& r) {
-  constexpr int rlo = K > NL - 1 ? K - (NL - 1) : 0;
-  constexpr int nr = (K < NL ? K : NL) - rlo;
-  if constexpr (nr > 0) {
-    uint32_t x[nr], y[nr];
-#pragma unroll
-    for (int u = 0; u < nr; u++) {
-      x[u] = q[rlo + u];
-      y[u] = P::MOD[K - rlo - u];
-    }
-    mad_vs<nr>(acc, x, y);
-  }
-  if constexpr (K < NL) {
-    q[K] = ((uint32_t)acc * P::INV) & LMASK;
-    const uint32_t x[1] = {q[K]}, y[1] = {P::MOD[0]};
-    mad_vs<1>(acc, x, y);
-  } else {
-    r.l[K - NL] = (uint32_t)acc & LMASK;
-  }
-  acc >>= 29;
-}
+// Montgomery products sum_t a[t] b[t] 2^-261 mod m in column (product-scanning)
+// order, the reduction interleaved.  acc holds one column of 29 bits plus what
+// the columns below carried into it.
+//   Columns 0..6: the digit is the column's low 32 bits as they are.  With
+//   k = -m^-1 mod 2^32, q (m k) clears them, and q (m k + 1) = q 2^29 EDIG adds
+//   q EDIG_j to column K + 1 + j; what is left of the column, its high 32
+//   bits, goes on as 8 hi (2^32 = 8 * 2^29).  No multiply and no mask for the
+//   digit.  Digit 6 counts at most 2^(32 + 174) m k < 2^(238) m in the sum that
+//   is divided by 2^261, so these digits add less than m / 2^22 to the result.
+//   Columns 7, 8: the ordinary digit q = acc (-m^-1) mod 2^29 with multiplier
+//   m; digit 8 adds less than m to the result.
+//   Columns 9..16: output limbs.
+// Columns stay below 2^64: the operands' products (limbs below 2^29: up to
+// 9 N of 2^58; one operand's or the square's limbs may be below 2^30), the
+// digits' 2^32 EDIG_j (column 8 has the most, 22.8 * 2^58 for q and 34.3 *
+// 2^58 for r), two digit products below 2^58 and the carry: for q at most
+// 36 + 22.8 + 2.1 (four products, or one square of limbs below 2^30), for r
+// 18 + 34.3 + 2.1, in units of 2^58 of 64 (mont_columns_fit).
+constexpr int MONT_ND = 7;  // columns with a 32-bit digit
 
-// Column K of sum_t a[t]*b[t]: the products a[t]_i b[t]_(K-i), then the reduction.
-template <class P, int N, int K>
-__device__ __forceinline__ void mont_col(uint64_t& acc, const fe<P>* a, const fe<P>* b, uint32_t* q, fe<P>& r) {
-  constexpr int ilo = K < NL ? 0 : K - NL + 1;
-  constexpr int np = (K < NL ? K : NL - 1) - ilo + 1;
-  uint32_t x[N * np], y[N * np];
-#pragma unroll
-  for (int t = 0; t < N; t++) {
-#pragma unroll
-    for (int u = 0; u < np; u++) {
-      x[t * np + u] = a[t].l[ilo + u];
-      y[t * np + u] = b[t].l[K - ilo - u];
-    }
+template <class P>
+constexpr bool mont_columns_fit(int products_2p58) {
+  bool ok = true;
+  for (int K = 0; K < 2 * NL - 1; K++) {
+    unsigned __int128 s = (unsigned __int128)products_2p58 << 58;
+    for (int i = 0; i < MONT_ND && i < K; i++)
+      if (K - 1 - i < NL) s += (unsigned __int128)0xffffffffu * P::EDIG[K - 1 - i];
+    s += (unsigned __int128)2 << 58;  // digits 7 and 8
+    s += (unsigned __int128)1 << 36;  // carry
+    ok = ok && (s >> 64) == 0;
   }
-  mad_vv<N * np>(acc, x, y);
-  mont_col_reduce<P, K>(acc, q, r);
+  return ok;
 }
+static_assert(mont_columns_fit<FqP>(36), "Fq column accumulator bound");
+static_assert(mont_columns_fit<FrP>(18), "Fr column accumulator bound");
 
-template <class P, int N, int... K>
-__device__ __forceinline__ fe<P> mont_product(const fe<P>* a, const fe<P>* b, std::integer_sequence<int, K...>) {
+#if !defined(__HIP_DEVICE_COMPILE__)
+// cols(K): the sum of the operands' products of column K.
+template <class P, class Cols>
+static inline fe<P> mont_columns(Cols&& cols) {
   uint32_t q[NL];
   fe<P> r;
   uint64_t acc = 0;
-  (mont_col<P, N, K>(acc, a, b, q, r), ...);
-  r.l[NL - 1] = (uint32_t)acc;
-  return r;
-}
-
-// Column K of a^2: cross products a_i (2 a_j), i < j, and the square of
-// a_(K/2) for even K.  With limbs below 2^30 the largest column (K = 8: four
-// cross products below 2^61, a square below 2^60, nine reduction products
-// below 2^58, a carry below 2^35) stays below 1.41 * 2^63.
-template <class P, int K>
-__device__ __forceinline__ void sqr_col(uint64_t& acc, const fe<P>& a, const uint32_t* a2, uint32_t* q, fe<P>& r) {
-  constexpr int ilo = K < NL ? 0 : K - NL + 1;
-  constexpr int ihi = K >= 1 ? (K - 1) / 2 : -1;  // i < K - i
-  constexpr int nc = ihi >= ilo ? ihi - ilo + 1 : 0;
-  constexpr int nd = (K % 2 == 0) ? 1 : 0;
-  uint32_t x[nc + nd], y[nc + nd];
-#pragma unroll
-  for (int u = 0; u < nc; u++) {
-    x[u] = a.l[ilo + u];
-    y[u] = a2[K - ilo - u];
+  for (int k = 0; k < 2 * NL - 1; k++) {
+    acc += cols(k);
+    for (int i = 0; i < MONT_ND && i < k; i++)
+      if (k - 1 - i < NL) acc += (uint64_t)q[i] * P::EDIG[k - 1 - i];
+    for (int i = MONT_ND; i < NL && i < k; i++)
+      if (k - i < NL) acc += (uint64_t)q[i] * P::MOD[k - i];
+    if (k < MONT_ND) {
+      q[k] = (uint32_t)acc;
+      acc = (acc >> 32) * 8;
+      continue;
+    }
+    if (k < NL) {
+      q[k] = ((uint32_t)acc * P::INV) & LMASK;
+      acc += (uint64_t)q[k] * P::MOD[0];
+    } else {
+      r.l[k - NL] = (uint32_t)acc & LMASK;
+    }
+    acc >>= 29;
   }
-  if constexpr (nd) {
-    x[nc] = a.l[K / 2];
-    y[nc] = a.l[K / 2];
-  }
-  mad_vv<nc + nd>(acc, x, y);
-  mont_col_reduce<P, K>(acc, q, r);
-}
-
-template <class P, int... K>
-__device__ __forceinline__ fe<P> mont_square(const fe<P>& a, std::integer_sequence<int, K...>) {
-  uint32_t q[NL], a2[NL];
-  fe<P> r;
-#pragma unroll
-  for (int i = 0; i < NL; i++) a2[i] = a.l[i] << 1;
-  uint64_t acc = 0;
-  (sqr_col<P, K>(acc, a, a2, q, r), ...);
   r.l[NL - 1] = (uint32_t)acc;
   return r;
 }
 #endif
 
-// Montgomery product a*b*2^-261 mod m, column (product-scanning) order with the
-// reduction interleaved per column.  Inputs: limbs < 2^30.  Output: limbs
-// < 2^29, value < a*b/2^261 + m, so below 2m for values < 8m, and also when
-// one operand is below m and the other anywhere below 2^261.
+// Montgomery product a*b*2^-261 mod m.  Inputs: limbs < 2^29, of one operand
+// < 2^30 (of both over Fq).  Output: limbs < 2^29, value < a*b/2^261 + m +
+// m/2^22, so below 2m for values < 8m, and also when one operand is below m
+// and the other anywhere below 2^261 - 2^239.
 template <class P>
 ZK_HD fe<P> fmul(const fe<P>& a, const fe<P>& b) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  return mont_product<P, 1>(&a, &b, std::make_integer_sequence<int, 2 * NL - 1>{});
-#else
-  uint32_t q[NL];
-  fe<P> r;
-  uint64_t acc = 0;
-#pragma unroll
-  for (int k = 0; k < 2 * NL - 1; k++) {
-#pragma unroll
-    for (int i = 0; i < NL; i++) {
-      const int j = k - i;
-      if (j >= 0 && j < NL) acc += (uint64_t)a.l[i] * b.l[j];
-    }
-#pragma unroll
-    for (int i = 0; i < NL; i++) {
-      const int j = k - i;
-      if (i < k && j >= 1 && j < NL) acc += (uint64_t)q[i] * P::MOD[j];
-    }
-    if (k < NL) {
-      q[k] = ((uint32_t)acc * P::INV) & LMASK;
-      acc += (uint64_t)q[k] * P::MOD[0];
-    } else {
-      r.l[k - NL] = (uint32_t)acc & LMASK;
-    }
-    acc >>= 29;
-  }
-  r.l[NL - 1] = (uint32_t)acc;
+  fe<P> r = a;  // in place when a is dead after the product
+  mont_mul_asm<P>(r.l, b.l);
   return r;
+#else
+  return mont_columns<P>([&](int k) {
+    uint64_t s = 0;
+    for (int i = k < NL ? 0 : k - NL + 1; i < NL && i <= k; i++) s += (uint64_t)a.l[i] * b.l[k - i];
+    return s;
+  });
 #endif
 }
 
-// sum_t a[t]*b[t] * 2^-261 mod m, N <= 4, with one Montgomery reduction for
-// all products.  Inputs: normalized limbs (< 2^29), values <= 4m.  Every
-// column then holds at most 9N + 9 terms below 2^58 plus a carry below 2^35,
-// which stays below 2^64, and the result is below 64m^2 / 2^261 + m < 1.4m.
+// sum_t a[t]*b[t] * 2^-261 mod q, N = 2 or 4, with one Montgomery reduction
+// for all products.  Inputs: normalized limbs (< 2^29), values <= 4q (the sum
+// of the products below 100 q^2).  The result is below 100 q^2 / 2^261 + q +
+// q/2^22 < 1.6 q.
 template <class P, int N>
 ZK_HD fe<P> fmul_sum(const fe<P> (&a)[N], const fe<P> (&b)[N]) {
-  static_assert(N >= 1 && N <= 4, "column accumulator bound");
+  static_assert(N == 2 || N == 4, "products of one reduction");
+  static_assert(mont_columns_fit<P>(9 * N), "column accumulator bound");
 #if defined(__HIP_DEVICE_COMPILE__)
-  return mont_product<P, N>(a, b, std::make_integer_sequence<int, 2 * NL - 1>{});
-#else
-  uint32_t q[NL];
-  fe<P> r;
-  uint64_t acc = 0;
-#pragma unroll
-  for (int k = 0; k < 2 * NL - 1; k++) {
-#pragma unroll
-    for (int i = 0; i < NL; i++) {
-      const int j = k - i;
-      if (j >= 0 && j < NL) {
-#pragma unroll
-        for (int t = 0; t < N; t++) acc += (uint64_t)a[t].l[i] * b[t].l[j];
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < NL; i++) {
-      const int j = k - i;
-      if (i < k && j >= 1 && j < NL) acc += (uint64_t)q[i] * P::MOD[j];
-    }
-    if (k < NL) {
-      q[k] = ((uint32_t)acc * P::INV) & LMASK;
-      acc += (uint64_t)q[k] * P::MOD[0];
-    } else {
-      r.l[k - NL] = (uint32_t)acc & LMASK;
-    }
-    acc >>= 29;
-  }
-  r.l[NL - 1] = (uint32_t)acc;
+  fe<P> r = a[0];  // in place when a[0] is dead after the products
+  if constexpr (N == 2)
+    mont_mul2_asm<P>(r.l, b[0].l, a[1].l, b[1].l);
+  else
+    mont_mul4_asm<P>(r.l, b[0].l, a[1].l, b[1].l, a[2].l, b[2].l, a[3].l, b[3].l);
   return r;
+#else
+  return mont_columns<P>([&](int k) {
+    uint64_t s = 0;
+    for (int t = 0; t < N; t++)
+      for (int i = k < NL ? 0 : k - NL + 1; i < NL && i <= k; i++) s += (uint64_t)a[t].l[i] * b[t].l[k - i];
+    return s;
+  });
 #endif
 }
 
@@ -299,40 +239,21 @@ ZK_HD fe<P> fmul2(const fe<P>& a, const fe<P>& b, const fe<P>& c, const fe<P>& e
   return fmul_sum<P, 2>(x, y);
 }
 
-// Squaring: cross products are summed once and doubled per column.
+// Squaring: every cross product once, by the doubled limb (limbs < 2^30 over
+// Fq, < 2^29 over Fr).
 template <class P>
 ZK_HD fe<P> fsqr(const fe<P>& a) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  return mont_square<P>(a, std::make_integer_sequence<int, 2 * NL - 1>{});
-#else
-  uint32_t q[NL];
   fe<P> r;
-  uint64_t acc = 0;
-#pragma unroll
-  for (int k = 0; k < 2 * NL - 1; k++) {
-    uint64_t cross = 0;
-#pragma unroll
-    for (int i = 0; i < NL; i++) {
-      const int j = k - i;
-      if (j > i && j < NL) cross += (uint64_t)a.l[i] * a.l[j];
-    }
-    acc += cross << 1;
-    if ((k & 1) == 0 && k / 2 < NL) acc += (uint64_t)a.l[k / 2] * a.l[k / 2];
-#pragma unroll
-    for (int i = 0; i < NL; i++) {
-      const int j = k - i;
-      if (i < k && j >= 1 && j < NL) acc += (uint64_t)q[i] * P::MOD[j];
-    }
-    if (k < NL) {
-      q[k] = ((uint32_t)acc * P::INV) & LMASK;
-      acc += (uint64_t)q[k] * P::MOD[0];
-    } else {
-      r.l[k - NL] = (uint32_t)acc & LMASK;
-    }
-    acc >>= 29;
-  }
-  r.l[NL - 1] = (uint32_t)acc;
+  mont_sqr_asm<P>(r.l, a.l);
   return r;
+#else
+  return mont_columns<P>([&](int k) {
+    uint64_t s = 0;
+    for (int i = k < NL ? 0 : k - NL + 1; 2 * i < k; i++) s += (uint64_t)a.l[i] * (2 * a.l[k - i]);
+    if (k % 2 == 0) s += (uint64_t)a.l[k / 2] * a.l[k / 2];
+    return s;
+  });
 #endif
 }
 

@@ -317,3 +317,36 @@ def test_xyzz_formulas(fh, g2flag):
     assert dec(xyzz_call(fh, g2flag, 0, enc(rng, None, rz()), affine_words(a))) == a
     assert dec(xyzz_call(fh, g2flag, 1, enc(rng, None, rz()), enc(rng, a, rz()))) == a
     assert dec(xyzz_call(fh, g2flag, 1, enc(rng, a, rz()), enc(rng, None, rz()))) == a
+
+
+def limbs_value(rng, hi):
+    """Nine limbs below `hi`, not normalized: all at the maximum, all but one
+    zero, or random; (limbs, value)."""
+    k = rng.randrange(4)
+    ws = [hi - 1] * 9 if k == 0 else [0] * 9 if k == 1 else [rng.randrange(hi) for _ in range(9)]
+    if k == 1:
+        ws[rng.randrange(9)] = hi - 1
+    return ws, from_l(ws)
+
+
+@pytest.mark.parametrize("field,code,hi", [("q", 0, (30, 30)), ("q", 1, (30,)), ("q", 2, (29,) * 4), ("q", 8, (29,) * 4),
+                                           ("r", 0, (30, 29)), ("r", 0, (29, 30))])
+def test_products_at_the_limb_bounds(fh, field, code, hi):
+    """Montgomery products at the largest limbs their columns may hold (the
+    64-bit accumulators must not wrap): congruent to the exact sum, limbs
+    normalized below the top one, and below sum / 2^261 + m + m / 2^22."""
+    rng = random.Random(31 + code)
+    m = Q if field == "q" else ORDER
+    for _ in range(300):
+        ops = [limbs_value(rng, 1 << h) for h in hi]
+        v = [x[1] for x in ops] + [0] * (4 - len(ops))
+        total = {0: v[0] * v[1], 1: v[0] * v[0], 2: v[0] * v[1] + v[2] * v[3], 8: (v[0] + v[2]) * (v[1] + v[3])}[code]
+        assert total >> 525 == 0  # the result's top limb fits 32 bits
+        w = [U32x9(*x[0]) for x in ops] + [U32x9()] * (4 - len(ops))
+        out = U32x9()
+        assert (fh.fh_op(code, *w, out) if field == "q" else fh.fh_fr_op(code, w[0], w[1], out)) == 0
+        ws = list(out)
+        assert all(x < 1 << 29 for x in ws[:8])
+        r = from_l(ws)
+        assert r % m == total * pow(RP, -1, m) % m
+        assert r <= total // RP + m + (m >> 22)
