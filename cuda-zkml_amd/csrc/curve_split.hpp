@@ -43,16 +43,19 @@ __device__ __forceinline__ fq2h fsub(const fq2h& a, const fq2h& b) { return fq2h
 __device__ __forceinline__ fq2h fdbl(const fq2h& a) { return fq2h{fdbl(a.c)}; }
 __device__ __forceinline__ fq2h fneg(const fq2h& a) { return fq2h{fneg(a.c)}; }
 __device__ __forceinline__ fq2h fneg_canon_if(const fq2h& a, bool neg) { return fq2h{fneg_canon_if(a.c, neg)}; }
-__device__ __forceinline__ fq2h fsub3(const fq2h& a, const fq2h& b, const fq2h& c) {
-  return fq2h{fsub3<FqP>(a.c, b.c, c.c)};
-}
 __device__ __forceinline__ fq2h fsub_m(const fq2h& a, const fq2h& b) { return fq2h{fsub_lazy(a.c, b.c)}; }
+__device__ __forceinline__ fq2h fsub_x(const fq2h& a, const fq2h& b) { return fq2h{fsub_off<6>(a.c, b.c)}; }
+__device__ __forceinline__ fq2h fsub3_lazy(const fq2h& a, const fq2h& b, const fq2h& c) {
+  return fq2h{fsub3_lazy(a.c, b.c, c.c)};
+}
+__device__ __forceinline__ fq2h ftriple_wide(const fq2h& a) { return fq2h{ftriple_wide(a.c)}; }
+__device__ __forceinline__ fq2h fadd_wide(const fq2h& a, const fq2h& b) { return fq2h{fadd_wide(a.c, b.c)}; }
 
 __device__ __forceinline__ bool fis_zero(const fq2h& a) {
   const uint32_t z = fis_zero(a.c) ? 1u : 0u;
   return (z & swap_pair(z)) != 0;
 }
-__device__ __forceinline__ bool fis_zero4(const fq2h& a) {
+__device__ __forceinline__ bool fis_zero_sqr(const fq2h& a) {
   const uint32_t z = fis_zero4<FqP>(a.c) ? 1u : 0u;
   return (z & swap_pair(z)) != 0;
 }
@@ -69,11 +72,13 @@ __device__ __forceinline__ fq2h fmul(const fq2h& a, const fq2h& b) {
   return fq2h{fmul_sum<FqP, 2>(x, y)};
 }
 
+__device__ __forceinline__ fq2h fmul_x(const fq2h& x, const fq2h& b) { return fmul(b, x); }
+
 // (a + bu)^2: even lane (a0 + a1)(a0 - a1), odd lane 2 a0 a1
 __device__ __forceinline__ fq2h fsqr(const fq2h& a) {
   const bool odd = lane_odd();
   const fq pa = swap_pair(a.c);
-  const fq t = fmul(fsel(odd, pa, fadd_lazy(a.c, pa)), fsel(odd, a.c, fsub_lazy4(a.c, pa)));
+  const fq t = fmul(fsel(odd, pa, fadd_lazy(a.c, pa)), fsel(odd, a.c, fsub_off<8>(a.c, pa)));
   return fq2h{fsel(odd, fdbl(t), t)};
 }
 
@@ -83,7 +88,7 @@ __device__ __forceinline__ fq2h fmul_sub(const fq2h& a, const fq2h& b, const fq2
   const bool odd = lane_odd();
   const fq pa = swap_pair(a.c), pb = swap_pair(b.c), pc = swap_pair(c.c), pd = swap_pair(d.c);
   const fq nc = fneg_lazy(c.c), npc = fneg_lazy(pc);
-  const fq x[4] = {fsel(odd, pa, a.c), fsel(odd, a.c, fneg_lazy4(pa)), fsel(odd, npc, nc), fsel(odd, nc, pc)};
+  const fq x[4] = {fsel(odd, pa, a.c), fsel(odd, a.c, fneg_lazy6(pa)), fsel(odd, npc, nc), fsel(odd, nc, pc)};
   const fq y[4] = {b.c, pb, d.c, pd};
   return fq2h{fmul_sum<FqP, 4>(x, y)};
 }
@@ -192,25 +197,23 @@ __device__ __forceinline__ split<E> fneg(const split<E>& a) {
 // p = 2p (dbl-2008-s-1): V = U^2 | X^2, then W = U V | S = X V, then M^2 |
 // V ZZ, then W ZZZ | Y3 = M (S - X3) - W Y.
 template <class E>
-__device__ __forceinline__ void xyzz_dbl(xyzz<split<E>>& p) {
+__device__ __forceinline__ void xyzz_dbl_lx(xyzz<split<E>>& p) {
   if (fis_zero(p.zz.v)) return;
   const bool r1 = split_role1<E>();
-  const E U = fdbl(p.y.v);
+  const E U = fadd_wide(p.y.v, p.y.v);
   const E a = fsqr(pick(r1, p.x.v, U));  // V | X^2
   const E ao = other_role(a);
   const E V = pick(r1, ao, a), X2 = pick(r1, a, ao);
-  const E b = fmul(pick(r1, p.x.v, U), V);  // W | S
+  const E b = fmul(V, pick(r1, p.x.v, U));  // W | S
   const E bo = other_role(b);
   const E W = pick(r1, bo, b), S = pick(r1, b, bo);
-  const E M = fadd(fdbl(X2), X2);
-  const E c = fmul(pick(r1, V, M), pick(r1, p.zz.v, M));  // M^2 | ZZ3 = V ZZ
-  const E co = other_role(c);
-  const E MM = pick(r1, co, c), ZZ3 = pick(r1, c, co);
+  const E M = ftriple_wide(X2);
+  const E MM = fsqr(M), ZZ3 = fmul(p.zz.v, V);
   E zero;
   fset_zero(zero);
-  const E X3 = fsub3(MM, zero, S);
+  const E X3 = fsub3_lazy(MM, zero, S);
   // W ZZZ - 0 | M (S - X3) - W Y
-  const E d = fmul_sub(pick(r1, M, W), pick(r1, fsub_m(S, X3), p.zzz.v), pick(r1, W, zero), pick(r1, p.y.v, zero));
+  const E d = fmul_sub(pick(r1, M, W), pick(r1, fsub_x(S, X3), p.zzz.v), pick(r1, W, zero), pick(r1, p.y.v, zero));
   const E dd = other_role(d);
   p.x.v = X3;
   p.y.v = pick(r1, d, dd);
@@ -221,14 +224,14 @@ __device__ __forceinline__ void xyzz_dbl(xyzz<split<E>>& p) {
 // p += q (add-2008-s): U1 | U2, S1 | S2, ZZ1 ZZ2 | ZZZ1 ZZZ2; then PP | RR;
 // then PPP | Q and ZZ3 on both; then ZZZ3 | Y3.
 template <class E>
-__device__ __forceinline__ void xyzz_add(xyzz<split<E>>& p, const xyzz<split<E>>& q) {
+__device__ __forceinline__ void xyzz_add_lx(xyzz<split<E>>& p, const xyzz<split<E>>& q) {
   if (fis_zero(q.zz.v)) return;
   if (fis_zero(p.zz.v)) {
     p = q;
     return;
   }
   const bool r1 = split_role1<E>();
-  const E a = fmul(pick(r1, q.x.v, p.x.v), pick(r1, p.zz.v, q.zz.v));     // U1 = X1 ZZ2 | U2 = X2 ZZ1
+  const E a = fmul(pick(r1, p.zz.v, q.zz.v), pick(r1, q.x.v, p.x.v));     // U1 = X1 ZZ2 | U2 = X2 ZZ1
   const E b = fmul(pick(r1, q.y.v, p.y.v), pick(r1, p.zzz.v, q.zzz.v));   // S1 = Y1 ZZZ2 | S2 = Y2 ZZZ1
   const E c = fmul(pick(r1, p.zzz.v, p.zz.v), pick(r1, q.zzz.v, q.zz.v)); // ZZ1 ZZ2 | ZZZ1 ZZZ2
   const E ao = other_role(a), bo = other_role(b), co = other_role(c);
@@ -237,23 +240,23 @@ __device__ __forceinline__ void xyzz_add(xyzz<split<E>>& p, const xyzz<split<E>>
   const E ZZ12 = pick(r1, co, c), ZZZ12 = pick(r1, c, co);
   const E P = fsub_m(U2, U1);  // lazy, (0, 4m)
   const E R = fsub_m(S2, S1);  // lazy, (0, 4m)
-  if (fis_zero4(P)) {
-    if (fis_zero4(R)) xyzz_dbl(p);
-    else xyzz_set_inf(p);
-    return;
-  }
   const E t = fsqr(pick(r1, R, P));  // PP | RR
   const E to = other_role(t);
   const E PP = pick(r1, to, t), RR = pick(r1, t, to);
+  if (fis_zero(PP)) {
+    if (fis_zero(RR)) xyzz_dbl_lx(p);
+    else xyzz_set_inf(p);
+    return;
+  }
   const E v = fmul(PP, pick(r1, U1, P));  // PPP | Q (P lazy: the second factor)
   const E ZZ3 = fmul(ZZ12, PP);
   const E vo = other_role(v);
   const E PPP = pick(r1, vo, v), Q = pick(r1, v, vo);
-  const E X3 = fsub3(RR, PPP, Q);
+  const E X3 = fsub3_lazy(RR, PPP, Q);
   E zero;
   fset_zero(zero);
   // ZZZ12 PPP - 0 | R (Q - X3) - S1 PPP
-  const E d = fmul_sub(pick(r1, R, ZZZ12), pick(r1, fsub_m(Q, X3), PPP), pick(r1, S1, zero), pick(r1, PPP, zero));
+  const E d = fmul_sub(pick(r1, R, ZZZ12), pick(r1, fsub_x(Q, X3), PPP), pick(r1, S1, zero), pick(r1, PPP, zero));
   const E dd = other_role(d);
   p.x.v = X3;
   p.y.v = pick(r1, d, dd);

@@ -334,19 +334,20 @@ ZK_HD fe<P> fneg_lazy(const fe<P>& a) {
 }
 
 // neg ? m - a : a for a canonical (in [0, m)); m - a is in (0, m], a valid
-// value of the lazy range [0, 2m).
+// value of the lazy range [0, 2m).  -a is ~a + 1 limb by limb under a mask,
+// not a select: nine selects in a row through VCC take 15-23 cycles each on
+// gfx950 (a mask operation 2.4 to 4.4).
 template <class P>
 ZK_HD fe<P> fneg_canon_if(const fe<P>& a, bool neg) {
+  const uint32_t mask = neg ? ~0u : 0u;
   fe<P> d;
-  int32_t br = 0;
+  int32_t c = 0;
 #pragma unroll
   for (int i = 0; i < NL; i++) {
-    int32_t v = (int32_t)P::MOD[i] - (int32_t)a.l[i] + br;
-    br = v >> 29;
+    int32_t v = (int32_t)((a.l[i] ^ mask) + (mask & (P::MOD[i] + 1u))) + c;
+    c = v >> 29;
     d.l[i] = (uint32_t)v & LMASK;
   }
-#pragma unroll
-  for (int i = 0; i < NL; i++) d.l[i] = neg ? d.l[i] : a.l[i];
   return d;
 }
 
@@ -460,6 +461,49 @@ ZK_HD fe<P> fsub3(const fe<P>& a, const fe<P>& b, const fe<P>& c) {
   return fcsub(fcsub(t, P::MOD4), P::MOD2);
 }
 
+// a - b - 2c + 4m, exact (normalized limbs), for a value that stays positive:
+// b + 2c < 4m.
+template <class P>
+ZK_HD fe<P> fsub3_lazy(const fe<P>& a, const fe<P>& b, const fe<P>& c) {
+  fe<P> t;
+  int32_t cy = 0;
+#pragma unroll
+  for (int i = 0; i < NL; i++) {
+    int32_t v = (int32_t)a.l[i] + (int32_t)P::MOD4[i] - (int32_t)b.l[i] - 2 * (int32_t)c.l[i] + cy;
+    cy = v >> 29;
+    t.l[i] = (uint32_t)v & LMASK;
+  }
+  return t;
+}
+
+// 3a with carries and no reduction (normalized limbs, value below 2^261).
+template <class P>
+ZK_HD fe<P> ftriple_wide(const fe<P>& a) {
+  fe<P> s;
+  uint32_t c = 0;
+#pragma unroll
+  for (int i = 0; i < NL; i++) {
+    uint32_t v = 3u * a.l[i] + c;
+    c = v >> 29;
+    s.l[i] = v & LMASK;
+  }
+  return s;
+}
+
+// 6m - a for a in [0, 6m]: value in [0, 6m], normalized limbs.
+template <class P>
+ZK_HD fe<P> fneg_lazy6(const fe<P>& a) {
+  fe<P> d;
+  int32_t c = 0;
+#pragma unroll
+  for (int i = 0; i < NL; i++) {
+    int32_t v = (int32_t)P::MOD6[i] - (int32_t)a.l[i] + c;
+    c = v >> 29;
+    d.l[i] = (uint32_t)v & LMASK;
+  }
+  return d;
+}
+
 // a - b + 4m for a in [0, 4m), b in [0, 4m]: value in (0, 8m), normalized
 // limbs.  Valid only as an fmul / fsqr input.
 template <class P>
@@ -489,12 +533,12 @@ ZK_HD fe<P> fneg_lazy4(const fe<P>& a) {
   return d;
 }
 
-// a - b + KM*m with carries (KM in {2, 4, 8}): for b < KM*m the value is
+// a - b + KM*m with carries (KM in {2, 4, 6, 8}): for b < KM*m the value is
 // a - b + KM*m > 0 with normalized limbs (valid while below 2^261).
 template <int KM, class P>
 ZK_HD fe<P> fsub_off(const fe<P>& a, const fe<P>& b) {
-  static_assert(KM == 2 || KM == 4 || KM == 8, "offset multiple");
-  const uint32_t(&K)[NL] = KM == 2 ? P::MOD2 : KM == 4 ? P::MOD4 : P::MOD8;
+  static_assert(KM == 2 || KM == 4 || KM == 6 || KM == 8, "offset multiple");
+  const uint32_t(&K)[NL] = KM == 2 ? P::MOD2 : KM == 4 ? P::MOD4 : KM == 6 ? P::MOD6 : P::MOD8;
   fe<P> d;
   int32_t c = 0;
 #pragma unroll

@@ -113,6 +113,16 @@ __device__ __forceinline__ void pack_coord(uint32_t* p, const fq2& a) {
   repack_out(a.c1, p + 8);
 }
 
+// All words zero (the point at infinity): one comparison for other points.
+template <int W>
+__device__ __forceinline__ bool all_zero(const uint32_t (&w)[W]) {
+  if (__builtin_expect(w[W - 8] != 0, 1)) return false;
+  uint32_t any = 0;
+#pragma unroll
+  for (int i = 0; i < W; i++) any |= w[i];
+  return any == 0;
+}
+
 // Record load through 16-byte vector loads; returns true for infinity.
 template <class F>
 __device__ __forceinline__ bool load_rec(const uint4* __restrict__ recs, uint32_t idx, F& x, F& y) {
@@ -127,12 +137,9 @@ __device__ __forceinline__ bool load_rec(const uint4* __restrict__ recs, uint32_
     w[4 * i + 2] = v.z;
     w[4 * i + 3] = v.w;
   }
-  uint32_t any = 0;
-#pragma unroll
-  for (int i = 0; i < W; i++) any |= w[i];
   unpack_coord(w, x);
   unpack_coord(w + W / 2, y);
-  return any == 0;
+  return all_zero<W>(w);
 }
 
 // pack_coord stores canonical values (repack_out), so a negative digit's -y
@@ -1001,7 +1008,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(acc_waves<L
           xyzz_set_affine(acc, x, y);
           empty = false;
         } else {
-          empty = xyzz_madd_fin(acc, x, y);
+          empty = xyzz_madd_fin_lx(acc, x, y);
         }
       }
     }
@@ -1060,7 +1067,7 @@ __global__ __launch_bounds__(256) void k_msm_combine_serial(ChunkSlots<F> all_sl
   const uint32_t c1 = (end[tk] - 1) / L0;
   if (c1 - ch > MSM_SERIAL_SPAN) return;  // a long span: the tree combine
   auto acc = LN::load(slots.tpt[ch]);
-  for (uint32_t j = ch + 1; j <= c1; j++) xyzz_add(acc, LN::load(slots.hpt[j]));
+  for (uint32_t j = ch + 1; j <= c1; j++) xyzz_add_lx(acc, LN::load(slots.hpt[j]));
   LN::store(buckets[tk], acc);
 }
 
@@ -1092,7 +1099,7 @@ __global__ __launch_bounds__(256) void k_msm_combine(ChunkSlots<F> all_slots, co
   if ((ch - c0) % (S * step) != 0 || ch + step > c1) return;  // nothing to fold here
   xyzz<F>* self = tail ? &slots.tpt[ch] : &slots.hpt[ch];
   auto acc = LN::load(*self);
-  for (uint32_t m = 1; m < S && ch + m * step <= c1; m++) xyzz_add(acc, LN::load(slots.hpt[ch + m * step]));
+  for (uint32_t m = 1; m < S && ch + m * step <= c1; m++) xyzz_add_lx(acc, LN::load(slots.hpt[ch + m * step]));
   if (tail && c1 - c0 + 1 <= S * step) self = &buckets[key];
   LN::store(*self, acc);
 }
@@ -1175,7 +1182,7 @@ __global__ __launch_bounds__(TB * LN::N) void k_msm_combine_tree(ChunkSlots<F> a
   const uint32_t levels_len = maxlen;
   for (uint32_t d = 1; d < levels_len; d <<= 1) {
     if (hk != KEY_INVALID && r % (2 * d) == 0 && r + d < len) {
-      xyzz_add(v, LN::load(V[t + d]));
+      xyzz_add_lx(v, LN::load(V[t + d]));
       LN::store(V[t], v);
     }
     __syncthreads();
@@ -1183,7 +1190,7 @@ __global__ __launch_bounds__(TB * LN::N) void k_msm_combine_tree(ChunkSlots<F> a
   // V[first item of a segment] = the segment's sum.  Contributions:
   if (tk != KEY_INVALID) {
     xyzz<R> acc = LN::load(slots.tpt[ch]);
-    if (ch + 1 < b1) xyzz_add(acc, LN::load(V[t + 1]));  // the heads that follow in this block
+    if (ch + 1 < b1) xyzz_add_lx(acc, LN::load(V[t + 1]));  // the heads that follow in this block
     if (tc1 < b1) {
       LN::store(buckets[tk], acc);  // the whole bucket is in this block
     } else {
@@ -1220,14 +1227,14 @@ __global__ __launch_bounds__(TB * LN::N) void k_msm_combine_tree(ChunkSlots<F> a
     const uint32_t j0 = fold_j0[f], n = fold_n[f];
     xyzz<R> a;
     xyzz_set_inf(a);
-    for (uint32_t i = t; i < n; i += TB) xyzz_add(a, LN::load(i == 0 ? cout[j0] : cin[j0 + i]));
+    for (uint32_t i = t; i < n; i += TB) xyzz_add_lx(a, LN::load(i == 0 ? cout[j0] : cin[j0 + i]));
     __syncthreads();
     LN::store(V[t], a);
     __syncthreads();
     const uint32_t m = min(n, (uint32_t)TB);
     for (uint32_t d = 1; d < m; d <<= 1) {
       if (t % (2 * d) == 0 && t + d < m) {
-        xyzz_add(a, LN::load(V[t + d]));
+        xyzz_add_lx(a, LN::load(V[t + d]));
         LN::store(V[t], a);
       }
       __syncthreads();
@@ -1265,7 +1272,7 @@ __device__ __forceinline__ xyzz<R> wg_suffix_scan(xyzz<R> v, xyzz<F>* sh, int T)
     if (has) o = LN::load(sh[t + d]);
     __syncthreads();
     if (has) {
-      xyzz_add(v, o);
+      xyzz_add_lx(v, o);
       LN::store(sh[t], v);
     }
     __syncthreads();
@@ -1282,7 +1289,7 @@ __device__ __forceinline__ xyzz<R> wg_sum(xyzz<R> v, xyzz<F>* sh, int T) {
   __syncthreads();
   for (int h = T / 2; h >= 1; h >>= 1) {
     if (t < h) {
-      xyzz_add(v, LN::load(sh[t + h]));
+      xyzz_add_lx(v, LN::load(sh[t + h]));
       LN::store(sh[t], v);
     }
     __syncthreads();
@@ -1315,13 +1322,13 @@ __global__ __launch_bounds__(TMAX * LN::N) void k_msm_reduce1(const xyzz<F>* __r
   xyzz_set_inf(acc);
   for (int i = G - 1; i >= 0; i--) {
     const uint32_t off = (t * G + i) * K;
-    if (end[sb + off] > start[sb + off]) xyzz_add(run, LN::load(buckets[kb + off]));
-    xyzz_add(acc, run);
+    if (end[sb + off] > start[sb + off]) xyzz_add_lx(run, LN::load(buckets[kb + off]));
+    xyzz_add_lx(acc, run);
   }
   xyzz<R> sr = wg_suffix_scan<F, LN, R>(run, sh, T);
   if (t >= 1) {
-    for (int d = 0; d < log2g; d++) xyzz_dbl(sr);
-    xyzz_add(acc, sr);
+    for (int d = 0; d < log2g; d++) xyzz_dbl_lx(sr);
+    xyzz_add_lx(acc, sr);
   } else {
     LN::store(RUN[blockIdx.x], sr);  // item 0 holds the group total
   }
@@ -1366,24 +1373,24 @@ __global__ __launch_bounds__(128) void k_msm_reduce2(const xyzz<F>* __restrict__
       xyzz<R> r = LN::load(RUN[w * K + t]);
       v = LN::load(P[w * K + t]);
       r.y = fneg(r.y);
-      xyzz_add(v, r);
-      for (int d = 0; d < log2k; d++) xyzz_dbl(v);
+      xyzz_add_lx(v, r);
+      for (int d = 0; d < log2k; d++) xyzz_dbl_lx(v);
       LN::store(ku[t], v);
     }
   } else {
     if (t < K) v = LN::load(RUN[w * K + t]);
     for (uint32_t d = 1; d < K; d <<= 1) {  // inclusive suffix scan
       const xyzz<R> o = shfl_down_pt(v, (int)(d * LN::N));
-      if (t + d < K) xyzz_add(v, o);
+      if (t + d < K) xyzz_add_lx(v, o);
     }
     if (plain && t == 0) LN::store(plain[w], v);
   }
   __syncthreads();
   if (wave0) {
-    if (t < K) xyzz_add(v, LN::load(ku[t]));
+    if (t < K) xyzz_add_lx(v, LN::load(ku[t]));
     for (uint32_t d = K / 2; d >= 1; d >>= 1) {  // tree sum into item 0
       const xyzz<R> o = shfl_down_pt(v, (int)(d * LN::N));
-      if (t < d) xyzz_add(v, o);
+      if (t < d) xyzz_add_lx(v, o);
     }
     if (t == 0) LN::store(out[w], v);
   }
@@ -2117,7 +2124,7 @@ __global__ void k_msm_tab_double(const uint4* __restrict__ recs, size_t count, i
   for (int w = 0; w < W; w++) {
     tmp[(size_t)w * count + j] = p;
     if (w + 1 < W)
-      for (int k = 0; k < window_width(w, W); k++) xyzz_dbl(p);
+      for (int k = 0; k < window_width(w, W); k++) xyzz_dbl_lx(p);
   }
 }
 

@@ -106,4 +106,39 @@ int fh_xyzz(int g2, int op, const uint32_t* p, const uint32_t* q, uint32_t* out)
   }
   return 0;
 }
+
+// The lazy-X forms (X in [0, 6q) in and out): op 0: p += (qx, qy) affine, p
+// finite   1: p += q   2: p = 2p   3: p = 2 (qx, qy).  Returns 1 where op 0
+// reports the point at infinity.
+int fh_xyzz_lx(int g2, int op, const uint32_t* p, const uint32_t* q, uint32_t* out) {
+  int inf = 0;
+  if (!g2) {
+    xyzz<fq> P{ld(p), ld(p + 9), ld(p + 18), ld(p + 27)}, Q{ld(q), ld(q + 9), ld(q + 18), ld(q + 27)};
+    switch (op) {
+      case 0: inf = xyzz_madd_fin_lx(P, Q.x, Q.y); break;
+      case 1: xyzz_add_lx(P, Q); break;
+      case 2: xyzz_dbl_lx(P); break;
+      case 3: xyzz_mdbl_lx(P, Q.x, Q.y); break;
+      default: return -1;
+    }
+    st(out, P.x);
+    st(out + 9, P.y);
+    st(out + 18, P.zz);
+    st(out + 27, P.zzz);
+  } else {
+    xyzz<fq2> P{ld2(p), ld2(p + 18), ld2(p + 36), ld2(p + 54)}, Q{ld2(q), ld2(q + 18), ld2(q + 36), ld2(q + 54)};
+    switch (op) {
+      case 0: inf = xyzz_madd_fin_lx(P, Q.x, Q.y); break;
+      case 1: xyzz_add_lx(P, Q); break;
+      case 2: xyzz_dbl_lx(P); break;
+      case 3: xyzz_mdbl_lx(P, Q.x, Q.y); break;
+      default: return -1;
+    }
+    st2(out, P.x);
+    st2(out + 18, P.y);
+    st2(out + 36, P.zz);
+    st2(out + 54, P.zzz);
+  }
+  return inf;
+}
 }

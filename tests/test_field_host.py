@@ -350,3 +350,114 @@ def test_products_at_the_limb_bounds(fh, field, code, hi):
         r = from_l(ws)
         assert r % m == total * pow(RP, -1, m) % m
         assert r <= total // RP + m + (m >> 22)
+
+
+@pytest.mark.parametrize("g2flag", [0, 1])
+def test_lazy_x_formulas(fh, g2flag):
+    """The forms the MSM kernels run: X anywhere in [0, 6q) in, below 6q out,
+    the other coordinates in [0, 2q) in and out, at the edges of these ranges
+    (every representative of the coordinates, the largest included), over
+    chains of operations, and in the doubling, inverse and infinity cases."""
+    rng = random.Random(41 + g2flag)
+    grp, gen = (g2, G2) if g2flag else (g1, G1)
+    n, nw = (2, 72) if g2flag else (1, 36)
+
+    def coords(pt, z):  # x, y, zz, zzz in the internal radix, as lists of Fq values
+        if pt is None:
+            return [[0] * n for _ in range(4)]
+        if g2flag:
+            zz = f2_mul(z, z)
+            zzz = f2_mul(zz, z)
+            c = [f2_mul(pt[0], zz), f2_mul(pt[1], zzz), zz, zzz]
+        else:
+            c = [(pt[0] * z * z % Q,), (pt[1] * z * z * z % Q,), (z * z % Q,), (z * z * z % Q,)]
+        return [[v * RP % Q for v in t] for t in c]
+
+    def words(cs, mode):  # representatives: 0 the smallest, 1 the largest, 2 random
+        out = []
+        for i, t in enumerate(cs):
+            top = 6 if i == 0 else 2
+            for v in t:
+                k = (0, top - 1, rng.randrange(top))[mode]
+                out += to_l(v + k * Q)
+        return out
+
+    def call(code, p, q):
+        arr = ctypes.c_uint32 * nw
+        out = arr()
+        inf = fh.fh_xyzz_lx(g2flag, code, arr(*p), arr(*(q + [0] * (nw - len(q)))), out)
+        return inf, list(out)
+
+    def decode(ws):
+        cs = [[from_l(ws[9 * (n * i + j):9 * (n * i + j) + 9]) for j in range(n)] for i in range(4)]
+        assert all(w < 1 << 29 for w in ws)
+        assert all(v < 6 * Q for v in cs[0]) and all(v < 2 * Q for t in cs[1:] for v in t)
+        X, Y, ZZ, ZZZ = (tuple(v % Q for v in t) for t in cs)
+        if not any(ZZ):
+            assert not any(ZZZ)
+            return None
+        if g2flag:
+            return f2_mul(X, f2_inv(ZZ)), f2_mul(Y, f2_inv(ZZZ))
+        return X[0] * pow(ZZ[0], -1, Q) % Q, Y[0] * pow(ZZZ[0], -1, Q) % Q
+
+    def rz():
+        return (rng.randrange(1, Q), rng.randrange(Q)) if g2flag else rng.randrange(1, Q)
+
+    def affine(pt):
+        c = coords(pt, (1, 0) if g2flag else 1)
+        return [w for t in c[:2] for v in t for w in to_l(v)]
+
+    for mode in (0, 1, 2, 2):
+        a, b = (grp.pmul(gen, rng.randrange(1, ORDER)) for _ in range(2))
+        wa, wb = words(coords(a, rz()), mode), words(coords(b, rz()), mode)
+        assert decode(call(0, wa, affine(b))[1]) == grp.padd(a, b)
+        assert decode(call(1, wa, wb)[1]) == grp.padd(a, b)
+        assert decode(call(2, wa, [])[1]) == grp.padd(a, a)
+        assert decode(call(3, [0] * nw, affine(a))[1]) == grp.padd(a, a)
+        inf, out = call(0, wa, affine(a))
+        assert not inf and decode(out) == grp.padd(a, a)
+        inf, out = call(0, wa, affine(grp.pneg(a)))
+        assert inf == 1 and decode(out) is None
+        assert decode(call(1, wa, words(coords(a, rz()), mode))[1]) == grp.padd(a, a)
+        assert decode(call(1, wa, words(coords(grp.pneg(a), rz()), mode))[1]) is None
+        assert decode(call(1, wa, words(coords(None, None), 0))[1]) == a
+        assert decode(call(1, words(coords(None, None), 0), wb)[1]) == b
+        # a chain: outputs feed the next operation
+        acc, want = wa, a
+        for _ in range(12):
+            p = grp.pmul(gen, rng.randrange(1, ORDER))
+            acc = call(0, acc, affine(p))[1]
+            want = grp.padd(want, p)
+            assert decode(acc) == want
+            acc = call(1, acc, wb)[1]
+            want = grp.padd(want, b)
+            acc = call(2, acc, [])[1]
+            want = grp.padd(want, want)
+            assert decode(acc) == want
+
+
+@pytest.mark.parametrize("g2flag", [0, 1])
+def test_lazy_x_ranges_at_random_residues(fh, g2flag):
+    """The output ranges of the lazy-X forms hold for any coordinate values
+    (points or not), the largest representatives above all: a mixed addition,
+    an addition and a doubling of random words."""
+    rng = random.Random(51 + g2flag)
+    n, nw = (2, 72) if g2flag else (1, 36)
+    arr = ctypes.c_uint32 * nw
+
+    def value(top):
+        return rng.choice([top * Q - 1, top * Q - 1 - rng.randrange(1 << 200), rng.randrange(top * Q)])
+
+    def point():
+        return [w for i in range(4) for _ in range(n) for w in to_l(value(6 if i == 0 else 2))]
+
+    for _ in range(400):
+        p, q = point(), point()
+        aff = [w for _ in range(2 * n) for w in to_l(rng.choice([Q - 1, rng.randrange(Q)]))]
+        for code, arg in ((0, aff), (1, q), (2, [])):
+            out = arr()
+            fh.fh_xyzz_lx(g2flag, code, arr(*p), arr(*(arg + [0] * (nw - len(arg)))), out)
+            ws = list(out)
+            assert all(w < 1 << 29 for w in ws)
+            vals = [from_l(ws[9 * k:9 * k + 9]) for k in range(4 * n)]
+            assert all(v < 6 * Q for v in vals[:n]) and all(v < 2 * Q for v in vals[n:])
