@@ -18,8 +18,8 @@
 // changes its cost.  Y, ZZ, ZZZ stay below 2m.  The plain forms take and give
 // coordinates below 2m.  Bounds, per coordinate and in units of m (a product
 // of a and b is below ab / 169.2 + 1.0000003; an Fq2 product is one of sums
-// a0 b0 + (2 - a1) b1 with a the reduced factor; an Fq2 square (a0 + a1)(a0 -
-// a1 + 8) and 2 a0 a1):
+// a0 b0 + (4 - a1) b1 with a the reduced factor; an Fq2 square (a0 + a1)(a0 -
+// a1 + 8) and (2 a0) a1):
 //   mixed addition: U2, S2 < 1.1; P = U2 - X + 6 in (0, 7), R = S2 - Y + 2 in
 //   (0, 3.3); P^2 < 2.2, R^2 < 1.5; PPP, Q < 1.2; X3 = R^2 - PPP - 2Q + 4 in (0.4,
 //   5.6); Q - X3 + 6 in (0.4, 6.9), so Y3 < 1.5; ZZ3, ZZZ3 < 1.1.
@@ -47,18 +47,17 @@ ZK_HD fq2 fneg_canon_if(const fq2& a, bool neg) { return fq2{fneg_canon_if(a.c0,
 // (a0 + a1 u)(b0 + b1 u) = (a0 b0 - a1 b1) + (a0 b1 + a1 b0) u, each
 // coordinate one fmul_sum (4 limb products, 2 reductions; the reference uses
 // Karatsuba, src/field/fp2.cuh:73-78: 3 multiplies, each with its own
-// reduction).  -a1 enters as 2q - a1, so a must be reduced (a1 < 2q); b may be
-// a lazy value (< 8q).
+// reduction).  -a1 enters as 4q - a1 (no carry pass), so a must be reduced (a1 <
+// 2q); b may be a lazy value (< 8q).
 ZK_HD fq2 fmul(const fq2& a, const fq2& b) {
-  const fq x0[2] = {a.c0, fneg_lazy(a.c1)}, y0[2] = {b.c0, b.c1};
+  const fq x0[2] = {a.c0, fneg_wide(a.c1)}, y0[2] = {b.c0, b.c1};
   const fq x1[2] = {a.c0, a.c1}, y1[2] = {b.c1, b.c0};
   return fq2{fmul_sum<FqP, 2>(x0, y0), fmul_sum<FqP, 2>(x1, y1)};
 }
-// (a + bu)^2 = (a+b)(a-b) + 2ab u; a may be a lazy value (< 8q; the result is
+// (a + bu)^2 = (a+b)(a-b) + (2a)b u; a may be a lazy value (< 8q; the result is
 // below 2q for a < 6q, its real part below 2.3q up to 7q).
 ZK_HD fq2 fsqr(const fq2& a) {
-  fq ab = fmul(a.c0, a.c1);
-  return fq2{fmul(fadd_lazy(a.c0, a.c1), fsub_off<8>(a.c0, a.c1)), fdbl(ab)};
+  return fq2{fmul(fadd_lazy(a.c0, a.c1), fsub_off<8>(a.c0, a.c1)), fmul(fadd_lazy(a.c0, a.c0), a.c1)};
 }
 ZK_HD bool fis_zero(const fq2& a) { return fis_zero(a.c0) && fis_zero(a.c1); }
 
@@ -74,7 +73,7 @@ ZK_HD fq2 fmul_x(const fq2& x, const fq2& b) { return fmul(b, x); }
 // a*b - c*d with one Montgomery reduction per coordinate (fmul_sum, the
 // subtracted products entering as (km - x) * y).  a and b may be lazy values
 // (a < 6m, b < 7m); c and d are reduced (< 2m).
-ZK_HD fq fmul_sub(const fq& a, const fq& b, const fq& c, const fq& d) { return fmul2(a, b, c, fneg_lazy(d)); }
+ZK_HD fq fmul_sub(const fq& a, const fq& b, const fq& c, const fq& d) { return fmul2(a, b, c, fneg_wide(d)); }
 ZK_HD fq2 fmul_sub(const fq2& a, const fq2& b, const fq2& c, const fq2& d) {
   // real: a0 b0 - a1 b1 - c0 d0 + c1 d1, imaginary: a0 b1 + a1 b0 - c0 d1 - c1 d0
   const fq na1 = fneg_lazy6(a.c1), nc0 = fneg_lazy(c.c0), nc1 = fneg_lazy(c.c1);

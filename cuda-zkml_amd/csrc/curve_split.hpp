@@ -62,34 +62,59 @@ __device__ __forceinline__ bool fis_zero_sqr(const fq2h& a) {
 __device__ __forceinline__ void fset_zero(fq2h& a) { a.c = fe_zero<FqP>(); }
 __device__ __forceinline__ void fset_one(fq2h& a) { a.c = lane_odd() ? fe_zero<FqP>() : fe_one<FqP>(); }
 
-// (a0 + a1 u)(b0 + b1 u): even lane a0 b0 + (-a1) b1, odd lane a1 b0 + a0 b1
-// (the pairs of the fq2 fmul of curve.hpp, with the same operand bounds).
-__device__ __forceinline__ fq2h fmul(const fq2h& a, const fq2h& b) {
-  const bool odd = lane_odd();
-  const fq pa = swap_pair(a.c), pb = swap_pair(b.c);
-  const fq x[2] = {fsel(odd, pa, a.c), fsel(odd, a.c, fneg_lazy(pa))};
-  const fq y[2] = {b.c, pb};
-  return fq2h{fmul_sum<FqP, 2>(x, y)};
+// The even / odd lane's coordinate on both lanes of the pair (DPP quad_perm
+// [0, 0, 2, 2] and [1, 1, 3, 3]).  The operations below take their operands by
+// these moves and by negations under a lane mask instead of selects.
+template <int CTRL>
+__device__ __forceinline__ fq dpp_fq(const fq& a) {
+  fq r;
+#pragma unroll
+  for (int i = 0; i < NL; i++) r.l[i] = (uint32_t)__builtin_amdgcn_mov_dpp((int)a.l[i], CTRL, 0xF, 0xF, false);
+  return r;
+}
+__device__ __forceinline__ fq even_both(const fq2h& a) { return dpp_fq<0xA0>(a.c); }
+__device__ __forceinline__ fq odd_both(const fq2h& a) { return dpp_fq<0xF5>(a.c); }
+// all ones on even lanes; opaque, so that the compiler does not keep the masked
+// modulus limbs of every operation in registers across a loop (36 of them, which
+// the G2 accumulation spilled)
+__device__ __forceinline__ uint32_t even_mask() {
+  uint32_t m = (threadIdx.x & 1u) - 1u;
+  asm volatile("" : "+v"(m));
+  return m;
 }
 
+// (a0 + a1 u)(b0 + b1 u): even lane a0 b0 + (-a1) b1, odd lane a0 b1 + a1 b0
+// (the pairs of the fq2 fmul of curve.hpp, with the same operand bounds).
+__device__ __forceinline__ fq2h fmul(const fq2h& a, const fq2h& b) {
+  const fq x[2] = {even_both(a), fneg_wide_mask(odd_both(a), even_mask())};
+  const fq y[2] = {b.c, swap_pair(b.c)};
+  return fq2h{fmul_sum<FqP, 2>(x, y)};
+}
 __device__ __forceinline__ fq2h fmul_x(const fq2h& x, const fq2h& b) { return fmul(b, x); }
 
-// (a + bu)^2: even lane (a0 + a1)(a0 - a1), odd lane 2 a0 a1
+// (a + bu)^2: even lane (a0 + a1)(a0 - a1 + 8q), odd lane (a0 + a0) a1; each
+// first factor is the partner's coordinate plus a0.
 __device__ __forceinline__ fq2h fsqr(const fq2h& a) {
-  const bool odd = lane_odd();
+  const uint32_t mask = even_mask();
   const fq pa = swap_pair(a.c);
-  const fq t = fmul(fsel(odd, pa, fadd_lazy(a.c, pa)), fsel(odd, a.c, fsub_off<8>(a.c, pa)));
-  return fq2h{fsel(odd, fdbl(t), t)};
+  fq w;  // even: a0 - a1 + 8q, odd: a1
+  int32_t c = 0;
+#pragma unroll
+  for (int i = 0; i < NL; i++) {
+    int32_t v = (int32_t)(a.c.l[i] + (mask & (FqP::MOD8[i] - pa.l[i]))) + c;
+    c = v >> 29;
+    w.l[i] = (uint32_t)v & LMASK;
+  }
+  return fq2h{fmul(fadd_lazy(pa, even_both(a)), w)};
 }
 
 // a b - c d (fq2 fmul_sub of curve.hpp): even lane a0 b0 - a1 b1 - c0 d0 +
-// c1 d1, odd lane a1 b0 + a0 b1 - c1 d0 - c0 d1.
+// c1 d1, odd lane a0 b1 + a1 b0 - c0 d1 - c1 d0.
 __device__ __forceinline__ fq2h fmul_sub(const fq2h& a, const fq2h& b, const fq2h& c, const fq2h& d) {
-  const bool odd = lane_odd();
-  const fq pa = swap_pair(a.c), pb = swap_pair(b.c), pc = swap_pair(c.c), pd = swap_pair(d.c);
-  const fq nc = fneg_lazy(c.c), npc = fneg_lazy(pc);
-  const fq x[4] = {fsel(odd, pa, a.c), fsel(odd, a.c, fneg_lazy6(pa)), fsel(odd, npc, nc), fsel(odd, nc, pc)};
-  const fq y[4] = {b.c, pb, d.c, pd};
+  const uint32_t mask = even_mask();
+  const fq x[4] = {even_both(a), fneg_mask<6>(odd_both(a), mask), fneg_lazy(even_both(c)),
+                   fneg_mask<2>(odd_both(c), ~mask)};
+  const fq y[4] = {b.c, swap_pair(b.c), d.c, swap_pair(d.c)};
   return fq2h{fmul_sum<FqP, 4>(x, y)};
 }
 
@@ -114,6 +139,7 @@ __device__ __forceinline__ void store_half(xyzz<fq2>& p, const xyzz<fq2h>& v) {
 template <class F>
 struct Lanes {
   typedef F R;
+  typedef xyzz<F> Pt;
   static constexpr int N = 1;
   __device__ static xyzz<F> load(const xyzz<F>& p) { return p; }
   __device__ static void store(xyzz<F>& p, const xyzz<F>& v) { p = v; }
@@ -121,6 +147,7 @@ struct Lanes {
 template <>
 struct Lanes<fq2> {
   typedef fq2h R;
+  typedef xyzz<fq2h> Pt;
   static constexpr int N = 2;
   __device__ static xyzz<fq2h> load(const xyzz<fq2>& p) { return load_half(p); }
   __device__ static void store(xyzz<fq2>& p, const xyzz<fq2h>& v) { store_half(p, v); }
@@ -134,17 +161,20 @@ namespace zk {
 // One point operation of a latency-bound chain dealt to two lane groups
 // ("roles"): G1 to a lane pair (E = fq, role = lane bit 0), G2 to two lane
 // pairs (E = fq2h, role = lane bit 1, each pair holding the two Fq2 halves).
-// Both roles hold the whole point.  The formulas' independent products are
-// split between the roles, each role computing one of them with operands it
-// selects by its role, and the results are exchanged through DPP lane swaps:
-// an addition's chain of 12 multiplications, 2 squarings and one two-product
-// sum becomes about 7.5 multiplications deep.  The roles branch together
-// (every branch tests values both hold).  Worth it where a chain runs alone
-// on its SIMD; beside other waves the extra selects and swaps cost issue
-// slots.
+// Role 0 holds x and zz of the point, role 1 y and zzz: the independent
+// products of the formulas then take their operands from the role's own half
+//   U1, U2, ZZ1 ZZ2, P, P^2   |   S1, S2, ZZZ1 ZZZ2, R, R^2
+// and only five values cross between the roles (U1, P^2, R^2, PPP, Q), each
+// as one broadcast lane move per limb.  An addition's 12 products, 2 squares
+// and one two-product sum become 5 products, a square and the sum deep; it
+// issues about 0.6 of the instructions of the one-lane form on each lane.
+// Holding the whole point in both roles instead took 12 nine-limb selects to
+// pick each role's operands (and the selects ran through VCC back to back, 15
+// to 23 cycles each).  The roles branch together (every branch tests values
+// both hold).
 template <class E>
-struct split {
-  E v;
+struct xyzz_half {
+  E a, b;  // role 0: x (lazy, as in the *_lx forms), zz; role 1: y, zzz
 };
 
 template <class E>
@@ -152,12 +182,12 @@ struct SplitRole;
 template <>
 struct SplitRole<fq> {
   static constexpr uint32_t BIT = 1;
-  static constexpr int DPP = 0xB1;  // quad_perm [1, 0, 3, 2]: the other lane of the pair
+  static constexpr int FROM0 = 0xA0, FROM1 = 0xF5;  // quad_perm [0, 0, 2, 2], [1, 1, 3, 3]
 };
 template <>
 struct SplitRole<fq2h> {
   static constexpr uint32_t BIT = 2;
-  static constexpr int DPP = 0x4E;  // quad_perm [2, 3, 0, 1]: the same half in the other pair
+  static constexpr int FROM0 = 0x44, FROM1 = 0xEE;  // quad_perm [0, 1, 0, 1], [2, 3, 2, 3]
 };
 
 template <class E>
@@ -166,128 +196,119 @@ __device__ __forceinline__ bool split_role1() {
 }
 
 template <int CTRL>
-__device__ __forceinline__ fq dpp_fq(const fq& a) {
-  fq r;
-#pragma unroll
-  for (int i = 0; i < NL; i++) r.l[i] = (uint32_t)__builtin_amdgcn_mov_dpp((int)a.l[i], CTRL, 0xF, 0xF, false);
-  return r;
+__device__ __forceinline__ fq2h dpp_fq(const fq2h& a) {
+  return fq2h{dpp_fq<CTRL>(a.c)};
 }
-__device__ __forceinline__ fq other_role(const fq& a) { return dpp_fq<SplitRole<fq>::DPP>(a); }
-__device__ __forceinline__ fq2h other_role(const fq2h& a) { return fq2h{dpp_fq<SplitRole<fq2h>::DPP>(a.c)}; }
+// role 0's / role 1's value of a, on both roles
+template <class E>
+__device__ __forceinline__ E from0(const E& a) {
+  return dpp_fq<SplitRole<E>::FROM0>(a);
+}
+template <class E>
+__device__ __forceinline__ E from1(const E& a) {
+  return dpp_fq<SplitRole<E>::FROM1>(a);
+}
 __device__ __forceinline__ fq pick(bool c, const fq& a, const fq& b) { return fsel(c, a, b); }
 __device__ __forceinline__ fq2h pick(bool c, const fq2h& a, const fq2h& b) { return fq2h{fsel(c, a.c, b.c)}; }
 
 template <class E>
-__device__ __forceinline__ void fset_zero(split<E>& a) {
-  fset_zero(a.v);
-}
-template <class E>
-__device__ __forceinline__ void fset_one(split<E>& a) {
-  fset_one(a.v);
-}
-template <class E>
-__device__ __forceinline__ bool fis_zero(const split<E>& a) {
-  return fis_zero(a.v);
-}
-template <class E>
-__device__ __forceinline__ split<E> fneg(const split<E>& a) {
-  return split<E>{fneg(a.v)};
+__device__ __forceinline__ void xyzz_set_inf(xyzz_half<E>& p) {
+  fset_zero(p.a);
+  fset_zero(p.b);
 }
 
-// p = 2p (dbl-2008-s-1): V = U^2 | X^2, then W = U V | S = X V, then M^2 |
-// V ZZ, then W ZZZ | Y3 = M (S - X3) - W Y.
+// zz and zzz are 0 mod m together, so both roles find the same answer
 template <class E>
-__device__ __forceinline__ void xyzz_dbl_lx(xyzz<split<E>>& p) {
-  if (fis_zero(p.zz.v)) return;
+__device__ __forceinline__ bool xyzz_is_inf(const xyzz_half<E>& p) {
+  return fis_zero(p.b);
+}
+
+template <class E>
+__device__ __forceinline__ void xyzz_neg(xyzz_half<E>& p) {
+  if (split_role1<E>()) p.a = fneg(p.a);
+}
+
+// p = 2p (dbl-2008-s-1): X^2 | V = U^2, S = X V | W = U V, M^2 and X3 on both,
+// ZZ3 = V ZZ | ZZZ3 = W ZZZ, then Y3 = M (S - X3) - W Y on role 1.
+template <class E>
+__device__ __forceinline__ void xyzz_dbl_lx(xyzz_half<E>& p) {
+  if (xyzz_is_inf(p)) return;
   const bool r1 = split_role1<E>();
-  const E U = fadd_wide(p.y.v, p.y.v);
-  const E a = fsqr(pick(r1, p.x.v, U));  // V | X^2
-  const E ao = other_role(a);
-  const E V = pick(r1, ao, a), X2 = pick(r1, a, ao);
-  const E b = fmul(V, pick(r1, p.x.v, U));  // W | S
-  const E bo = other_role(b);
-  const E W = pick(r1, bo, b), S = pick(r1, b, bo);
-  const E M = ftriple_wide(X2);
-  const E MM = fsqr(M), ZZ3 = fmul(p.zz.v, V);
+  const E s = pick(r1, fadd_wide(p.a, p.a), p.a);  // X | U = 2 Y
+  const E t = fsqr(s);
+  const E V = from1(t), M = ftriple_wide(from0(t));
+  const E w = fmul(V, s);  // S | W
+  p.b = fmul(pick(r1, w, V), p.b);
+  const E S = from0(w);
   E zero;
   fset_zero(zero);
-  const E X3 = fsub3_lazy(MM, zero, S);
-  // W ZZZ - 0 | M (S - X3) - W Y
-  const E d = fmul_sub(pick(r1, M, W), pick(r1, fsub_x(S, X3), p.zzz.v), pick(r1, W, zero), pick(r1, p.y.v, zero));
-  const E dd = other_role(d);
-  p.x.v = X3;
-  p.y.v = pick(r1, d, dd);
-  p.zz.v = ZZ3;
-  p.zzz.v = pick(r1, dd, d);
+  const E X3 = fsub3_lazy(fsqr(M), zero, S);
+  const E d = fmul_sub(M, fsub_x(S, X3), w, p.a);
+  p.a = pick(r1, d, X3);
 }
 
-// p += q (add-2008-s): U1 | U2, S1 | S2, ZZ1 ZZ2 | ZZZ1 ZZZ2; then PP | RR;
-// then PPP | Q and ZZ3 on both; then ZZZ3 | Y3.
+// p += q (add-2008-s)
 template <class E>
-__device__ __forceinline__ void xyzz_add_lx(xyzz<split<E>>& p, const xyzz<split<E>>& q) {
-  if (fis_zero(q.zz.v)) return;
-  if (fis_zero(p.zz.v)) {
+__device__ __forceinline__ void xyzz_add_lx(xyzz_half<E>& p, const xyzz_half<E>& q) {
+  if (xyzz_is_inf(q)) return;
+  if (xyzz_is_inf(p)) {
     p = q;
     return;
   }
   const bool r1 = split_role1<E>();
-  const E a = fmul(pick(r1, p.zz.v, q.zz.v), pick(r1, q.x.v, p.x.v));     // U1 = X1 ZZ2 | U2 = X2 ZZ1
-  const E b = fmul(pick(r1, q.y.v, p.y.v), pick(r1, p.zzz.v, q.zzz.v));   // S1 = Y1 ZZZ2 | S2 = Y2 ZZZ1
-  const E c = fmul(pick(r1, p.zzz.v, p.zz.v), pick(r1, q.zzz.v, q.zz.v)); // ZZ1 ZZ2 | ZZZ1 ZZZ2
-  const E ao = other_role(a), bo = other_role(b), co = other_role(c);
-  const E U1 = pick(r1, ao, a), U2 = pick(r1, a, ao);
-  const E S1 = pick(r1, bo, b), S2 = pick(r1, b, bo);
-  const E ZZ12 = pick(r1, co, c), ZZZ12 = pick(r1, c, co);
-  const E P = fsub_m(U2, U1);  // lazy, (0, 4m)
-  const E R = fsub_m(S2, S1);  // lazy, (0, 4m)
-  const E t = fsqr(pick(r1, R, P));  // PP | RR
-  const E to = other_role(t);
-  const E PP = pick(r1, to, t), RR = pick(r1, t, to);
-  if (fis_zero(PP)) {
-    if (fis_zero(RR)) xyzz_dbl_lx(p);
+  const E a = fmul(q.b, p.a);                // U1 | S1
+  const E PR = fsub_m(fmul(p.b, q.a), a);    // P | R, lazy, (0, 4m)
+  const E t = fsqr(PR);                      // PP | RR
+  const E PP = from0(t);
+  if (__builtin_expect(fis_zero(PP), 0)) {
+    if (fis_zero(from1(t))) xyzz_dbl_lx(p);
     else xyzz_set_inf(p);
     return;
   }
-  const E v = fmul(PP, pick(r1, U1, P));  // PPP | Q (P lazy: the second factor)
-  const E ZZ3 = fmul(ZZ12, PP);
-  const E vo = other_role(v);
-  const E PPP = pick(r1, vo, v), Q = pick(r1, v, vo);
-  const E X3 = fsub3_lazy(RR, PPP, Q);
-  E zero;
-  fset_zero(zero);
-  // ZZZ12 PPP - 0 | R (Q - X3) - S1 PPP
-  const E d = fmul_sub(pick(r1, R, ZZZ12), pick(r1, fsub_x(Q, X3), PPP), pick(r1, S1, zero), pick(r1, PPP, zero));
-  const E dd = other_role(d);
-  p.x.v = X3;
-  p.y.v = pick(r1, d, dd);
-  p.zz.v = ZZ3;
-  p.zzz.v = pick(r1, dd, d);
+  const E v = fmul(PP, pick(r1, from0(a), PR));        // PPP | Q = U1 PP
+  const E PPP = from0(v);
+  p.b = fmul(fmul(p.b, q.b), pick(r1, PPP, PP));       // ZZ3 | ZZZ3
+  const E Q = from1(v);
+  const E X3 = fsub3_lazy(from1(t), PPP, Q);
+  const E d = fmul_sub(PR, fsub_x(Q, X3), a, PPP);     // | Y3 = R (Q - X3) - S1 PPP
+  p.a = pick(r1, d, X3);
 }
 
-// Register forms of the latency-bound kernels with the operations split
-// over two roles: a G1 point on a lane pair, a G2 point on four lanes.  Only
-// role 0 stores (both hold the same point).
+// The point in the register form of each layout: Lanes (and one lane per
+// point): xyzz<R>; SplitLanes: xyzz_half<E>, the coordinates moved by the role
+// that holds them.
 template <class F>
 struct SplitLanes;
 template <>
 struct SplitLanes<fq> {
-  typedef split<fq> R;
+  typedef xyzz_half<fq> Pt;
   static constexpr int N = 2;
-  __device__ static xyzz<R> load(const xyzz<fq>& p) { return xyzz<R>{R{p.x}, R{p.y}, R{p.zz}, R{p.zzz}}; }
-  __device__ static void store(xyzz<fq>& p, const xyzz<R>& v) {
-    if (!split_role1<fq>()) p = xyzz<fq>{v.x.v, v.y.v, v.zz.v, v.zzz.v};
+  __device__ static Pt load(const xyzz<fq>& p) {
+    const int r = split_role1<fq>() ? 1 : 0;
+    const fq* w = (const fq*)&p;
+    return Pt{w[r], w[2 + r]};
+  }
+  __device__ static void store(xyzz<fq>& p, const Pt& v) {
+    const int r = split_role1<fq>() ? 1 : 0;
+    fq* w = (fq*)&p;
+    w[r] = v.a;
+    w[2 + r] = v.b;
   }
 };
 template <>
 struct SplitLanes<fq2> {
-  typedef split<fq2h> R;
+  typedef xyzz_half<fq2h> Pt;
   static constexpr int N = 4;
-  __device__ static xyzz<R> load(const xyzz<fq2>& p) {
-    const xyzz<fq2h> h = load_half(p);
-    return xyzz<R>{R{h.x}, R{h.y}, R{h.zz}, R{h.zzz}};
+  // fq words of p: x0 x1 y0 y1 zz0 zz1 zzz0 zzz1; this lane's are at 2 role + half
+  __device__ static int word() { return (int)(threadIdx.x & 3); }
+  __device__ static Pt load(const xyzz<fq2>& p) {
+    const fq* w = (const fq*)&p;
+    return Pt{fq2h{w[word()]}, fq2h{w[4 + word()]}};
   }
-  __device__ static void store(xyzz<fq2>& p, const xyzz<R>& v) {
-    if (!split_role1<fq2h>()) store_half(p, xyzz<fq2h>{v.x.v, v.y.v, v.zz.v, v.zzz.v});
+  __device__ static void store(xyzz<fq2>& p, const Pt& v) {
+    fq* w = (fq*)&p;
+    w[word()] = v.a.c;
+    w[4 + word()] = v.b.c;
   }
 };
 

@@ -208,13 +208,13 @@ ZK_HD fe<P> fmul(const fe<P>& a, const fe<P>& b) {
 }
 
 // sum_t a[t]*b[t] * 2^-261 mod q, N = 2 or 4, with one Montgomery reduction
-// for all products.  Inputs: normalized limbs (< 2^29), values <= 4q (the sum
-// of the products below 100 q^2).  The result is below 100 q^2 / 2^261 + q +
-// q/2^22 < 1.6 q.
+// for all products.  Inputs: normalized limbs (< 2^29), with N = 2 of one
+// factor below 2^30 (fneg_wide); the sum of the products below 100 q^2.  The
+// result is below 100 q^2 / 2^261 + q + q/2^22 < 1.6 q.
 template <class P, int N>
 ZK_HD fe<P> fmul_sum(const fe<P> (&a)[N], const fe<P> (&b)[N]) {
   static_assert(N == 2 || N == 4, "products of one reduction");
-  static_assert(mont_columns_fit<P>(9 * N), "column accumulator bound");
+  static_assert(mont_columns_fit<P>(N == 2 ? 27 : 36), "column accumulator bound");
 #if defined(__HIP_DEVICE_COMPILE__)
   fe<P> r = a[0];  // in place when a[0] is dead after the products
   if constexpr (N == 2)
@@ -330,6 +330,32 @@ ZK_HD fe<P> fneg_lazy(const fe<P>& a) {
     c = v >> 29;
     d.l[i] = (uint32_t)v & LMASK;
   }
+  return d;
+}
+
+// 4m with 2^29 moved down into every limb below the top one: digit by digit not
+// less than any normalized value below 2m, so KWIDE_i - a_i needs no borrow.
+template <class P>
+constexpr uint32_t kwide(int i) {
+  return i == 0 ? P::MOD4[0] + LMASK + 1u : i < NL - 1 ? P::MOD4[i] + LMASK : P::MOD4[NL - 1] - 1u;
+}
+
+// 4m - a for a in [0, 2m), limbs below 2^30 without a carry pass: an operand of
+// a two-product sum or of fmul only.
+template <class P>
+ZK_HD fe<P> fneg_wide(const fe<P>& a) {
+  fe<P> d;
+#pragma unroll
+  for (int i = 0; i < NL; i++) d.l[i] = kwide<P>(i) - a.l[i];
+  return d;
+}
+
+// neg ? 4m - a : a under a mask, as fneg_wide.
+template <class P>
+ZK_HD fe<P> fneg_wide_mask(const fe<P>& a, uint32_t mask) {
+  fe<P> d;
+#pragma unroll
+  for (int i = 0; i < NL; i++) d.l[i] = (a.l[i] ^ mask) + (mask & (kwide<P>(i) + 1u));
   return d;
 }
 
@@ -513,6 +539,22 @@ ZK_HD fe<P> fsub_lazy4(const fe<P>& a, const fe<P>& b) {
 #pragma unroll
   for (int i = 0; i < NL; i++) {
     int32_t v = (int32_t)a.l[i] + (int32_t)P::MOD4[i] - (int32_t)b.l[i] + c;
+    c = v >> 29;
+    d.l[i] = (uint32_t)v & LMASK;
+  }
+  return d;
+}
+
+// mask ? KM*m - a : a with carries (mask all ones or zero; KM = 2 or 6, a <= KM*m).
+template <int KM, class P>
+ZK_HD fe<P> fneg_mask(const fe<P>& a, uint32_t mask) {
+  static_assert(KM == 2 || KM == 6, "offset multiple");
+  const uint32_t(&K)[NL] = KM == 2 ? P::MOD2 : P::MOD6;
+  fe<P> d;
+  int32_t c = 0;
+#pragma unroll
+  for (int i = 0; i < NL; i++) {
+    int32_t v = (int32_t)((a.l[i] ^ mask) + (mask & (K[i] + 1u))) + c;
     c = v >> 29;
     d.l[i] = (uint32_t)v & LMASK;
   }

@@ -572,9 +572,6 @@ int zk_quotient_h(zk_context* ctx, const zk_r1cs* c, const void* d_witness, size
 #ifndef ZK_PK_TAB_W_HUGE
 #define ZK_PK_TAB_W_HUGE 13
 #endif
-#ifndef ZK_PK_TAB_SUB
-#define ZK_PK_TAB_SUB 10
-#endif
 #ifndef ZK_PK_TAB_W_LARGE
 #define ZK_PK_TAB_W_LARGE 16
 #endif
@@ -585,30 +582,17 @@ int zk_quotient_h(zk_context* ctx, const zk_r1cs* c, const void* d_witness, size
 #define ZK_PK_TAB_W_LARGE_H 20
 #endif
 
-// H's sub-windows: 2^8 buckets, level 1 one bucket per thread (H sorts and
-// reduces after the quotient, on the 2^16 proof's critical path: its reduction
-// 4 -> 16 workgroups, H 0.70 -> 0.66 ms)
-#ifndef ZK_PK_TAB_SUB_H
-#define ZK_PK_TAB_SUB_H 8
-#endif
-// B2's sub-windows: 2^9 buckets (the G2 job ends the 2^16 proof; its
-// reduction chains are Fq2 additions, one level shallower this way: config 4
-// 1.32-1.36 -> 1.30 ms; 2^8 and 2^7 1.30-1.31 ms)
-#ifndef ZK_PK_TAB_SUB_B2
-#define ZK_PK_TAB_SUB_B2 9
-#endif
 // Table shape for MSMs of n scalars (W = 0: no table); wlarge: windows from
-// 2^15 scalars on; sub: log2 of the sub-window size up to 2^18 scalars.
-static MsmTab table_shape(size_t n, int wlarge, int sub = ZK_PK_TAB_SUB) {
+// 2^15 scalars on.
+static MsmTab table_shape(size_t n, int wlarge) {
   MsmTab t;
   if (n < ((size_t)1 << ZK_PK_TAB_MIN_LOG) || n > ((size_t)1 << ZK_PK_TAB_MAX_LOG)) return t;
   const bool huge = n > ((size_t)1 << 18);
   t.W = huge ? ZK_PK_TAB_W_HUGE : n >= ((size_t)1 << 15) ? wlarge : 20;
   if ((size_t)t.W * n > MSM_MAX_N) return MsmTab{};  // positions of all windows beyond the sort's range
   const int c = (254 + t.W - 1) / t.W;  // widest window
-  // above 2^18 scalars: 2^15-bucket sub-windows (the plain MSMs' reduction
-  // shape at 2^20 .. 2^22 points)
-  t.log_sub = std::min(huge ? 15 : sub, c - 1);
+  // reduced as sub-windows of up to 2^15 buckets: one up to 2^18 scalars
+  t.log_sub = std::min(15, c - 1);
   return t;
 }
 
@@ -632,8 +616,8 @@ static void pk_drop_tables(zk_pk* pk) {
 
 static int pk_tables_build(zk_context* ctx, zk_pk* pk) {
   pk->tab_w = table_shape((size_t)pk->m, ZK_PK_TAB_W_LARGE);
-  pk->tab_b2 = table_shape((size_t)pk->m, ZK_PK_TAB_W_LARGE_B2, ZK_PK_TAB_SUB_B2);
-  pk->tab_h = table_shape((size_t)pk->n, ZK_PK_TAB_W_LARGE_H, ZK_PK_TAB_SUB_H);
+  pk->tab_b2 = table_shape((size_t)pk->m, ZK_PK_TAB_W_LARGE_B2);
+  pk->tab_h = table_shape((size_t)pk->n, ZK_PK_TAB_W_LARGE_H);
   if (pk->tab_w.W) {
     ZK_TRY(pk_table(ctx, false, pk->A, pk->nA, pk->tab_w, &pk->tA));
     ZK_TRY(pk_table(ctx, false, pk->B1, pk->nB1, pk->tab_w, &pk->tB1));

@@ -24,11 +24,10 @@
 //                folded in groups (one launch for ordinary buckets,
 //                ~log8(size/L0) for hot buckets such as many scalars equal
 //                to 1).
-//  6. reduce     sum_b b*S_b per window: G-bucket segments with running sums
-//                plus (segment offset)*run, then LDS scans and trees per
-//                group of T segments and per window.
-//  7. host       remaining per-window partials are summed and combined with
-//                W*c doublings on the CPU (serial chain: a CPU core beats a
+//  6. reduce     sum_b b*S_b per window: plain row and column sums of its
+//                buckets, then the weighted sums of those (at most 256 each).
+//  7. host       one to four points per window are combined with W*c
+//                doublings on the CPU (serial chain: a CPU core beats a
 //                lone wave64 by an order of magnitude on it).
 #include <string.h>
 #include <stdlib.h>
@@ -175,8 +174,8 @@ __device__ __forceinline__ void std_to_coord(const uint32_t* e, fq2& a) {
 // 0 for infinity) -> records.
 // Issue priority of the MSM's waves.  Inside a proof several MSMs and the
 // quotient share the GPU.  The accumulation is throughput-bound and always
-// ready to issue; the digit sort and the chunk combine / bucket reduction are
-// short or latency-bound and sit on some MSM's critical path.  Those waves
+// ready to issue; the digit sort and the chunk combine are short or
+// latency-bound and sit on some MSM's critical path.  Those waves
 // run at priority 2 so that the SIMD arbiter serves them first and the
 // accumulation takes the remaining issue slots (at equal priority a lone
 // chain wave would get a fraction of its SIMD; at lower priority next to an
@@ -186,6 +185,11 @@ template <class F>
 __device__ __forceinline__ void msm_priority() {
   msm_short_priority();
 }
+// The bucket reduction stays at priority 0: its kernels take 100 registers a
+// lane on split lanes, so another job's accumulation waves fit beside them on a
+// SIMD, and at priority 2 they starved there (a 2^13 proof's H accumulation took
+// 135 us instead of 43; the proof 0.54 instead of 0.49 ms).
+__device__ __forceinline__ void msm_reduce_priority() { __builtin_amdgcn_s_setprio(0); }
 // The G2 accumulation is the longest throughput phase of a proof and starts
 // its MSM's critical path: priority 1, above the G1 accumulations (0).
 template <class F>
@@ -1127,7 +1131,7 @@ __global__ __launch_bounds__(TB * LN::N) void k_msm_combine_tree(ChunkSlots<F> a
                                                                  xyzz<F>* __restrict__ buckets,
                                                                  uint32_t* __restrict__ fold_cnt,
                                                                  xyzz<F>* __restrict__ cin, xyzz<F>* __restrict__ cout) {
-  typedef typename LN::R R;
+  typedef typename LN::Pt Pt;
   msm_priority<F>();
   __shared__ xyzz<F> V[TB];
   __shared__ uint32_t fold_key[2], fold_j0[2], fold_n[2], maxlen;
@@ -1172,7 +1176,7 @@ __global__ __launch_bounds__(TB * LN::N) void k_msm_combine_tree(ChunkSlots<F> a
   __syncthreads();
   if (!__syncthreads_or(hk != KEY_INVALID || tk != KEY_INVALID)) return;  // no long bucket here
   if (hk != KEY_INVALID && r == 0 && lead) atomicMax(&maxlen, len);
-  xyzz<R> v;
+  Pt v;
   xyzz_set_inf(v);
   if (hk != KEY_INVALID) {
     v = LN::load(slots.hpt[ch]);
@@ -1189,7 +1193,7 @@ __global__ __launch_bounds__(TB * LN::N) void k_msm_combine_tree(ChunkSlots<F> a
   }
   // V[first item of a segment] = the segment's sum.  Contributions:
   if (tk != KEY_INVALID) {
-    xyzz<R> acc = LN::load(slots.tpt[ch]);
+    Pt acc = LN::load(slots.tpt[ch]);
     if (ch + 1 < b1) xyzz_add_lx(acc, LN::load(V[t + 1]));  // the heads that follow in this block
     if (tc1 < b1) {
       LN::store(buckets[tk], acc);  // the whole bucket is in this block
@@ -1225,7 +1229,7 @@ __global__ __launch_bounds__(TB * LN::N) void k_msm_combine_tree(ChunkSlots<F> a
     if (key == KEY_INVALID) continue;  // uniform over the block
     __threadfence();
     const uint32_t j0 = fold_j0[f], n = fold_n[f];
-    xyzz<R> a;
+    Pt a;
     xyzz_set_inf(a);
     for (uint32_t i = t; i < n; i += TB) xyzz_add_lx(a, LN::load(i == 0 ? cout[j0] : cin[j0 + i]));
     __syncthreads();
@@ -1245,160 +1249,240 @@ __global__ __launch_bounds__(TB * LN::N) void k_msm_combine_tree(ChunkSlots<F> a
 }
 
 // ------------------------------------------------------------------ bucket reduction
-// Window sum  sum_{b=1..B} b S_b,  B = 2^(c-1).
-//
-// Bucket b of a window holds digit b + 1.  Level 1: K workgroups per window;
-// group k owns the buckets b = k + K p (every K-th bucket, positions
-// p = 0 .. T G - 1), its thread t the positions p = t G + i, i < G, forming
-//   run_t = sum_i S,  acc_t = sum_i (i+1) S      (2G additions, from the top).
-// With the inclusive suffix sums SR_t = sum_{u >= t} run_u (Hillis-Steele scan
-// in LDS),  sum_p (p+1) S = sum_t acc_t + G sum_{t >= 1} SR_t,  so each thread
-// adds G*SR_t (log2 G doublings) to acc_t and a tree sums the group.  Outputs
-// per group: P_k (that sum) and RUN_k = SR_0.
-// Level 2 (k_msm_reduce2) weights group k by K and k + 1 - K, so its chain
-// holds log2 K doublings where contiguous groups would need log2(T G).
-// "Thread" t is an item of the lane layout LN; T = blockDim.x / LN::N.
+// Window sum  sum_b (b + 1) S_b  over its B = 2^l buckets (bucket b holds digit
+// b + 1).  With b = r C + c, C = 2^lc columns and R = B / C rows,
+//   sum_b (b + 1) S_b = C sum_r r Y_r + sum_c (c + 1) X_c,
+// where Y_r and X_c are the plain row and column sums.  Those are 2 additions
+// per bucket like the running sums they replace, but independent ones:
+//   k_msm_rowcol  every item sums G buckets of one row or one column, then a
+//                 tree in LDS joins the items of a row / column;
+//   k_msm_weigh   the weighted sum of a window's C (or R) sums, at most 256:
+//                 the same split again (trees of up to 16), then 16 + 16 values
+//                 with a suffix scan and a tree in one wave (G2: two).  It
+//                 leaves up to four points per window, which the host's
+//                 combination over the windows' doublings adds at their own bit
+//                 offsets (no doublings on the GPU).
+// Windows of up to 256 buckets take k_msm_weigh alone.  A running-sum pass of 8
+// buckets per item followed by a 256-item suffix scan and tree took 35
+// dependent additions at 2^15 buckets and spent half of its additions in the
+// scan; this takes 7 + 5 and 1 + 3 + 8 on split lanes.
 
-// Inclusive suffix scan over the T values held by the items of a workgroup;
-// returns this item's sum_{u >= t} v_u.
-template <class F, class LN, class R>
-__device__ __forceinline__ xyzz<R> wg_suffix_scan(xyzz<R> v, xyzz<F>* sh, int T) {
-  const int t = threadIdx.x / LN::N;
-  LN::store(sh[t], v);
-  __syncthreads();
-  for (int d = 1; d < T; d <<= 1) {
-    xyzz<R> o;
-    const bool has = t + d < T;
-    if (has) o = LN::load(sh[t + d]);
-    __syncthreads();
-    if (has) {
-      xyzz_add_lx(v, o);
-      LN::store(sh[t], v);
-    }
-    __syncthreads();
-  }
-  return v;
-}
-
-// Sum of the T values of a workgroup (T a power of two), valid in item 0.
-template <class F, class LN, class R>
-__device__ __forceinline__ xyzz<R> wg_sum(xyzz<R> v, xyzz<F>* sh, int T) {
-  const int t = threadIdx.x / LN::N;
-  __syncthreads();
-  LN::store(sh[t], v);
-  __syncthreads();
-  for (int h = T / 2; h >= 1; h >>= 1) {
-    if (t < h) {
-      xyzz_add_lx(v, LN::load(sh[t + h]));
-      LN::store(sh[t], v);
-    }
-    __syncthreads();
-  }
-  return v;
-}
-
-// Level 1: block k of window w (blockIdx.x = w*K + k), T items of G buckets
-// each (G = 2^log2g).  Windows of several base sets follow each other (W_set
-// windows per set); the sorted-list bounds start/end are those of the window
-// within its set.
-template <class F, int TMAX, class LN>
-__global__ __launch_bounds__(TMAX * LN::N) void k_msm_reduce1(const xyzz<F>* __restrict__ buckets,
-                                                              const uint32_t* __restrict__ start,
-                                                              const uint32_t* __restrict__ end, uint32_t B1,
-                                                              uint32_t K, uint32_t W_set, int log2g,
-                                                              xyzz<F>* __restrict__ P, xyzz<F>* __restrict__ RUN) {
-  typedef typename LN::R R;
-  msm_priority<F>();
-  __shared__ xyzz<F> sh[TMAX];
-  const int T = blockDim.x / LN::N, G = 1 << log2g;
-  const uint32_t w = blockIdx.x / K, k = blockIdx.x % K;
-  const uint32_t t = threadIdx.x / LN::N;
-  // group k owns buckets k + K p, p = 0, 1, ...; this item the positions
-  // p = t G + i, i < G
-  const uint32_t kb = w * B1 + k;            // bucket of position 0
-  const uint32_t sb = (w % W_set) * B1 + k;  // its key in the sorted list
-  xyzz<R> run, acc;
+// Row (blockIdx.y 0) and column (1) sums.  Items of a row: bucket r C + t +
+// (C / G) i, i < G, so that neighbouring items read neighbouring buckets; of a
+// column: bucket (t + (R / G) i) C + c, neighbouring items on neighbouring
+// columns.  LC: lane layout of the item chains; the tree runs on split lanes
+// (half as many additions as items, twice the lanes).  Windows of several base
+// sets follow each other (W_set windows per set); the sorted-list bounds
+// start/end are those of the window within its set.
+template <class F, class LC>
+__global__ __launch_bounds__(256) void k_msm_rowcol(const xyzz<F>* __restrict__ buckets,
+                                                    const uint32_t* __restrict__ start,
+                                                    const uint32_t* __restrict__ end, uint32_t windows,
+                                                    uint32_t W_set, int l, int lc, int log2g,
+                                                    xyzz<F>* __restrict__ X, xyzz<F>* __restrict__ Y) {
+  typedef SplitLanes<F> LT;
+  constexpr uint32_t I = 256 / LC::N;  // items of a block
+  msm_reduce_priority();
+  __shared__ xyzz<F> sh[I];
+  const bool cols = blockIdx.y != 0;
+  const uint32_t G = 1u << log2g;
+  const uint32_t ls = (uint32_t)(cols ? l - lc : lc) - log2g;  // log2 of the items per row / column
+  const uint32_t nseg = I >> ls;                             // rows / columns of a block
+  const uint32_t segs = windows << (cols ? lc : l - lc);     // all of them
+  const uint32_t q = threadIdx.x / LC::N;
+  const uint32_t sl = cols ? q % nseg : q >> ls, t = cols ? q / nseg : q & ((1u << ls) - 1);
+  const uint32_t seg = blockIdx.x * nseg + sl;
+  typename LC::Pt run;
   xyzz_set_inf(run);
-  xyzz_set_inf(acc);
-  for (int i = G - 1; i >= 0; i--) {
-    const uint32_t off = (t * G + i) * K;
-    if (end[sb + off] > start[sb + off]) xyzz_add_lx(run, LN::load(buckets[kb + off]));
-    xyzz_add_lx(acc, run);
+  if (seg < segs) {
+    uint32_t b0, step, w;  // first bucket within the window, bucket stride
+    if (cols) {
+      w = seg >> lc;
+      b0 = (t << lc) + (seg & ((1u << lc) - 1));
+      step = 1u << (ls + lc);
+    } else {
+      w = seg >> (l - lc);
+      b0 = ((seg & ((1u << (l - lc)) - 1)) << lc) + t;
+      step = 1u << ls;
+    }
+    const uint32_t sb = ((w % W_set) << l) + b0;
+    const size_t kb = ((size_t)w << l) + b0;
+    for (uint32_t i = 0; i < G; i++) {
+      const uint32_t o = i * step;
+      if (end[sb + o] > start[sb + o]) xyzz_add_lx(run, LC::load(buckets[kb + o]));
+    }
   }
-  xyzz<R> sr = wg_suffix_scan<F, LN, R>(run, sh, T);
-  if (t >= 1) {
-    for (int d = 0; d < log2g; d++) xyzz_dbl_lx(sr);
-    xyzz_add_lx(acc, sr);
-  } else {
-    LN::store(RUN[blockIdx.x], sr);  // item 0 holds the group total
+  LC::store(sh[(sl << ls) + t], run);
+  __syncthreads();
+  const uint32_t item = threadIdx.x / LT::N;
+  for (int lh = (int)ls - 1; lh >= 0; lh--) {  // pairs (j, j + 2^lh) of every row / column
+    const uint32_t sg = item >> lh, j = item & ((1u << lh) - 1);
+    if (sg < nseg) {
+      const uint32_t at = (sg << ls) + j;
+      typename LT::Pt v = LT::load(sh[at]);
+      xyzz_add_lx(v, LT::load(sh[at + (1u << lh)]));
+      LT::store(sh[at], v);
+    }
+    __syncthreads();
   }
-  xyzz<R> tot = wg_sum<F, LN, R>(acc, sh, T);
-  if (t == 0) LN::store(P[blockIdx.x], tot);
+  if (item < nseg) {
+    const uint32_t sg = blockIdx.x * nseg + item;
+    if (sg < segs) LT::store((cols ? X : Y)[sg], LT::load(sh[item << ls]));
+  }
 }
 
 // A point from the lane `lanes` above (ds_bpermute per 32-bit word); every
 // lane of the wave must execute it.
-template <class R>
-__device__ __forceinline__ xyzz<R> shfl_down_pt(const xyzz<R>& p, int lanes) {
-  xyzz<R> q;
+template <class Pt>
+__device__ __forceinline__ Pt shfl_down_pt(const Pt& p, int lanes) {
+  Pt q;
   const uint32_t* s = reinterpret_cast<const uint32_t*>(&p);
   uint32_t* d = reinterpret_cast<uint32_t*>(&q);
 #pragma unroll
-  for (int i = 0; i < (int)(sizeof(xyzz<R>) / 4); i++) d[i] = (uint32_t)__shfl_down((int)s[i], lanes, 64);
+  for (int i = 0; i < (int)(sizeof(Pt) / 4); i++) d[i] = (uint32_t)__shfl_down((int)s[i], lanes, 64);
   return q;
 }
 
-// Level 2: one workgroup of two waves per window over its K group results
-// (K a power of two, at most one wave of items).  With P_k and RUN_k of the
-// strided groups above,
-//   sum_b (b+1) S_b = sum_k [(k+1) RUN_k + K (P_k - RUN_k)]
-//                   = sum_k [SR_k + K (P_k - RUN_k)],  SR_k = sum_{k' >= k} RUN_k'.
-// Wave 1 forms K (P_k - RUN_k) (log2 K doublings) while wave 0 forms the
-// suffix sums with lane shuffles; wave 0 then adds them and sums the items.
-// plain (when not null) gets the window's plain bucket sum SR_0.
-template <class F, class LN>
-__global__ __launch_bounds__(128) void k_msm_reduce2(const xyzz<F>* __restrict__ P, const xyzz<F>* __restrict__ RUN,
-                                                     uint32_t K, int log2k, xyzz<F>* __restrict__ out,
-                                                     xyzz<F>* __restrict__ plain) {
-  typedef typename LN::R R;
-  msm_priority<F>();
-  __shared__ xyzz<F> ku[64];
-  const uint32_t w = blockIdx.x;
-  const uint32_t t = (threadIdx.x & 63) / LN::N;  // item within its wave
-  const bool wave0 = threadIdx.x < 64;
-  xyzz<R> v;
-  xyzz_set_inf(v);
-  if (!wave0) {
-    if (t < K) {
-      xyzz<R> r = LN::load(RUN[w * K + t]);
-      v = LN::load(P[w * K + t]);
-      r.y = fneg(r.y);
-      xyzz_add_lx(v, r);
-      for (int d = 0; d < log2k; d++) xyzz_dbl_lx(v);
-      LN::store(ku[t], v);
+// Weighted sum of the 2^ln values of window blockIdx.x, part blockIdx.y: part
+// 0 the column sums X (or the buckets themselves, with their bounds; weights i +
+// 1), part 1 the row sums Y (weights i).  i = r b + c with b = 2^lb columns: the
+// b column sums and a = 2^(ln - lb) row sums (a, b <= 16) are formed by trees,
+// then out[0] = sum_c (c + 1 or c) col_c and out[1] = sum_r r row_r (to be taken
+// b times).  plain (part 0, when not null): the sum of all values.
+// G2 adds b times out[1] to out[0] here instead (log2 b doublings): a point more
+// costs the host about 1 us over Fq2 (0.3 us over Fq), and there are two or four
+// per window (62779 points, 26 windows: 930 -> 890 us; G1 2^20 lost 12 us this way).
+template <class F>
+constexpr bool weigh_merge() {
+  return sizeof(F) == sizeof(fq2);
+}
+// NMAX: most values of a window part (a block of NMAX items; fewer items leave
+// each lane more registers).
+template <class F, int NMAX>
+__global__ __launch_bounds__(NMAX * SplitLanes<F>::N) void k_msm_weigh(
+    const xyzz<F>* __restrict__ X, const xyzz<F>* __restrict__ Y, const uint32_t* __restrict__ start,
+    const uint32_t* __restrict__ end, uint32_t W_set, int lnx, int lny, xyzz<F>* __restrict__ out,
+    xyzz<F>* __restrict__ plain) {
+  typedef SplitLanes<F> LN;
+  typedef typename LN::Pt Pt;
+  msm_reduce_priority();
+  __shared__ xyzz<F> U[NMAX / 2], V[NMAX / 2];
+  const uint32_t w = blockIdx.x, part = blockIdx.y;
+  const int ln = part ? lny : lnx, lb = (ln + 1) / 2, la = ln - lb;
+  const uint32_t n = 1u << ln, a = 1u << la, b = 1u << lb;
+  const xyzz<F>* src = (part ? Y : X) + ((size_t)w << ln);
+  const uint32_t sb = (w % W_set) << ln;
+  auto value = [&](uint32_t i) {
+    if (start && end[sb + i] <= start[sb + i]) {
+      Pt z;
+      xyzz_set_inf(z);
+      return z;
     }
-  } else {
-    if (t < K) v = LN::load(RUN[w * K + t]);
-    for (uint32_t d = 1; d < K; d <<= 1) {  // inclusive suffix scan
-      const xyzz<R> o = shfl_down_pt(v, (int)(d * LN::N));
-      if (t + d < K) xyzz_add_lx(v, o);
-    }
-    if (plain && t == 0) LN::store(plain[w], v);
+    return LN::load(src[i]);
+  };
+  // rows on the first n / 2 items, columns on the next: the first tree level
+  // from global memory, the others in place
+  const uint32_t item = threadIdx.x / LN::N;
+  if (item < n / 2) {
+    const uint32_t r = item >> (lb - 1), c = item & (b / 2 - 1);
+    Pt v = value((r << lb) + c);
+    xyzz_add_lx(v, value((r << lb) + c + b / 2));
+    LN::store(U[item], v);
+  } else if (item < n) {
+    const uint32_t j = item - n / 2;
+    Pt v = value(j);
+    xyzz_add_lx(v, value(j + n / 2));
+    LN::store(V[j], v);
   }
   __syncthreads();
-  if (wave0) {
-    if (t < K) xyzz_add_lx(v, LN::load(ku[t]));
-    for (uint32_t d = K / 2; d >= 1; d >>= 1) {  // tree sum into item 0
-      const xyzz<R> o = shfl_down_pt(v, (int)(d * LN::N));
-      if (t < d) xyzz_add_lx(v, o);
+  for (int i = 2; i <= lb; i++) {
+    if (item < n / 2) {
+      const int lh = lb - i;
+      const uint32_t r = item >> lh, at = (r << (lb - 1)) + (item & ((1u << lh) - 1));
+      if (r < a) {
+        Pt v = LN::load(U[at]);
+        xyzz_add_lx(v, LN::load(U[at + (1u << lh)]));
+        LN::store(U[at], v);
+      }
+    } else if (i <= la && item < n) {
+      const uint32_t j = item - n / 2, h = (a >> i) << lb;  // values left after this level
+      if (j < h) {
+        Pt v = LN::load(V[j]);
+        xyzz_add_lx(v, LN::load(V[j + h]));
+        LN::store(V[j], v);
+      }
     }
-    if (t == 0) LN::store(out[w], v);
+    __syncthreads();
   }
+  // 16 row sums, then 16 column sums: suffix sums, and the sum of the suffixes
+  // (of those past the first for weights that start at 0)
+  const uint32_t k = item & 15;
+  const bool row = item < 16;
+  Pt v;
+  xyzz_set_inf(v);
+  if (item < 32) {
+    if (row && k < a) v = LN::load(U[k << (lb - 1)]);
+    if (!row && k < b) v = LN::load(V[k]);
+    for (uint32_t d = 1; d < 16; d <<= 1) {
+      const Pt o = shfl_down_pt(v, (int)(d * LN::N));
+      if (k + d < 16) xyzz_add_lx(v, o);
+    }
+    if (plain && part == 0 && !row && k == 0) LN::store(plain[w], v);
+    if (k == 0 && (row || part)) xyzz_set_inf(v);
+    for (uint32_t d = 8; d >= 1; d >>= 1) {
+      const Pt o = shfl_down_pt(v, (int)(d * LN::N));
+      if (k < d) xyzz_add_lx(v, o);
+    }
+  }
+  const size_t at = (size_t)w * gridDim.y + part;
+  if constexpr (!weigh_merge<F>()) {
+    if (item < 32 && k == 0) LN::store(out[at * 2 + (row ? 1 : 0)], v);
+  } else {
+    __syncthreads();
+    if (item == 16) LN::store(V[0], v);
+    __syncthreads();
+    if (item == 0) {
+      for (int d = 0; d < lb; d++) xyzz_dbl_lx(v);
+      xyzz_add_lx(v, LN::load(V[0]));
+      LN::store(out[at], v);
+    }
+  }
+}
+
+// Shape of the reduction of windows of 2^l buckets: the points k_msm_weigh
+// leaves per window and the bit offset of each.
+struct RedShape {
+  int l, lc, parts, npts;
+  int offs[4];
+};
+// Windows small enough go to k_msm_weigh directly: 2^8 buckets for G1, 2^7 for
+// G2 (512 lanes either way; 1024 would leave 128 registers, too few for Fq2).
+static RedShape red_shape(int l, bool g2) {
+  RedShape r{};
+  r.l = l;
+  if (l <= (g2 ? 7 : 8)) {
+    r.parts = 1;
+    r.lc = l;
+  } else {
+    r.parts = 2;
+    r.lc = (l + 1) / 2;
+  }
+  if (g2 ? weigh_merge<fq2>() : weigh_merge<fq>()) {
+    r.npts = r.parts;
+    r.offs[1] = r.lc;
+    return r;
+  }
+  r.npts = 2 * r.parts;
+  r.offs[0] = 0;
+  r.offs[1] = (r.lc + 1) / 2;
+  r.offs[2] = r.lc;
+  r.offs[3] = r.lc + (l - r.lc + 1) / 2;
+  return r;
 }
 
 // ------------------------------------------------------------------ workspace
 constexpr int MSM_MAX_W = 32;   // windows of the narrowest window (8 bits)
-constexpr int MSM_PARTS = 192;  // window (or sub-window) partials of one MSM, all sets
+constexpr int MSM_PARTS = 512;  // points of one MSM's reduction, all windows (or sub-windows) and sets
 
 struct MsmWorkspace {
   DevBuf recs, dig, hist, tot, lex, bsum, bmax, boff, tmp, sorted, start, end, wstat, buckets, hkey, tkey, hpt, tpt,
@@ -1503,13 +1587,12 @@ static void host_result(const zkh::Jac<typename HostSide<F>::E>& r, bool jac_out
   HostSide<F>::out(ax, ay, out);
 }
 
-// XYZZ partials (device layout, copied to the host) -> affine via one batch
-// inversion -> per-window sums -> Horner over windows.
+// XYZZ points (device layout, copied to the host) as affine points, by one
+// batch inversion.
 template <class F>
-static void host_finish(const std::vector<xyzz<F>>& parts, int W, int per_w, uint64_t* out, bool jac_out) {
+static std::vector<zkh::Jac<typename HostSide<F>::E>> host_points(const xyzz<F>* parts, size_t m) {
   typedef typename HostSide<F>::E E;
   typedef zkh::Jac<E> J;
-  const size_t m = parts.size();
   std::vector<E> X(m), Y(m), ZZ(m), ZZZ(m), prod(m);
   std::vector<char> inf(m);
   E acc = E::one();
@@ -1523,21 +1606,30 @@ static void host_finish(const std::vector<xyzz<F>>& parts, int W, int per_w, uin
     if (!inf[i]) acc = acc * (ZZ[i] * ZZZ[i]);
   }
   E inv = acc.inv();
-  std::vector<J> win(W, J::inf());
+  std::vector<J> pt(m, J::inf());
   for (size_t i = m; i-- > 0;) {
     if (inf[i]) continue;
-    E d = ZZ[i] * ZZZ[i];
-    E di = inv * prod[i];
+    const E d = ZZ[i] * ZZZ[i];
+    const E di = inv * prod[i];
     inv = inv * d;
-    E x = X[i] * (di * ZZZ[i]);  // X / ZZ
-    E y = Y[i] * (di * ZZ[i]);   // Y / ZZZ
-    const int w = (int)(i / per_w);
-    win[w] = win[w].add(J::affine(x, y));
+    pt[i] = J::affine(X[i] * (di * ZZZ[i]), Y[i] * (di * ZZ[i]));  // X / ZZ, Y / ZZZ
   }
-  J r = win[W - 1];
-  for (int w = W - 2; w >= 0; w--) {
-    for (int k = 0; k < window_width(w, W); k++) r = r.dbl();
-    r = r.add(win[w]);
+  return pt;
+}
+
+// sum_w 2^(bits below window w) (sum_j 2^offs[j] pts[w][j]) over W windows:
+// Horner over the offsets from the top.
+template <class F>
+static void host_finish(const xyzz<F>* parts, int W, const RedShape& rs, uint64_t* out, bool jac_out) {
+  typedef zkh::Jac<typename HostSide<F>::E> J;
+  const std::vector<J> pt = host_points<F>(parts, (size_t)W * rs.npts);
+  J r = J::inf();
+  for (int w = W - 1; w >= 0; w--) {
+    int at = window_width(w, W);
+    for (int j = rs.npts - 1; j >= 0; j--) {
+      for (; at > rs.offs[j]; at--) r = r.dbl();
+      r = r.add(pt[(size_t)w * rs.npts + j]);
+    }
   }
   host_result<F>(r, jac_out, out);
 }
@@ -1787,125 +1879,89 @@ static int msm_accumulate(zk_context* ctx, MsmWorkspace& ws, const MsmShape& sh,
   return ZK_OK;
 }
 
-// Bucket reduction of Wr windows of Br buckets per set (level 1: T threads
-// x G buckets per group, level 2 per window); the window sums sum_b (b+1) S_b
-// (set-major) are copied to the pinned ws.h_parts on st, followed, with
+// Bucket reduction of Wr windows of 2^rs.l buckets per set: rs.npts points per
+// window (set-major) are copied to the pinned ws.h_parts on st, followed, with
 // `plain`, by the windows' plain sums sum_b S_b.
 template <class F>
-static int msm_reduce(zk_context* ctx, MsmWorkspace& ws, int Wr, uint32_t Br, int nsets, bool beside, bool plain,
+static int msm_reduce(zk_context* ctx, MsmWorkspace& ws, int Wr, const RedShape& rs, int nsets, bool plain,
                       hipStream_t st) {
   typedef SplitLanes<F> SL;
-  const uint32_t B = Br;
-  // items per workgroup (a G2 item is a lane pair: 256 lanes either way)
-  constexpr int TMAX = sizeof(F) == sizeof(fq) ? 256 : 128;
-  constexpr int KMAX = 64 / Lanes<F>::N;  // level 2 holds the K groups of a window in one wave
-  // Level 1 splits its point operations (SplitLanes) when the plain layout
-  // would fill at most half of the SIMDs.  Alone on the GPU a split
-  // workgroup takes half the items (256 lanes, one wave per SIMD) and a
-  // window twice the groups, so the chains spread over more CUs instead of
-  // sharing SIMDs (G1 2^16 0.58 -> 0.53 ms, G2 2^16 1.08 -> 1.00 ms); beside
-  // other MSMs it keeps the full items (fewer workgroups find CU slots
-  // sooner: proofs 3-5% shorter that way).  At 2^15 buckets per window and
-  // one wave per SIMD splitting lost (G1 2^20: 0.28 -> 0.31 ms), and so did
-  // G = 4 there (0.37 ms).
-  const bool split1 = (size_t)Wr * nsets * B / 4 * Lanes<F>::N <= (size_t)512 * 64;
-  const bool half1 = split1 && !beside;
-  const int TM = half1 ? TMAX / 2 : TMAX;
-  // measured: T = TMAX; G = 8 for 2^15 buckets per window, else 4
-  int T1 = TM, log2g = B >= 32768 ? 3 : 2;
-  // shrink the group for small windows: T1 * G <= B
-  while (log2g > 0 && (T1 << log2g) > (int)B) log2g--;
-  while (T1 > 1 && (T1 << log2g) > (int)B) T1 >>= 1;
-  uint32_t K = B / ((uint32_t)T1 << log2g);
-  while (K > KMAX) {  // too many groups for level 2: widen the groups
-    log2g++;
-    K >>= 1;
-  }
-  if (T1 < 1 || T1 > TM || (T1 & (T1 - 1)) || K < 1 || (size_t)K * ((size_t)T1 << log2g) != B)
-    return ctx->fail(ZK_ERR_INVALID, "msm: unsupported reduction shape");
   const uint32_t WS = (uint32_t)Wr * nsets;  // windows of all sets
-  if (WS > MSM_PARTS) return ctx->fail(ZK_ERR_INVALID, "msm: too many windows");
-  ZK_TRY(ctx->ensure(ws.seg, (size_t)K * WS * sizeof(xyzz<F>)));
-  ZK_TRY(ctx->ensure(ws.grp, (size_t)K * WS * sizeof(xyzz<F>)));
-  ZK_TRY(ctx->ensure(ws.win, (size_t)2 * WS * sizeof(xyzz<F>)));
+  const size_t npts = (size_t)WS * rs.npts + (plain ? WS : 0);
+  if (npts > MSM_PARTS || rs.l < 7 || rs.l > 16) return ctx->fail(ZK_ERR_INVALID, "msm: unsupported reduction shape");
+  ZK_TRY(ctx->ensure(ws.win, npts * sizeof(xyzz<F>)));
   const xyzz<F>* buckets = (const xyzz<F>*)ws.buckets.p;
   const uint32_t* start = (const uint32_t*)ws.start.p;
   const uint32_t* end = (const uint32_t*)ws.end.p;
-  xyzz<F>* Pk = (xyzz<F>*)ws.seg.p;
-  xyzz<F>* RUNk = (xyzz<F>*)ws.grp.p;
   xyzz<F>* win = (xyzz<F>*)ws.win.p;
-  xyzz<F>* pln = plain ? win + WS : nullptr;
-  if (half1) {
-    ZK_LAUNCH(ctx, st, "msm_reduce", (k_msm_reduce1<F, TMAX / 2, SL>), dim3(K * WS), dim3(T1 * SL::N), 0, buckets,
-              start, end, B, K, (uint32_t)Wr, log2g, Pk, RUNk);
-  } else if (split1) {
-    ZK_LAUNCH(ctx, st, "msm_reduce", (k_msm_reduce1<F, TMAX, SL>), dim3(K * WS), dim3(T1 * SL::N), 0, buckets, start,
-              end, B, K, (uint32_t)Wr, log2g, Pk, RUNk);
-  } else {
-    ZK_LAUNCH(ctx, st, "msm_reduce", (k_msm_reduce1<F, TMAX, Lanes<F>>), dim3(K * WS), dim3(T1 * Lanes<F>::N), 0,
-              buckets, start, end, B, K, (uint32_t)Wr, log2g, Pk, RUNk);
+  xyzz<F>* pln = plain ? win + (size_t)WS * rs.npts : nullptr;
+  const int lr = rs.l - rs.lc;
+  if (rs.parts == 2) {
+    ZK_TRY(ctx->ensure(ws.seg, ((size_t)WS << rs.lc) * sizeof(xyzz<F>)));
+    ZK_TRY(ctx->ensure(ws.grp, ((size_t)WS << lr) * sizeof(xyzz<F>)));
+    xyzz<F>* X = (xyzz<F>*)ws.seg.p;
+    xyzz<F>* Y = (xyzz<F>*)ws.grp.p;
+    // 8 buckets per item where that gives every SIMD a wave (two of them fill it:
+    // a wave alone issues at about 0.7 of the rate), else 4, on split lanes, which
+    // shortens the chains and fills the chip with twice the lanes.  Measured (G1
+    // 2^16, 24 windows of 2^10 buckets): split 437 us, not split 463 us; at 2^20
+    // (16 of 2^15) split 1.83 ms, not split 1.80 ms.
+    const size_t lanes8 = ((size_t)2 * WS << rs.l) / 8 * Lanes<F>::N;
+    const bool split = lanes8 < (size_t)1024 * 64;
+    const int log2g = std::min(split ? 2 : 3, lr);
+    const uint32_t items = split ? 256 / SL::N : 256 / Lanes<F>::N;
+    const dim3 grid(cdiv((size_t)WS << (rs.l - log2g), items), 2);
+    if (split)
+      ZK_LAUNCH(ctx, st, "msm_reduce", (k_msm_rowcol<F, SL>), grid, dim3(256), 0, buckets, start, end, WS,
+                (uint32_t)Wr, rs.l, rs.lc, log2g, X, Y);
+    else
+      ZK_LAUNCH(ctx, st, "msm_reduce", (k_msm_rowcol<F, Lanes<F>>), grid, dim3(256), 0, buckets, start, end, WS,
+                (uint32_t)Wr, rs.l, rs.lc, log2g, X, Y);
   }
-  int log2k = 0;
-  while ((1u << log2k) < K) log2k++;
-  // one group per window: its P is the window sum (no level-2 launch, which
-  // beside other MSMs would wait for a CU with room for its two waves); level
-  // 2 holds a window's K groups in one wave, split when they fit
-  if (K > 1 && K * SL::N <= 64) {
-    ZK_LAUNCH(ctx, st, "msm_reduce2", (k_msm_reduce2<F, SL>), dim3(WS), dim3(128), 0, Pk, RUNk, K, log2k, win, pln);
-  } else if (K > 1) {
-    ZK_LAUNCH(ctx, st, "msm_reduce2", (k_msm_reduce2<F, Lanes<F>>), dim3(WS), dim3(128), 0, Pk, RUNk, K, log2k, win,
-              pln);
-  }
+  // the weighted sums: of the row and column sums, or of the buckets themselves
+  const bool direct = rs.parts == 1;
+  const xyzz<F>* X = direct ? buckets : (const xyzz<F>*)ws.seg.p;
+  const xyzz<F>* Y = (const xyzz<F>*)ws.grp.p;
+  const uint32_t* vs = direct ? start : nullptr;
+  const uint32_t* ve = direct ? end : nullptr;
+  const dim3 wg(WS, rs.parts), wb(std::max(32u, 1u << rs.lc) * SL::N);
+  if (rs.lc <= 6)
+    ZK_LAUNCH(ctx, st, "msm_reduce2", (k_msm_weigh<F, 64>), wg, wb, 0, X, Y, vs, ve, (uint32_t)Wr, rs.lc, lr, win, pln);
+  else if (rs.lc == 7)
+    ZK_LAUNCH(ctx, st, "msm_reduce2", (k_msm_weigh<F, 128>), wg, wb, 0, X, Y, vs, ve, (uint32_t)Wr, rs.lc, lr, win, pln);
+  else
+    ZK_LAUNCH(ctx, st, "msm_reduce2", (k_msm_weigh<F, 256>), wg, wb, 0, X, Y, vs, ve, (uint32_t)Wr, rs.lc, lr, win, pln);
   // pinned destination: a copy to pageable memory costs a staged transfer
   // (measured: G1 2^16 MSM 0.535 -> 0.505 ms, the 2^16 proof 1.70 -> 1.62 ms)
-  ZK_HIP(ctx, hipMemcpyAsync(ws.h_parts, K > 1 ? win : Pk, (size_t)WS * sizeof(xyzz<F>), hipMemcpyDeviceToHost, st));
-  // with one group per window the plain sum is that group's RUN
-  if (plain)
-    ZK_HIP(ctx, hipMemcpyAsync((xyzz<F>*)ws.h_parts + WS, K > 1 ? pln : RUNk, (size_t)WS * sizeof(xyzz<F>),
-                               hipMemcpyDeviceToHost, st));
+  ZK_HIP(ctx, hipMemcpyAsync(ws.h_parts, win, npts * sizeof(xyzz<F>), hipMemcpyDeviceToHost, st));
   return ZK_OK;
 }
 
-// Window-table MSM: one bucket space split into H sub-windows of 2^log_sub
-// buckets; P[h] = sum_b (b+1) S_{h,b}, R[h] = sum_b S_{h,b} (device XYZZ).
-// The sum over all buckets of (h 2^log_sub + b + 1) S_{h,b} is
-//   sum_h P[h] + 2^log_sub sum_h h R[h],
-// the second sum as running sums from the top sub-window down.
+// Window-table MSM: one bucket space split into H sub-windows of 2^rs.l
+// buckets; P: rs.npts points per sub-window with P_h = sum_j 2^offs[j] P[h][j] =
+// sum_b (b+1) S_{h,b}, R[h] = sum_b S_{h,b} (only for H > 1).  The sum over all
+// buckets of (h 2^l + b + 1) S_{h,b} is
+//   sum_h P_h + 2^l sum_h h R[h],
+// the first sum point by point before its one Horner pass, the second as
+// running sums from the top sub-window down.
 template <class F>
-static void host_finish_sub(const xyzz<F>* P, const xyzz<F>* R, int H, int log_sub, uint64_t* out, bool jac_out) {
-  typedef typename HostSide<F>::E E;
-  typedef zkh::Jac<E> J;
-  const size_t m = 2 * (size_t)H;
-  std::vector<E> X(m), Y(m), ZZ(m), ZZZ(m), prod(m);
-  std::vector<char> inf(m);
-  E acc = E::one();
-  for (size_t i = 0; i < m; i++) {
-    const xyzz<F>& q = i < (size_t)H ? P[i] : R[i - H];
-    X[i] = HostSide<F>::conv(q.x);
-    Y[i] = HostSide<F>::conv(q.y);
-    ZZ[i] = HostSide<F>::conv(q.zz);
-    ZZZ[i] = HostSide<F>::conv(q.zzz);
-    inf[i] = ZZ[i].is_zero();
-    prod[i] = acc;
-    if (!inf[i]) acc = acc * (ZZ[i] * ZZZ[i]);
-  }
-  E inv = acc.inv();
-  std::vector<J> pt(m, J::inf());
-  for (size_t i = m; i-- > 0;) {
-    if (inf[i]) continue;
-    E d = ZZ[i] * ZZZ[i];
-    E di = inv * prod[i];
-    inv = inv * d;
-    pt[i] = J::affine(X[i] * (di * ZZZ[i]), Y[i] * (di * ZZ[i]));
-  }
-  J run = J::inf(), weighted = J::inf(), sum = J::inf();
+static void host_finish_sub(const xyzz<F>* P, const xyzz<F>* R, int H, const RedShape& rs, uint64_t* out,
+                            bool jac_out) {
+  typedef zkh::Jac<typename HostSide<F>::E> J;
+  std::vector<xyzz<F>> parts(P, P + (size_t)H * rs.npts);
+  if (H > 1) parts.insert(parts.end(), R, R + H);
+  const std::vector<J> pt = host_points<F>(parts.data(), parts.size());
+  J run = J::inf(), r = J::inf();  // r: sum_h h R[h], then the total
   for (int h = H - 1; h >= 1; h--) {
-    run = run.add(pt[H + h]);
-    weighted = weighted.add(run);
+    run = run.add(pt[(size_t)H * rs.npts + h]);
+    r = r.add(run);
   }
-  for (int k = 0; k < log_sub; k++) weighted = weighted.dbl();
-  for (int h = 0; h < H; h++) sum = sum.add(pt[h]);
-  host_result<F>(sum.add(weighted), jac_out, out);
+  int at = rs.l;
+  for (int j = rs.npts - 1; j >= 0; j--) {
+    for (; at > rs.offs[j]; at--) r = r.dbl();
+    for (int h = 0; h < H; h++) r = r.add(pt[(size_t)h * rs.npts + j]);
+  }
+  host_result<F>(r, jac_out, out);
 }
 
 // MSMs of `nsets` point sets over one scalar vector of n entries (see
@@ -1973,7 +2029,7 @@ static int msm_run_sets(zk_context* ctx, MsmWorkspace& ws, const BaseSets& sets_
   ZK_TRY(ctx->ensure(ws.buckets, nsets * nbuckets * sizeof(xyzz<F>)));
   if (!ws.h_stat) ZK_HIP(ctx, hipHostMalloc((void**)&ws.h_stat, 2 * MSM_MAX_W * 4, hipHostMallocDefault));
   if (!ws.h_parts)
-    ZK_HIP(ctx, hipHostMalloc(&ws.h_parts, 2 * MSM_PARTS * sizeof(xyzz<fq2>), hipHostMallocDefault));
+    ZK_HIP(ctx, hipHostMalloc(&ws.h_parts, MSM_PARTS * sizeof(xyzz<fq2>), hipHostMallocDefault));
   if (!ws.stat_ready) ZK_HIP(ctx, hipEventCreateWithFlags(&ws.stat_ready, hipEventDisableTiming));
 
   ZK_LAUNCH(ctx, st, "msm_digits", k_msm_digits, dim3(cdiv(n, 256)), dim3(256), 0, (uint32_t*)ws.dig.p,
@@ -1993,8 +2049,10 @@ static int msm_run_sets(zk_context* ctx, MsmWorkspace& ws, const BaseSets& sets_
   ZK_TRY(msm_accumulate<F>(ctx, ws, sh, sets, nsets, ap, beside, st));
   // a window table's bucket space reduces as sub-windows of 2^log_sub buckets
   const int Wr = tab ? (int)(sh.B >> tab->log_sub) : W;
-  const uint32_t Br = tab ? 1u << tab->log_sub : sh.B;
-  ZK_TRY(msm_reduce<F>(ctx, ws, Wr, Br, nsets, beside, tab != nullptr, st));
+  int l = 0;
+  while ((2u << l) <= (tab ? 1u << tab->log_sub : sh.B)) l++;
+  const RedShape rs = red_shape(l, G2);
+  ZK_TRY(msm_reduce<F>(ctx, ws, Wr, rs, nsets, tab != nullptr && Wr > 1, st));
   ZK_HIP(ctx, hipStreamSynchronize(st));
   const xyzz<F>* parts = (const xyzz<F>*)ws.h_parts;
   // window combination on the host (W * c doublings per set): one thread per set
@@ -2002,11 +2060,10 @@ static int msm_run_sets(zk_context* ctx, MsmWorkspace& ws, const BaseSets& sets_
   auto finish = [&](int k) {
     try {
       if (tab)
-        host_finish_sub<F>(parts + (size_t)k * Wr, parts + (size_t)(nsets + k) * Wr, Wr, tab->log_sub, outs[k],
-                           jac_out);
+        host_finish_sub<F>(parts + (size_t)k * Wr * rs.npts, parts + (size_t)nsets * Wr * rs.npts + (size_t)k * Wr,
+                           Wr, rs, outs[k], jac_out);
       else
-        host_finish<F>(std::vector<xyzz<F>>(parts + (size_t)k * W, parts + (size_t)(k + 1) * W), W, 1, outs[k],
-                       jac_out);
+        host_finish<F>(parts + (size_t)k * W * rs.npts, W, rs, outs[k], jac_out);
     } catch (...) {
       rc_fin[k] = ZK_ERR_OOM;
     }

@@ -415,3 +415,31 @@ def test_msm_g2_host_reference_layout(ctx):
     assert np.array_equal(out[:16], expect)
     # z = 1 in Fq2 (Montgomery): c0 = 1, c1 = 0
     assert Z.from_mont(Z.from_limbs(out[16:20]), Z.P) == 1 and not out[20:24].any()
+
+
+@pytest.mark.parametrize("g2,n", [(False, 60), (False, 33000), (False, 65537), (False, 140001), (False, 300007),
+                                  (True, 60), (True, 9000), (True, 70001), (True, 140001)])
+def test_msm_bucket_reduction_shapes(ctx, g2, n):
+    """The window sizes' bucket reductions (windows reduced directly and by row
+    and column sums, square and not, few and many buckets per item), with
+    digits that hit the first and last bucket, rows and columns of a window and
+    with windows that hold one bucket or none: sum k_i s_i over ragged n."""
+    import zkml_amd
+    rng = np.random.default_rng(n + g2)
+    kstd = rand_std(n, rng)
+    dp = gpu_points(ctx, to_mont(kstd), g2=g2)
+    run = ctx.msm_g2 if g2 else ctx.msm_g1
+    G, gen, from_words = (Z.g2, Z.G2, Z.g2_from_words) if g2 else (Z.g1, Z.G1, Z.g1_from_words)
+    c, _ = zkml_amd.Context.msm_config(n, g2)
+    half = 1 << (c - 1)
+    lists = {
+        "uniform": rand_std(n, rng),
+        "edges": std_words([(half, half - 1, 1, 2, 16, 17, half // 2, half // 2 + 1)[i % 8] for i in range(n)]),
+        "one bucket": std_words([half - 1] * n),
+        "sparse": std_words([0] * n),
+    }
+    lists["sparse"][::max(1, n // 7)] = rand_std(len(lists["sparse"][::max(1, n // 7)]), rng)
+    for name, s in lists.items():
+        print(f"[msm shapes {'g2' if g2 else 'g1'} {n} c={c}] {name}", flush=True)
+        got = run(dp, ctx.upload(to_mont(s)), n)
+        assert from_words(got) == G.pmul(gen, closed_form_scalar(kstd, s)), name
