@@ -25,6 +25,7 @@
 
 #if defined(__HIPCC__)
 #include <hip/hip_runtime.h>
+#include "const_mul_asm.hpp"
 #include "mont_asm.hpp"
 #define ZK_HD __host__ __device__ __forceinline__
 #else
@@ -82,6 +83,10 @@ struct FrP {
   static constexpr uint32_t INV = 0x0fffffffu;  // -r^-1 mod 2^29
   static constexpr uint32_t EDIG[9] = {0x08f05368u, 0x1a996a5bu, 0x13e27f6bu, 0x15166c9eu, 0x1e906a17u,
                                        0x04c58463u, 0x16877334u, 0x0b82ba37u, 0x016af04cu};  // (r k + 1) / 2^29, k = -r^-1 mod 2^32
+  static constexpr uint32_t NEGMOD[9] = {0x0fffffffu, 0x00f05360u, 0x11a3dbafu, 0x182f6f0cu, 0x0a7a2d7cu,
+                                         0x1d24bf3fu, 0x1f591ebeu, 0x11a3d9cbu, 0x1fcf9bb1u};  // 2^261 - r
+  static constexpr uint32_t NINV[9] = {0x0fffffffu, 0x170fac9fu, 0x1a446cf0u, 0x0d0c9698u, 0x02391658u,
+                                       0x0c144c83u, 0x06cb8e6au, 0x03a1b068u, 0x1273f82fu};  // -r^-1 mod 2^261
   static constexpr uint32_t ONE[9] = {0x0fffff57u, 0x1ea70ab4u, 0x052c068bu, 0x17504f49u, 0x0aa8075bu,
                                       0x1d4240ceu, 0x11d54c07u, 0x052ac7a8u, 0x000dc836u};  // 2^261 mod r
   static constexpr uint32_t R2[9] = {0x05b69bd4u, 0x06170a5au, 0x020cddceu, 0x1db6310bu, 0x0e54d0ffu,
@@ -257,6 +262,97 @@ ZK_HD fe<P> fsqr(const fe<P>& a) {
 #endif
 }
 
+// a w mod m for a constant w (canonical, not Montgomery) with its quotient wq =
+// floor(w 2^261 / m): q = floor(a wq / 2^261) from the columns 7 and up of a wq,
+// then a w - q m from the low nine columns, modulo 2^261.  The dropped columns
+// and the two floors leave q short by less than 2 + 2^-22, so the result is in
+// [0, 2m + m / 2^22), limbs normalized.  a: any value below 2^261 with limbs
+// below LU 2^29 (not normalized).  Columns stay below 2^64: a's products 9 LU
+// 2^58, the quotient's 5.6 * 2^58, with LU <= 5.  Up to LU = 3 the quotient
+// digits may be the columns' low 32 bits as they are (8 * hi goes on, as in the
+// Montgomery products): their products take 36.9 * 2^58 in column 7 (in column 8
+// only the low bits count).
+template <int LU, class P>
+ZK_HD fe<P> fmul_const(const fe<P>& a, const fe<P>& w, const fe<P>& wq) {
+  static_assert(LU >= 1 && LU <= 5, "limb bound");
+#if defined(__HIP_DEVICE_COMPILE__)
+  fe<P> r = wq;
+  if constexpr (LU <= 3)
+    const_mul32_asm<P>(r.l, a.l, w.l);
+  else
+    const_mul29_asm<P>(r.l, a.l, w.l);
+  return r;
+#else
+  uint32_t q[NL];
+  fe<P> r;
+  uint64_t acc = 0;
+  for (int k = NL - 2; k < 2 * NL - 1; k++) {
+    for (int i = k < NL ? 0 : k - NL + 1; i < NL && i <= k; i++) acc += (uint64_t)a.l[i] * wq.l[k - i];
+    if (k < NL) {
+      acc >>= 29;
+    } else if (LU <= 3) {
+      q[k - NL] = (uint32_t)acc;
+      acc = (acc >> 32) * 8;
+    } else {
+      q[k - NL] = (uint32_t)acc & LMASK;
+      acc >>= 29;
+    }
+  }
+  q[NL - 1] = (uint32_t)acc;
+  acc = 0;
+  for (int k = 0; k < NL; k++) {
+    for (int i = 0; i <= k; i++) acc += (uint64_t)a.l[i] * w.l[k - i] + (uint64_t)q[i] * P::NEGMOD[k - i];
+    r.l[k] = (uint32_t)acc & LMASK;
+    acc >>= 29;
+  }
+  return r;
+#endif
+}
+
+// wq = floor(w 2^261 / m) for w in internal form wi = w 2^261 mod m (canonical):
+// w 2^261 = wq m + wi, so wq = wi (-m^-1) modulo 2^261.
+template <class P>
+ZK_HD fe<P> const_quotient(const fe<P>& wi) {
+  fe<P> r;
+  uint64_t acc = 0;
+  for (int k = 0; k < NL; k++) {
+    for (int i = 0; i <= k; i++) acc += (uint64_t)wi.l[i] * P::NINV[k - i];
+    r.l[k] = (uint32_t)acc & LMASK;
+    acc >>= 29;
+  }
+  return r;
+}
+
+// keep ? a : b.  On the device nine v_cndmask with the mask in a scalar register
+// pair: the compiler's form of nine selects on one condition reads it from VCC
+// back to back, where each takes 15 to 23 cycles on gfx950 instead of 4.  (s_nop:
+// the two wait states between a compare that writes the pair and its first
+// reader, which the compiler does not place before an assembly block.)
+template <class P>
+ZK_HD fe<P> fselect(bool keep, const fe<P>& a, const fe<P>& b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  fe<P> r = b;
+  const uint64_t mask = __ballot(keep);
+  asm("s_nop 1\n"
+      "v_cndmask_b32_e64 %0, %0, %9, %18\n"
+      "v_cndmask_b32_e64 %1, %1, %10, %18\n"
+      "v_cndmask_b32_e64 %2, %2, %11, %18\n"
+      "v_cndmask_b32_e64 %3, %3, %12, %18\n"
+      "v_cndmask_b32_e64 %4, %4, %13, %18\n"
+      "v_cndmask_b32_e64 %5, %5, %14, %18\n"
+      "v_cndmask_b32_e64 %6, %6, %15, %18\n"
+      "v_cndmask_b32_e64 %7, %7, %16, %18\n"
+      "v_cndmask_b32_e64 %8, %8, %17, %18\n"
+      : "+&v"(r.l[0]), "+&v"(r.l[1]), "+&v"(r.l[2]), "+&v"(r.l[3]), "+&v"(r.l[4]), "+&v"(r.l[5]), "+&v"(r.l[6]),
+        "+&v"(r.l[7]), "+&v"(r.l[8])
+      : "v"(a.l[0]), "v"(a.l[1]), "v"(a.l[2]), "v"(a.l[3]), "v"(a.l[4]), "v"(a.l[5]), "v"(a.l[6]), "v"(a.l[7]),
+        "v"(a.l[8]), "s"(mask));
+  return r;
+#else
+  return keep ? a : b;
+#endif
+}
+
 // (a + b) mod m into [0, 2m).  Inputs normalized, values < 2m.
 template <class P>
 ZK_HD fe<P> fadd(const fe<P>& a, const fe<P>& b) {
@@ -275,10 +371,7 @@ ZK_HD fe<P> fadd(const fe<P>& a, const fe<P>& b) {
     br = v >> 29;
     t.l[i] = (uint32_t)v & LMASK;
   }
-  // br == -1: s < 2m, keep s.
-#pragma unroll
-  for (int i = 0; i < NL; i++) s.l[i] = br ? s.l[i] : t.l[i];
-  return s;
+  return fselect(br != 0, s, t);  // br == -1: s < 2m, keep s
 }
 
 // (a - b) mod m into [0, 2m).  Inputs normalized, values < 2m.
@@ -348,6 +441,31 @@ ZK_HD fe<P> fneg_wide(const fe<P>& a) {
 #pragma unroll
   for (int i = 0; i < NL; i++) d.l[i] = kwide<P>(i) - a.l[i];
   return d;
+}
+
+// a - b + 4m limb by limb, no carry pass, for a normalized b below 2m + m / 2^22:
+// limbs at most 2^30 above a's.
+template <class P>
+ZK_HD fe<P> fsub_wide(const fe<P>& a, const fe<P>& b) {
+  fe<P> d;
+#pragma unroll
+  for (int i = 0; i < NL; i++) d.l[i] = a.l[i] + (kwide<P>(i) - b.l[i]);
+  return d;
+}
+
+// Carry pass: the same value (below 2^261) with normalized limbs; limbs at most
+// 2^32 - 8 in.
+template <class P>
+ZK_HD fe<P> fcarry(const fe<P>& a) {
+  fe<P> s;
+  uint32_t c = 0;
+#pragma unroll
+  for (int i = 0; i < NL; i++) {
+    const uint32_t v = a.l[i] + c;
+    s.l[i] = v & LMASK;
+    c = v >> 29;
+  }
+  return s;
 }
 
 // neg ? 4m - a : a under a mask, as fneg_wide.
@@ -423,10 +541,7 @@ ZK_HD fe<P> fcanon(const fe<P>& a) {
     br = v >> 29;
     t.l[i] = (uint32_t)v & LMASK;
   }
-  fe<P> r;
-#pragma unroll
-  for (int i = 0; i < NL; i++) r.l[i] = br ? a.l[i] : t.l[i];
-  return r;
+  return fselect(br != 0, a, t);
 }
 
 // a == 0 mod m for a in [0, 2m): a is 0 or m.
@@ -466,10 +581,7 @@ ZK_HD fe<P> fcsub(const fe<P>& t, const uint32_t (&K)[NL]) {
     br = v >> 29;
     u.l[i] = (uint32_t)v & LMASK;
   }
-  fe<P> r;
-#pragma unroll
-  for (int i = 0; i < NL; i++) r.l[i] = br ? t.l[i] : u.l[i];
-  return r;
+  return fselect(br != 0, t, u);
 }
 
 // (a - b - 2c) mod m into [0, 2m) for a, b, c in [0, 2m): one pass forms

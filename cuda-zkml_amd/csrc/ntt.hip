@@ -27,18 +27,23 @@
 //   * the last step writes its outputs straight to HBM, multiplied by the
 //     inter-pass twiddle (or the coset / 1/n factor of the last pass).
 //
-// Butterflies are lazy: u + w v and u - w v + 2m with carries normalised but
-// no modular reduction, so a value grows by at most 2m per stage (w v is a
-// Montgomery product, below 2m).  After the eight stages of a pass it is
-// below 26m, far inside the 2^261 range of nine 29-bit limbs; the pass's
-// output multiply brings it back below 2m, and the last pass reduces to the
-// canonical range.  The inverse transform's 1/n rides in the first
-// inter-pass table, so it costs no multiply.
+// Butterflies are lazy: u + w v and u - w v + 4m limb by limb, with one carry
+// pass per element at the end of a step (limbs stay below 2^32 through its
+// three stages) and no modular reduction: a value grows by at most 4m + per
+// stage (w v is below 2m + m / 2^22), the first step's twiddle-free ones by up to
+// 8m.  After the eight stages of a pass it is below 40m, far inside the 2^261
+// (169m) of nine 29-bit limbs; the pass's output multiply brings it back below
+// 2m, and the last pass reduces to the canonical range.  The twiddles are
+// constants, so their products use a precomputed quotient (fmul_const): with it
+// and without the two carry passes per butterfly a butterfly of a radix-8 step
+// takes 218 instructions instead of 268.  The inverse transform's 1/n rides in
+// the first inter-pass table, so it costs no multiply.
 //
 // Radix bookkeeping: the NTT is linear, so the kernels run directly on the
-// 256-bit words of the reference's Montgomery form (repack only); twiddles and
-// scale tables are prepared in the internal 2^261 radix so that each fmul
-// multiplies the stored integers by the intended field constant.
+// 256-bit words of the reference's Montgomery form (repack only); the inter-pass
+// and scale tables are prepared in the internal 2^261 radix so that each fmul
+// multiplies the stored integers by the intended field constant, the DFT steps'
+// twiddles as plain constants.
 #include <string.h>
 
 #include <utility>
@@ -50,8 +55,9 @@ namespace zk {
 constexpr int NTT_MAX_LOG = 24;
 constexpr int NTT_MAX_LOGR = 8;
 
-// Table of internal-form field elements.  Twiddles of a DFT step (copied to
-// LDS planes) are limb-major: limb l of entry i at l*count + i.  Tables read
+// Table of field elements.  Twiddles of a DFT step (copied to LDS planes) are
+// plain constants with their quotients, limb-major: limb l of entry i at l*count
+// + i, the quotient's limbs after the constant's nine planes.  Tables read
 // per element from HBM (inter-pass twiddles, coset factors) are packed like
 // the elements, 8 words per entry: a tile row of T columns then reads T * 32
 // contiguous bytes, where nine limb planes would read nine runs of T * 4
@@ -78,8 +84,9 @@ struct CosetTables {
   FrTable pre, post_inv, post_fold;
 };
 
-__device__ __forceinline__ void store_table(uint32_t* __restrict__ t, size_t count, size_t i, const fr& x) {
-  fr c = fcanon(x);
+__device__ __forceinline__ void store_table(uint32_t* __restrict__ t, size_t count, size_t i, const fr& x,
+                                            bool reduce = true) {
+  const fr c = reduce ? fcanon(x) : x;
 #pragma unroll
   for (int l = 0; l < NL; l++) t[l * count + i] = c.l[l];
 }
@@ -158,11 +165,19 @@ __device__ __forceinline__ void lds_put(uint32_t* s, uint32_t E, uint32_t ix, co
   for (int l = 0; l < NL; l++) s[l * E + ix] = x.l[l];
 }
 
-__device__ __forceinline__ fr tw_get(const uint32_t* tw, uint32_t half, uint32_t e) {
-  fr x;
+// A twiddle of a DFT step: the constant and its quotient (fmul_const).
+struct Twiddle {
+  fr w, wq;
+};
+constexpr int TW_PLANES = 2 * NL;
+__device__ __forceinline__ Twiddle tw_get(const uint32_t* tw, uint32_t half, uint32_t e) {
+  Twiddle t;
 #pragma unroll
-  for (int l = 0; l < NL; l++) x.l[l] = tw[l * half + e];
-  return x;
+  for (int l = 0; l < NL; l++) {
+    t.w.l[l] = tw[l * half + e];
+    t.wq.l[l] = tw[(NL + l) * half + e];
+  }
+  return t;
 }
 
 // f(integral_constant<int, I>) for I = 0 .. N-1, expanded at compile time so
@@ -176,12 +191,17 @@ __device__ __forceinline__ void unroll(F&& f) {
   unroll_seq(f, std::make_integer_sequence<int, N>{});
 }
 
-// One lazy DIT butterfly with a twiddle: (u + w v, u - w v + 2m).
-__device__ __forceinline__ void bfly(fr& u, fr& v, const fr& w) {
-  const fr t = fmul(v, w);
-  v = fsub_off<2>(u, t);
-  u = fadd_wide(u, t);
+// One lazy DIT butterfly with a twiddle: (u + w v, u - w v + 4m), limb by limb
+// without carry passes.  Limbs of u and v below LU 2^29 become below (LU + 1)
+// 2^29 and (LU + 2) 2^29; w v is normalized and below 2m + m / 2^22.
+template <int LU>
+__device__ __forceinline__ void bfly(fr& u, fr& v, const Twiddle& t) {
+  const fr p = fmul_const<LU>(v, t.w, t.wq);
+  v = fsub_wide(u, p);
+  u = fadd_lazy(u, p);
 }
+// Largest limb bound (units of 2^29) before sub-stage i of a step.
+constexpr int step_units(int i) { return 2 * i + 1; }
 
 // Index of the p-th pair's lower element at sub-stage i (bit i clear).
 template <int I, int P>
@@ -205,9 +225,12 @@ __device__ __forceinline__ void first_step(fr (&x)[1 << K], const uint32_t* tw, 
         x[t] = fadd_wide(u, v);
         x[t + hi] = fsub_off<(i == 0 ? 2 : i == 1 ? 4 : 8)>(u, v);
       } else {
-        bfly(x[t], x[t + hi], tw_get(tw, half, (uint32_t)lo << (logR - 1 - i)));
+        bfly<step_units(i) <= 3 ? step_units(i) : 3>(x[t], x[t + hi], tw_get(tw, half, (uint32_t)lo << (logR - 1 - i)));
       }
     });
+  });
+  unroll<(1 << K)>([&](auto T) {
+    if constexpr ((T & ((1 << (K - 1)) - 1)) != 0) x[T] = fcarry(x[T]);
   });
 }
 
@@ -222,9 +245,10 @@ __device__ __forceinline__ void mid_step(fr (&x)[1 << K], const uint32_t* tw, ui
     unroll<(1 << K) / 2>([&](auto Pp) {
       constexpr int t = pair_lo<i, decltype(Pp)::value>();
       const uint32_t e = (jl + ((uint32_t)(t & (hi - 1)) << s)) << (logR - 1 - s - i);
-      bfly(x[t], x[t + hi], tw_get(tw, half, e));
+      bfly<step_units(i)>(x[t], x[t + hi], tw_get(tw, half, e));
     });
   });
+  unroll<(1 << K)>([&](auto T) { x[T] = fcarry(x[T]); });
 }
 // Tile origin of a pass: middle passes read and write (row r, column c) at
 // base + (r << logS) + c, base = u R S + m0 (m0 = the tile's first column);
@@ -340,8 +364,8 @@ __device__ __forceinline__ void tile_copy_out(const TileCtx& tc, const PassGeo& 
 
 // ---- fixed-geometry tiles: the elements stay in registers between steps
 // and move through LDS in two halves (limbs 0-4, then 5-8) over five planes,
-// so a 2048-element tile takes 45 KB of LDS instead of 78 KB and three
-// blocks (three waves per SIMD) fit on a CU where two did.
+// so a 2048-element tile takes 50 KB of LDS instead of 83 KB and three
+// blocks fit on a CU where one would.
 constexpr int NTT_XPLANES = 5;
 
 // LDS rows of a step of K stages starting at stage s: group gi of the
@@ -436,7 +460,7 @@ __device__ __forceinline__ void tile_fixed(const TileCtx& tc, const PassGeo& g, 
 
 // One pass over tiles of R = 2^logR rows and T = 2^logT columns; block =
 // T*R / 2^min(KMAX, logR) threads; grid = (tiles, batch).  Dynamic LDS: nine
-// planes of T*R words plus nine planes of R/2 twiddles.  Inputs below 2m
+// planes of T*R words plus 18 planes of R/2 twiddles.  Inputs below 2m
 // (canonical words, or the previous pass's outputs).  The DFT runs in steps
 // of KMAX stages, the remainder in the last step.
 //
@@ -448,16 +472,15 @@ __device__ __forceinline__ void tile_fixed(const TileCtx& tc, const PassGeo& g, 
 // from g.
 constexpr uint32_t NTT_TILE_FIXED_LOG = 11;
 
-// Occupancy: the fixed-geometry passes target 3 waves per SIMD, the runtime-
-// geometry radix-8 passes 2.  The small transforms' radix-4 passes (KMAX 2)
-// target 4: they then fit in 96 VGPRs without spills, so in a proof the
-// quotient's passes find room on a SIMD beside three MSM accumulation waves
-// (128 VGPRs each) instead of waiting for one to end (at 3 waves they took
-// 132 VGPRs; config 1 proof 0.543-0.548 -> 0.528-0.536 ms, standalone
-// transforms of 2^12-2^18 points unchanged).
+// Occupancy: the radix-8 passes target 2 waves per SIMD.  At 3 (168 VGPRs) the
+// fixed-geometry ones spill 53 to 74 words, and their 2^11-element tiles come in
+// 2.67 rounds of three per CU at 2^22 instead of 4 of two (2^22 409-411 us at 3,
+// 407-410 at 2; 2^20 121 / 116; three of 2^18 114 / 105).  The smaller radixes
+// target 4 (112 and 76 VGPRs): in a proof the quotient's passes then find room on
+// a SIMD beside MSM accumulation waves instead of waiting for one to end.
 template <int KMAX, bool LAST, int LR = 0>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(LR > 0 ? 3 : KMAX != 3 ? 4 : 2))) void k_ntt_pass(PassGeo g, PassIO io) {
+__attribute__((amdgpu_waves_per_eu(LR > 0 ? 2 : KMAX != 3 ? 4 : 2))) void k_ntt_pass(PassGeo g, PassIO io) {
   quotient_priority();
   extern __shared__ uint32_t smem[];
   constexpr int EPT = 1 << KMAX;
@@ -499,7 +522,7 @@ __attribute__((amdgpu_waves_per_eu(LR > 0 ? 3 : KMAX != 3 ? 4 : 2))) void k_ntt_
   uint32_t* twl = (uint32_t*)tc.tw;
   for (uint32_t e = tc.tid; e < tc.half; e += tc.nthr) {
 #pragma unroll
-    for (int l = 0; l < NL; l++) twl[l * tc.half + e] = io.twr[l * tc.half + e];
+    for (int l = 0; l < TW_PLANES; l++) twl[l * tc.half + e] = io.twr[l * tc.half + e];
   }
   __syncthreads();
   if constexpr (LR > 0) {
@@ -557,7 +580,8 @@ __global__ void k_fill_pow_table(uint32_t* __restrict__ t, size_t count, uint32_
   store_packed(t, e, fmul(r, mul));
 }
 
-// table[e] = base^e * mul, limb-major or packed.
+// table[e] = base^e * mul: packed, or as the limb-major twiddles of a DFT step
+// (the plain constant's nine planes, then its quotient's).
 __global__ void k_fill_pow_linear(uint32_t* __restrict__ t, size_t count, fr base, fr mul, int packed) {
   size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
   if (e >= count) return;
@@ -568,10 +592,15 @@ __global__ void k_fill_pow_linear(uint32_t* __restrict__ t, size_t count, fr bas
     b = fsqr(b);
     ex >>= 1;
   }
-  if (packed)
+  if (packed) {
     store_packed(t, e, fmul(r, mul));
-  else
-    store_table(t, count, e, fmul(r, mul));
+  } else {
+    const fr wi = fcanon(fmul(r, mul));
+    fr one = fe_zero<FrP>();
+    one.l[0] = 1;
+    store_table(t, count, e, fmul(wi, one));
+    store_table(t + NL * count, count, e, const_quotient(wi), false);
+  }
 }
 
 // h = (a*b - c) * zinv on the reference's Montgomery words (kept for callers
@@ -655,7 +684,7 @@ static size_t plan_table_words(const PassShape& sh, int log_n) {
   size_t w = 0;
   int below = log_n;
   for (int q = 0; q < sh.P; q++) {
-    w += 2 * ((size_t)1 << (sh.logR[q] - 1)) * NL;
+    w += 2 * ((size_t)1 << (sh.logR[q] - 1)) * TW_PLANES;
     if (q < sh.P - 1) w += 2 * ((size_t)1 << below) * PACKED_WORDS;
     below -= sh.logR[q];
   }
@@ -710,7 +739,7 @@ static void plan_place(NttPlan* p, uint32_t* words) {
     for (int d = 0; d < 2; d++) {
       p->twr[q][d].count = (size_t)1 << (p->logR[q] - 1);
       p->twr[q][d].d = words;
-      words += p->twr[q][d].count * NL;
+      words += p->twr[q][d].count * TW_PLANES;
       if (q < p->P - 1) {
         p->twp[q][d].count = (size_t)1 << below;
         p->twp[q][d].d = words;
@@ -805,6 +834,11 @@ static int coset_get(zk_context* ctx, int log_n, uint64_t g, const NttPlan* plan
   return ZK_OK;
 }
 
+// Tile of a call's passes: 2^kmax elements per thread, 2^logE per tile.
+struct NttTile {
+  int kmax, logE;
+};
+
 // One transform (or a batch of them) over prepared tables.
 //   src -> dst; mid: n*batch elements for the passes before the last (may be
 //   src when src is writable and differs from dst; never dst);
@@ -818,7 +852,7 @@ struct NttCall {
   const uint32_t* pre;
   const uint32_t* post;
   fr kc, zk;
-  int kmax;  // 2 or 3: elements per thread 4 or 8
+  NttTile tile;
 };
 
 // Tiles of 2048 elements take 78 KB of LDS: above the 64 KB a launch may
@@ -845,8 +879,8 @@ static int ntt_exec(zk_context* ctx, const NttPlan* plan, const NttCall& c, hipS
   const int d = c.inverse ? 1 : 0;
   const int L = c.log_n, P = plan->P;
   const size_t n = (size_t)1 << L;
-  const int kmax = c.kmax;
-  const int logE = std::min(L, kmax == 3 ? 11 : 10);
+  const int kmax = c.tile.kmax;
+  const int logE = std::min(L, c.tile.logE);
   int logS[3];
   {
     int s = L;
@@ -888,7 +922,7 @@ static int ntt_exec(zk_context* ctx, const NttPlan* plan, const NttCall& c, hipS
     const uint32_t tiles = (uint32_t)(n / E);
     const bool fixed = kmax == 3 && E == (1u << NTT_TILE_FIXED_LOG) && threads == (E >> 3) && g.logR >= 6 &&
                        g.logR <= 8;
-    const size_t lds = (size_t)4 * ((fixed ? NTT_XPLANES : NL) * E + NL * (1u << (g.logR - 1)));
+    const size_t lds = (size_t)4 * ((fixed ? NTT_XPLANES : NL) * E + TW_PLANES * (1u << (g.logR - 1)));
     const dim3 grid(tiles, c.batch), block(threads);
     if (fixed && g.logR == 8) {
       if (last)
@@ -910,7 +944,7 @@ static int ntt_exec(zk_context* ctx, const NttPlan* plan, const NttCall& c, hipS
         ZK_LAUNCH(ctx, st, "ntt_pass", (k_ntt_pass<3, true>), grid, block, lds, g, io);
       else
         ZK_LAUNCH(ctx, st, "ntt_pass", (k_ntt_pass<3, false>), grid, block, lds, g, io);
-    } else if (g.logR >= 2) {
+    } else if (kmax >= 2 && g.logR >= 2) {
       if (last)
         ZK_LAUNCH(ctx, st, "ntt_pass", (k_ntt_pass<2, true>), grid, block, lds, g, io);
       else
@@ -925,17 +959,20 @@ static int ntt_exec(zk_context* ctx, const NttPlan* plan, const NttCall& c, hipS
   return ZK_OK;
 }
 
-// Elements per thread: 8 for large transforms (throughput), 4 below (a
-// thread's elements are a serial chain, so small transforms want more
-// threads).
-#ifndef ZK_NTT_KMAX_LARGE
-#define ZK_NTT_KMAX_LARGE 3
-#endif
-#ifndef ZK_NTT_LARGE_LOG
-#define ZK_NTT_LARGE_LOG 19
-#endif
-static int choose_kmax(int log_n, int batch) {
-  return ((size_t)batch << log_n) >= ((size_t)1 << ZK_NTT_LARGE_LOG) ? ZK_NTT_KMAX_LARGE : 2;
+// A thread's elements are a serial chain of butterflies, and a wave alone on its
+// SIMD issues at about 0.7 of the rate, so a call takes the fewest elements per
+// thread that still leave about two waves per SIMD; more per thread then save
+// exchanges.  Below 2^16 elements tiles of 128 threads spread them over more CUs.
+// Measured (us): 2^12 15.5 with 2 elements per thread and tiles of 2^8, 23.9
+// with 4 and 2^10; 2^16 21.8 / 30.7; 2^17 2^9-element tiles 28.6 / 38.5; 2^18 42.4
+// / 44.7; three of 2^18 92.6 / 87.1, with 8 per thread 98.3; 2^20 132.8 / 124.3,
+// with 8 117.5; 2^22 496 / 442 / 425.
+static NttTile choose_tile(int log_n, int batch) {
+  const size_t total = (size_t)batch << log_n;
+  if (total <= ((size_t)1 << 16)) return {1, 8};
+  if (total <= ((size_t)1 << 17)) return {1, 9};
+  if (total < ((size_t)1 << 20)) return {2, 10};
+  return {3, 11};
 }
 
 int ntt_run(zk_context* ctx, void* d_out, const void* d_in, int log_n, int inverse, int batch, uint64_t coset_g,
@@ -953,7 +990,7 @@ int ntt_run(zk_context* ctx, void* d_out, const void* d_in, int log_n, int inver
   c.log_n = log_n;
   c.inverse = inverse;
   c.batch = batch;
-  c.kmax = choose_kmax(log_n, batch);
+  c.tile = choose_tile(log_n, batch);
   if (plan->P > 1) {
     ZK_TRY(ctx->ensure(ctx->scratch_a, n * 32 * (size_t)batch));
     c.mid = ctx->scratch_a.p;
@@ -1009,7 +1046,7 @@ int quotient_ntts(zk_context* ctx, void* d_h, void* d_abc, void* d_work, int log
   NttCall c{};
   c.log_n = log_n;
   c.batch = 3;
-  c.kmax = choose_kmax(log_n, 3);
+  c.tile = choose_tile(log_n, 3);
   // coefficients * g^i: X -> Y (X is writable: the passes before the last run in it)
   c.src = d_abc;
   c.dst = d_work;
@@ -1026,10 +1063,11 @@ int quotient_ntts(zk_context* ctx, void* d_h, void* d_abc, void* d_work, int log
   c.post_mode = POST_NONE;
   c.post = nullptr;
   ZK_TRY(ntt_exec(ctx, plan, c, st));
-  // h: (A B - C) / Z from X, through Y, to d_h
+  // h: (A B - C) / Z from X, through Y, to d_h.  The tile stays that of the three:
+  // a proof's MSMs share the GPU, and more elements per thread issue fewer
+  // instructions (the 2^16 proof 1.087 ms, with the lone transform's tile 1.117)
   quotient_consts(zinv_mont, c.kc, c.zk);
   c.batch = 1;
-  c.kmax = choose_kmax(log_n, 1);
   c.src = d_abc;
   c.dst = d_h;
   c.mid = d_work;
@@ -1054,11 +1092,11 @@ int quotient_ntts(zk_context* ctx, void* d_h, void* d_abc, void* d_work, int log
 constexpr int NTT_NA_MAX_LOG = 16;
 constexpr int NTT_NA_MAX_ELEMS_LOG = 18;
 // the table slots of log_n = 1..16: each plan has at most 3 passes of at most
-// 2^8 rows (2 * 128 DFT twiddles of NL words per direction and pass) and
+// 2^8 rows (128 DFT twiddles of TW_PLANES words per direction and pass) and
 // inter-pass tables of at most 2^log_n packed entries per direction; the exact
 // layout is checked against this bound at set-up (ntt_scratch_init)
 constexpr size_t NTT_NA_TABLE_WORDS =
-    NTT_NA_MAX_LOG * 3 * 2 * 128 * NL + 2 * (((size_t)2 << NTT_NA_MAX_LOG) - 2) * PACKED_WORDS;
+    NTT_NA_MAX_LOG * 3 * 2 * 128 * TW_PLANES + 2 * (((size_t)2 << NTT_NA_MAX_LOG) - 2) * PACKED_WORDS;
 constexpr size_t NTT_NA_MID_WORDS = ((size_t)1 << NTT_NA_MAX_ELEMS_LOG) * 8;
 constexpr size_t NTT_NA_WORDS = NTT_NA_TABLE_WORDS + NTT_NA_MID_WORDS;
 
@@ -1136,7 +1174,7 @@ int ntt_run_noalloc(zk_context* ctx, void* d_out, const void* d_in, int log_n, i
   c.log_n = log_n;
   c.inverse = inverse;
   c.batch = batch;
-  c.kmax = choose_kmax(log_n, batch);
+  c.tile = choose_tile(log_n, batch);
   if (inverse) c.post_mode = plan.P == 1 ? POST_SCALE : POST_NONE;
   return ntt_exec(ctx, &plan, c, st);
 }

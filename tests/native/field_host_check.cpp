@@ -141,4 +141,36 @@ int fh_xyzz_lx(int g2, int op, const uint32_t* p, const uint32_t* q, uint32_t* o
   }
   return inf;
 }
+
+// Products by a constant over Fr: limbs of a below lu 2^29 (lu 1, 3 or 5).
+int fh_fr_const(int lu, const uint32_t* a, const uint32_t* w, const uint32_t* wq, uint32_t* out) {
+  fr A, W, Q, r;
+  memcpy(A.l, a, sizeof(A.l));
+  memcpy(W.l, w, sizeof(W.l));
+  memcpy(Q.l, wq, sizeof(Q.l));
+  switch (lu) {
+    case 1: r = fmul_const<1>(A, W, Q); break;
+    case 3: r = fmul_const<3>(A, W, Q); break;
+    case 5: r = fmul_const<5>(A, W, Q); break;
+    default: return -1;
+  }
+  memcpy(out, r.l, sizeof(r.l));
+  return 0;
+}
+
+// 0 const_quotient(a), 1 fsub_wide(a, b), 2 fadd_lazy(a, b), 3 fcarry(a)
+int fh_fr_wide(int op, const uint32_t* a, const uint32_t* b, uint32_t* out) {
+  fr A, B, r;
+  memcpy(A.l, a, sizeof(A.l));
+  memcpy(B.l, b, sizeof(B.l));
+  switch (op) {
+    case 0: r = const_quotient(A); break;
+    case 1: r = fsub_wide(A, B); break;
+    case 2: r = fadd_lazy(A, B); break;
+    case 3: r = fcarry(A); break;
+    default: return -1;
+  }
+  memcpy(out, r.l, sizeof(r.l));
+  return 0;
+}
 }

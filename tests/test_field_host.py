@@ -461,3 +461,62 @@ def test_lazy_x_ranges_at_random_residues(fh, g2flag):
             assert all(w < 1 << 29 for w in ws)
             vals = [from_l(ws[9 * k:9 * k + 9]) for k in range(4 * n)]
             assert all(v < 6 * Q for v in vals[:n]) and all(v < 2 * Q for v in vals[n:])
+
+
+@pytest.mark.parametrize("lu", [1, 3, 5])
+def test_product_by_constant(fh, lu):
+    """fmul_const: a w mod r from w and floor(w 2^261 / r), for operands with
+    limbs up to lu 2^29 - 1 (all at the maximum, one, or random): congruent,
+    limbs normalized, below 2r + r / 2^22; const_quotient gives the quotient."""
+    rng = random.Random(61 + lu)
+    r = ORDER
+    for i in range(400):
+        w = (0, 1, r - 1, r // 2)[i] if i < 4 else rng.randrange(r)
+        wq = w * RP // r
+        out = U32x9()
+        assert fh.fh_fr_wide(0, U32x9(*to_l(w * RP % r)), U32x9(), out) == 0
+        assert from_l(list(out)) == wq
+        ws, a = limbs_value(rng, lu << 29)
+        ws[8] = min(ws[8], (1 << 29) - 1 - 64)  # values below 2^261
+        a = from_l(ws)
+        if a >= RP:
+            continue
+        assert fh.fh_fr_const(lu, U32x9(*ws), U32x9(*to_l(w)), U32x9(*to_l(wq)), out) == 0
+        got = from_l(list(out))
+        assert all(x < 1 << 29 for x in out)
+        assert got % r == a * w % r and got <= 2 * r + (r >> 22)
+
+
+def test_ntt_step_without_carries(fh):
+    """Three twiddled stages as a pass runs them: u + w v and u - w v + 4r limb by
+    limb (limb bounds 1, 3, 5 then 7 times 2^29), one carry pass, then the next
+    step, eight stages in all: exact residues, values below 40r."""
+    rng = random.Random(71)
+    r = ORDER
+
+    def wide(op, a, b=None):
+        out = U32x9()
+        assert fh.fh_fr_wide(op, U32x9(*a), U32x9(*(b or [0] * 9)), out) == 0
+        return list(out)
+
+    for trial in range(60):
+        xs = [2 * r - 1 if trial == 0 else rng.randrange(2 * r) for _ in range(2)]
+        u, v = (to_l(x) for x in xs)
+        eu, ev = xs
+        for stage in range(8):
+            lu = (1, 3, 5)[stage % 3]
+            assert max(u + v) < lu << 29
+            w = rng.randrange(r)
+            out = U32x9()
+            fh.fh_fr_const(lu, U32x9(*v), U32x9(*to_l(w)), U32x9(*to_l(w * RP // r)), out)
+            p = list(out)
+            u, v = wide(2, u, p), wide(1, u, p)
+            eu, ev = (eu + ev * w) % r, (eu - ev * w) % r
+            assert from_l(u) % r == eu and from_l(v) % r == ev
+            if trial % 2:  # the other wire carries the larger limbs on
+                u, v, eu, ev = v, u, ev, eu
+            if stage % 3 == 2 or stage == 7:
+                a, b = from_l(u), from_l(v)
+                u, v = wide(3, u), wide(3, v)
+                assert from_l(u) == a and from_l(v) == b and max(u + v) < 1 << 29
+        assert from_l(u) < 40 * r and from_l(v) < 40 * r

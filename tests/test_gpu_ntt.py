@@ -125,3 +125,20 @@ def test_ntt_rejects_bad_sizes(ctx):
         ctx.ntt(d, d, 25, False)
     with pytest.raises(zkml_amd.ZkError):
         ctx.ntt(d, d, 0, False)
+
+
+@pytest.mark.parametrize("log_n,batch", [(5, 3), (9, 1), (9, 65), (13, 9), (15, 3), (16, 1), (16, 2), (17, 1), (17, 3),
+                                         (18, 1), (18, 2), (18, 3), (12, 256), (8, 4096), (19, 3)])
+def test_ntt_tile_rule(ctx, log_n, batch):
+    """Transforms on both sides of every limit of the tile rule (elements of the
+    call: 2^16, 2^18, 2^20), and batches that reach them with small transforms:
+    the first, a middle and the last transform of the batch, forward, inverse
+    and inverse coset, against the oracle."""
+    n = 1 << log_n
+    a = rand_words(batch * n, 300 + log_n + batch)
+    for inverse, g in ((False, 0), (True, 0), (True, 5)):
+        got = run_gpu(ctx, a, log_n, inverse, batch=batch, coset=g)
+        for b in sorted({0, batch // 2, batch - 1}):
+            x = a[b * n:(b + 1) * n]
+            want = oracle_coset(x, log_n, g, inverse) if g else oracle_ntt(x, log_n, inverse)
+            assert np.array_equal(got[b * n:(b + 1) * n], want), (b, inverse, g)
