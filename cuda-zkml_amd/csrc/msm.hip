@@ -53,7 +53,6 @@ constexpr int SORT_T = 1024;       // threads of the histogram / scatter blocks
 constexpr int SORT_U = 8;          // loads in flight per thread in the sort passes
 constexpr int SCAN_T = 128;        // buckets per column-scan block (<= the smallest B)
 constexpr int MSM_NCB = 256;       // coarse bins per window of the two-pass placement
-constexpr int MSM_BPC_MAX = 128;   // buckets per coarse bin at B = 2^15
 constexpr int PLACE_T = 1024;      // threads of a placement block
 constexpr uint32_t MSM_SERIAL_SPAN = 8;  // longest serial chunk-partial chain of the one-launch combine
 // Partials folded per bucket group by each level of the level combine.  A
@@ -463,50 +462,6 @@ __device__ __forceinline__ uint32_t wave_claim(uint32_t* ctr, uint32_t key, uint
   return pos;
 }
 
-// Tile-sorted writes of the placement.  A block takes its bin's entries in
-// tiles of TILE_E; each entry's bucket gives it a rank from LDS counters
-// (wave_claim), one wave turns the tile's counts into offsets, the entries are
-// staged in LDS in bucket order and written out by consecutive threads, so
-// every bucket's share of the tile leaves as one contiguous run (~32 entries
-// at 2^15 buckets) where entry-by-entry stores would each touch their own
-// cache line.
-constexpr int TILE_U = 4;
-constexpr int TILE_E = PLACE_T * TILE_U;  // entries per tile
-
-// Wave 0 only (threadIdx.x < 64): toff = exclusive scan of cnt[0, ns) (ns <=
-// 256), gbase = the buckets' global write positions for this tile (cur
-// advances by the counts), cnt cleared for the next tile, *tot = the tile's
-// entry count.
-__device__ __forceinline__ void tile_offsets(uint32_t* cnt, uint32_t* toff, uint32_t* gbase, uint32_t* cur,
-                                             uint32_t ns, uint32_t* tot) {
-  const uint32_t lane = threadIdx.x;
-  uint32_t c[4], sum = 0;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const uint32_t j = lane * 4 + i;
-    c[i] = j < ns ? cnt[j] : 0u;
-    sum += c[i];
-  }
-  uint32_t inc = sum;
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t o = (uint32_t)__shfl_up((int)inc, off, 64);
-    if (lane >= (uint32_t)off) inc += o;
-  }
-  uint32_t ex = inc - sum;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const uint32_t j = lane * 4 + i;
-    if (j < ns) {
-      toff[j] = ex;
-      gbase[j] = cur[j];
-      cur[j] += c[i];
-      cnt[j] = 0u;
-      ex += c[i];
-    }
-  }
-  if (lane == 63) *tot = inc;
-}
-
 // Two-pass placement for wide windows (B >= 2^13 buckets): one-pass random
 // 8-byte writes across the whole window region leave every cache line
 // partially written by many blocks.
@@ -523,7 +478,9 @@ __global__ __launch_bounds__(SORT_T) void k_msm_scatter_coarse(const uint32_t* _
                                                                const uint32_t* __restrict__ lex,
                                                                const uint32_t* __restrict__ tot,
                                                                uint32_t* __restrict__ start,
-                                                               uint32_t* __restrict__ end, uint2* __restrict__ tmp) {
+                                                               uint32_t* __restrict__ end,
+                                                               uint32_t* __restrict__ cursor,
+                                                               uint2* __restrict__ tmp) {
   msm_short_priority();
   __shared__ uint32_t cur[MSM_NCB];
   const uint32_t s = blockIdx.x, w = blockIdx.y, t = threadIdx.x;
@@ -540,6 +497,7 @@ __global__ __launch_bounds__(SORT_T) void k_msm_scatter_coarse(const uint32_t* _
       const uint32_t st = w * n_pad + boff[k / SCAN_T] + lex[k];
       start[k] = st;
       end[k] = st + tot[k];
+      cursor[k] = st;
     }
   }
   __syncthreads();
@@ -564,94 +522,77 @@ __global__ __launch_bounds__(SORT_T) void k_msm_scatter_coarse(const uint32_t* _
   }
 }
 
-// Pass 2 (block per window x coarse bin): LDS cursors for the bin's BPC
-// buckets; every write stays inside the bin's region.  A bin whose largest
-// bucket holds at least half of its entries (the hot bucket of skewed
-// scalars) writes entry by entry: a wave's lanes then mostly share that
-// bucket and take consecutive positions with one atomic (wave_claim), so its
-// stores are contiguous already and the tile staging would only add barriers
-// on the one block that decides the launch's length.  Other bins go through
-// the tile-sorted writes above.
+// Pass 2: a block takes PLACE_E consecutive entries of a window's binned list,
+// whatever bins they belong to.  Their buckets span the bins of the first and
+// last entry (bins are in order); up to PLACE_R buckets, each entry's bucket
+// gives it a rank from an LDS counter (one atomic per wave where all its lanes
+// hold one bucket), the counters are scanned, every bucket's share of the tile
+// claims its place in the bucket with one global atomic on the bucket's cursor,
+// and the entries are staged in LDS in bucket order and written by consecutive
+// threads: each share leaves as one contiguous run.  A tile over more buckets
+// (few entries in a wide window) claims entry by entry.
+// Every tile costs the same whatever the bucket sizes: with a block per bin the
+// bin that holds a skewed window's hot buckets (digit 1 of a witness of small
+// values: 240,000 of 300,007 entries) took 164 us of one block; uniform scalars
+// (2^20 points) took 66 us that way.
+constexpr int PLACE_U = 4;
+constexpr int PLACE_E = PLACE_T * PLACE_U;  // entries per tile
+constexpr int PLACE_R = 1024;               // most buckets a tile counts in LDS
 __global__ __launch_bounds__(PLACE_T) void k_msm_place(const uint2* __restrict__ tmp, uint32_t B, uint32_t BPC,
-                                                       const uint32_t* __restrict__ start,
-                                                       const uint32_t* __restrict__ end,
-                                                       const uint32_t* __restrict__ bmax, uint2* __restrict__ out) {
-  static_assert(MSM_BPC_MAX <= 256 && MSM_BPC_MAX <= SCAN_T, "one wave scans the bin's counters");
+                                                       uint32_t n_pad, const uint32_t* __restrict__ wstat,
+                                                       uint32_t* __restrict__ cursor, uint2* __restrict__ out) {
+  static_assert(PLACE_R == PLACE_T, "one counter per thread in the scan");
   msm_short_priority();
-  __shared__ uint32_t cur[MSM_BPC_MAX], cnt[MSM_BPC_MAX], toff[MSM_BPC_MAX], gbase[MSM_BPC_MAX], ttot;
-  __shared__ uint2 stg[TILE_E];
-  const uint32_t cb = blockIdx.x, w = blockIdx.y, t = threadIdx.x;
-  const uint32_t k0 = w * B + cb * BPC;
-  const uint32_t lo = start[k0], hi = end[k0 + BPC - 1];
-  for (uint32_t j = t; j < BPC; j += PLACE_T) {
-    cur[j] = start[k0 + j];
-    cnt[j] = 0u;
+  __shared__ uint32_t cnt[PLACE_R], toff[PLACE_R], gbase[PLACE_R], wsum[PLACE_T / 64];
+  __shared__ uint2 stg[PLACE_E];
+  const uint32_t w = blockIdx.y, t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const uint32_t lo = w * n_pad + blockIdx.x * PLACE_E, whi = w * n_pad + wstat[2 * w];
+  if (lo >= whi) return;
+  const uint32_t hi = min(lo + PLACE_E, whi);
+  const uint32_t k0 = (tmp[lo].x - w * B) / BPC * BPC + w * B;                      // first bucket of the first bin
+  const uint32_t kr = (tmp[hi - 1].x - w * B) / BPC * BPC + w * B + BPC - k0;       // buckets of the tile's bins
+  uint2 e[PLACE_U];
+#pragma unroll
+  for (int u = 0; u < PLACE_U; u++) {
+    const uint32_t p = lo + t + u * PLACE_T;
+    e[u] = p < hi ? tmp[p] : make_uint2(KEY_INVALID, 0u);
   }
-  // the largest bucket of the column-scan block holding this bin (BPC <=
-  // SCAN_T: that block's buckets include the bin's), an upper bound of the
-  // bin's own largest bucket
-  const bool hot = 2u * bmax[k0 / SCAN_T] >= hi - lo;
-  __syncthreads();
-  if (hot) {
-    for (uint32_t p0 = lo + t; p0 < hi; p0 += PLACE_T * SORT_U) {
-      uint2 e[SORT_U];
+  if (kr > PLACE_R) {  // uniform over the block
 #pragma unroll
-      for (int u = 0; u < SORT_U; u++) {
-        const uint32_t p = p0 + u * PLACE_T;
-        e[u] = p < hi ? tmp[p] : make_uint2(KEY_INVALID, 0u);
-      }
-      // When every active lane of a wave holds the same bucket, the wave
-      // takes its positions with one atomic (order inside a bucket is free:
-      // its points are summed); a hot bucket would otherwise serialize the
-      // CU's LDS on one counter.  All eight atomics are issued before any
-      // result is read, so their round trips overlap.
-      uint32_t pos[SORT_U], rank[SORT_U];
-      bool agg[SORT_U];
-#pragma unroll
-      for (int u = 0; u < SORT_U; u++) {
-        const uint32_t key = e[u].x;
-        const uint32_t lead = __builtin_amdgcn_readfirstlane(key);
-        const uint64_t same = __ballot(key == lead);
-        agg[u] = same == __ballot(1) && lead != KEY_INVALID;
-        rank[u] = __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
-        pos[u] = 0;
-        if (agg[u]) {
-          if (rank[u] == 0) pos[u] = atomicAdd(&cur[lead - k0], (uint32_t)__popcll(same));
-        } else if (key != KEY_INVALID) {
-          pos[u] = atomicAdd(&cur[key - k0], 1u);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < SORT_U; u++) {
-        if (agg[u]) pos[u] = __builtin_amdgcn_readfirstlane(pos[u]) + rank[u];
-        if (e[u].x != KEY_INVALID) out[pos[u]] = e[u];
-      }
-    }
+    for (int u = 0; u < PLACE_U; u++)
+      if (e[u].x != KEY_INVALID) out[atomicAdd(&cursor[e[u].x], 1u)] = e[u];
     return;
   }
-  for (uint32_t p0 = lo; p0 < hi; p0 += TILE_E) {
-    uint2 e[TILE_U];
-    uint32_t rank[TILE_U];
+  cnt[t] = 0u;
+  __syncthreads();
+  uint32_t rank[PLACE_U];
 #pragma unroll
-    for (int u = 0; u < TILE_U; u++) {
-      const uint32_t p = p0 + t + u * PLACE_T;
-      e[u] = p < hi ? tmp[p] : make_uint2(KEY_INVALID, 0u);
-    }
+  for (int u = 0; u < PLACE_U; u++) rank[u] = wave_claim(cnt, e[u].x, e[u].x == KEY_INVALID ? 0 : e[u].x - k0);
+  __syncthreads();
+  // exclusive scan of the counters, thread t owns counter t; its share's place
+  const uint32_t c = cnt[t];
+  uint32_t inc = c;
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t o = (uint32_t)__shfl_up((int)inc, off);
+    if (lane >= (uint32_t)off) inc += o;
+  }
+  if (lane == 63) wsum[wv] = inc;
+  if (c) gbase[t] = atomicAdd(&cursor[k0 + t], c);
+  __syncthreads();
+  uint32_t base = 0;
 #pragma unroll
-    for (int u = 0; u < TILE_U; u++) rank[u] = wave_claim(cnt, e[u].x, e[u].x == KEY_INVALID ? 0 : e[u].x - k0);
-    __syncthreads();
-    if (t < 64) tile_offsets(cnt, toff, gbase, cur, BPC, &ttot);
-    __syncthreads();
+  for (int v = 0; v < PLACE_T / 64; v++)
+    if ((uint32_t)v < wv) base += wsum[v];
+  toff[t] = base + inc - c;
+  __syncthreads();
 #pragma unroll
-    for (int u = 0; u < TILE_U; u++)
-      if (e[u].x != KEY_INVALID) stg[toff[e[u].x - k0] + rank[u]] = e[u];
-    __syncthreads();
-    const uint32_t nt = ttot;
-    for (uint32_t lp = t; lp < nt; lp += PLACE_T) {
-      const uint2 x = stg[lp];
-      const uint32_t j = x.x - k0;
-      out[gbase[j] + (lp - toff[j])] = x;
-    }
+  for (int u = 0; u < PLACE_U; u++)
+    if (e[u].x != KEY_INVALID) stg[toff[e[u].x - k0] + rank[u]] = e[u];
+  __syncthreads();
+  for (uint32_t lp = t; lp < hi - lo; lp += PLACE_T) {
+    const uint2 x = stg[lp];
+    const uint32_t j = x.x - k0;
+    out[gbase[j] + (lp - toff[j])] = x;
   }
 }
 
@@ -1485,7 +1426,7 @@ constexpr int MSM_MAX_W = 32;   // windows of the narrowest window (8 bits)
 constexpr int MSM_PARTS = 512;  // points of one MSM's reduction, all windows (or sub-windows) and sets
 
 struct MsmWorkspace {
-  DevBuf recs, dig, hist, tot, lex, bsum, bmax, boff, tmp, sorted, start, end, wstat, buckets, hkey, tkey, hpt, tpt,
+  DevBuf recs, dig, hist, tot, lex, bsum, bmax, boff, tmp, sorted, start, end, wstat, cursor, buckets, hkey, tkey, hpt, tpt,
       seg, grp, win, fcnt, fin, fout;
   uint32_t* h_stat = nullptr;  // pinned, 2 words per window
   void* h_parts = nullptr;     // pinned, the per-window partials of every set
@@ -1498,7 +1439,7 @@ void msm_workspace_gate(MsmWorkspace* ws, MsmGate* wait_before_accumulate) { ws-
 void msm_workspace_free(MsmWorkspace* ws) {
   if (!ws) return;
   for (DevBuf* b : {&ws->recs, &ws->dig, &ws->hist, &ws->tot, &ws->lex, &ws->bsum, &ws->bmax, &ws->boff, &ws->tmp,
-                    &ws->sorted, &ws->start, &ws->end, &ws->wstat, &ws->buckets, &ws->hkey, &ws->tkey, &ws->hpt,
+                    &ws->sorted, &ws->start, &ws->end, &ws->wstat, &ws->cursor, &ws->buckets, &ws->hkey, &ws->tkey, &ws->hpt,
                     &ws->tpt, &ws->seg, &ws->grp, &ws->win, &ws->fcnt, &ws->fin, &ws->fout})
     if (b->p) (void)hipFree(b->p);
   if (ws->h_stat) (void)hipHostFree(ws->h_stat);
@@ -1696,9 +1637,9 @@ static int msm_sort(zk_context* ctx, MsmWorkspace& ws, const MsmShape& sh, bool 
     const uint32_t BPC = B / MSM_NCB;  // 32..128
     uint2* tmp = (uint2*)ws.tmp.p;
     ZK_LAUNCH(ctx, st, "msm_scatter", k_msm_scatter_coarse, dim3(S, W), dim3(SORT_T), 0, dig, n, slice, S, B, BPC,
-              n_pad, hist, boff, lex, tot, start, end, tmp);
-    ZK_LAUNCH(ctx, st, "msm_place", k_msm_place, dim3(MSM_NCB, W), dim3(PLACE_T), 0, tmp, B, BPC, start, end, bmax,
-              sorted);
+              n_pad, hist, boff, lex, tot, start, end, (uint32_t*)ws.cursor.p, tmp);
+    ZK_LAUNCH(ctx, st, "msm_place", k_msm_place, dim3(cdiv(n, PLACE_E), W), dim3(PLACE_T), 0, tmp, B, BPC, n_pad, wstat,
+              (uint32_t*)ws.cursor.p, sorted);
   }
   return ZK_OK;
 }
@@ -2022,7 +1963,10 @@ static int msm_run_sets(zk_context* ctx, MsmWorkspace& ws, const BaseSets& sets_
   ZK_TRY(ctx->ensure(ws.bmax, nbuckets / SCAN_T * 4));
   ZK_TRY(ctx->ensure(ws.boff, nbuckets / SCAN_T * 4));
   ZK_TRY(ctx->ensure(ws.sorted, (size_t)W * sh.n_pad * 8));
-  if (sh.B > 4096) ZK_TRY(ctx->ensure(ws.tmp, (size_t)W * sh.n_pad * 8));
+  if (sh.B > 4096) {
+    ZK_TRY(ctx->ensure(ws.tmp, (size_t)W * sh.n_pad * 8));
+    ZK_TRY(ctx->ensure(ws.cursor, nbuckets * 4));
+  }
   ZK_TRY(ctx->ensure(ws.start, nbuckets * 4));
   ZK_TRY(ctx->ensure(ws.end, nbuckets * 4));
   ZK_TRY(ctx->ensure(ws.wstat, (size_t)W * 8));

@@ -443,3 +443,31 @@ def test_msm_bucket_reduction_shapes(ctx, g2, n):
         print(f"[msm shapes {'g2' if g2 else 'g1'} {n} c={c}] {name}", flush=True)
         got = run(dp, ctx.upload(to_mont(s)), n)
         assert from_words(got) == G.pmul(gen, closed_form_scalar(kstd, s)), name
+
+
+@pytest.mark.parametrize("g2,n,kind", [(False, 600001, "hot"), (False, 600001, "sparse"), (False, 600001, "tile"),
+                                       (True, 540001, "hot"), (True, 540001, "sparse")])
+def test_msm_wide_window_placement(ctx, g2, n, kind):
+    """Windows of more than 2^12 buckets are placed in tiles of 4096 binned
+    entries: tiles inside one hot bucket, tiles that end on an entry count of
+    4095 to 4097, and tiles over more buckets than are counted in LDS."""
+    import zkml_amd
+    c, _ = zkml_amd.Context.msm_config(n, g2)
+    assert c > 13, "a window of more than 2^12 buckets"
+    rng = np.random.default_rng(n)
+    kstd = rand_std(n, rng)
+    dp = gpu_points(ctx, to_mont(kstd), g2=g2)
+    ds = np.zeros((n, 4), dtype=np.uint64)
+    if kind == "hot":
+        ds[:, 0] = 1
+        ds[::5] = rand_std(len(ds[::5]), rng)
+    elif kind == "sparse":
+        ds[::600] = rand_std(len(ds[::600]), rng)
+    else:
+        at = rng.permutation(n)
+        for w, count in enumerate((4095, 4096, 4097)):  # entries of window w
+            ds[at[:count], 0] += np.uint64(1 + w) << np.uint64(c * w)
+    run = ctx.msm_g2 if g2 else ctx.msm_g1
+    G, gen, from_words = (Z.g2, Z.G2, Z.g2_from_words) if g2 else (Z.g1, Z.G1, Z.g1_from_words)
+    got = run(dp, ctx.upload(to_mont(ds)), n)
+    assert from_words(got) == G.pmul(gen, closed_form_scalar(kstd, ds))
