@@ -16,10 +16,10 @@
 //                region [w*n_pad, w*n_pad + n_pad)); a scatter pass with LDS
 //                cursors writes (bucket, point | sign<<31) pairs.  The order
 //                inside a bucket is arbitrary, which cannot change the sum.
-//  4. accumulate every thread sums exactly L0 consecutive sorted entries
-//                with mixed XYZZ additions (perfect load balance whatever the
-//                bucket sizes); runs that cross a chunk edge leave a head /
-//                tail partial.
+//  4. accumulate every thread sums a chunk of L0 consecutive sorted entries
+//                (L0 chosen so that the chunks fill the SIMDs in whole waves)
+//                with mixed XYZZ additions, whatever the bucket sizes; runs
+//                that cross a chunk edge leave a head / tail partial.
 //  5. combine    the chunk partials of each bucket that spans chunks are
 //                folded in groups (one launch for ordinary buckets,
 //                ~log8(size/L0) for hot buckets such as many scalars equal
@@ -46,6 +46,7 @@
 namespace zk {
 
 constexpr uint32_t KEY_INVALID = 0xffffffffu;
+constexpr int MSM_MAX_W = 32;   // windows of the narrowest window (8 bits)
 constexpr int MSM_L0 = 64;         // sorted entries per accumulation thread (largest)
 constexpr int MSM_CMAX = 16;       // widest window: 2^15 LDS counters (128 KB)
 constexpr uint32_t MSM_LDS_B = 32768;  // most buckets a window's slice histogram holds in LDS
@@ -64,14 +65,7 @@ constexpr uint32_t MSM_COMBINE_S = 2;
 #define ZK_MSM_TREE_SPAN 512
 #endif
 constexpr uint32_t MSM_TREE_SPAN = ZK_MSM_TREE_SPAN;
-// G2 accumulation tuning: chunk length divided by 2^ZK_MSM_G2_L0_SHIFT (down
-// to MSM_L0 / 8), waves per SIMD the register budget is cut to.
-#ifndef ZK_MSM_G2_L0_SHIFT
-#define ZK_MSM_G2_L0_SHIFT 0
-#endif
-#ifndef ZK_MSM_G2_ONE_LANE
-#define ZK_MSM_G2_ONE_LANE 1
-#endif
+// G2 accumulation tuning: waves per SIMD the register budget is cut to.
 #ifndef ZK_MSM_G2_ACC_WAVES
 #define ZK_MSM_G2_ACC_WAVES 3
 #endif
@@ -816,6 +810,36 @@ struct ChunkSlots {
   }
 };
 
+// Chunks of the sorted list: window w's entries [w n_pad, w n_pad + count) are
+// the chunks [first[w], first[w + 1]) of L0 entries, the last one shorter.  Only
+// chunks that hold entries are numbered: with the windows' full length a
+// witness's upper windows were waves without work that left others two on a SIMD.
+struct ChunkMap {
+  uint32_t L0, n_pad;
+  int lb;  // log2 of the buckets per window
+  uint32_t first[MSM_MAX_W];  // UINT32_MAX past the last window
+  // Window and first chunk by selects over the whole array, which is then a few
+  // scalar loads: a lane's own index would read the kernel arguments through
+  // vector memory (8 us of a 240 us MSM in the accumulation and combine).
+  __device__ void find(uint32_t ch, uint32_t& w, uint32_t& c0) const {
+    w = c0 = 0;
+#pragma unroll
+    for (int v = 1; v < MSM_MAX_W; v++)
+      if (ch >= first[v]) {
+        w = v;
+        c0 = first[v];
+      }
+  }
+  // the chunk of sorted position p, which bucket `key` holds
+  __device__ uint32_t of(uint32_t key, uint32_t p) const {
+    const uint32_t w = key >> lb;
+    uint32_t c0 = 0;
+#pragma unroll
+    for (int v = 1; v < MSM_MAX_W; v++) c0 = w == (uint32_t)v ? first[v] : c0;
+    return c0 + (p - w * n_pad) / L0;
+  }
+};
+
 // Point sets sharing one scalar vector (and so one sorted digit list): set s
 // takes the scalars with index i in [lo[s], hi[s]) and the point recs[s][i -
 // lo[s]]; entries outside the range add nothing to that set's buckets.
@@ -877,34 +901,20 @@ static_assert(acc_waves<Lanes<fq>>() == 4 && acc_waves<Lanes<fq2>>() == ZK_MSM_G
                   acc_waves<OneLane<fq2>>() == 2,
               "accumulation wave targets by lane layout");
 
-// Chunk ch covers sorted positions [ch*L0, ch*L0 + L0) of window
-// ch / chunks_per_window; positions past the window's entry count are empty.
 // blockIdx.y selects the base set; its buckets start at set * nbuckets.  A
 // chunk is one lane (G1) or one lane pair (G2, Lanes<F>): split over a pair
 // the G2 accumulator needs half the registers per lane, so that more waves
 // fit on a SIMD to cover the gathers' latency.
-//
-// Waves are scattered over the chunk space: wave v of the grid takes the
-// 64 / Lanes<F>::N chunks of chunk-wave (v * wave_mul) mod nwaves (wave_mul
-// coprime to nwaves, so every chunk is taken once).  With skewed scalars most entries
-// sit in a few windows (small witness values fill the low ones); in chunk
-// order those windows' waves would land on a fraction of the CUs, scattered
-// they spread over all of them.
 template <class F, bool TAB, class LN = Lanes<F>>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(acc_waves<LN>()))) void k_msm_accumulate(const uint2* __restrict__ sorted, BaseSets sets,
                                                         const uint32_t* __restrict__ start,
                                                         const uint32_t* __restrict__ end,
                                                         const uint32_t* __restrict__ wstat, uint32_t nchunks,
-                                                        uint32_t chunks_per_window, uint32_t n_pad, uint32_t L0,
-                                                        size_t nbuckets, xyzz<F>* __restrict__ buckets,
-                                                        ChunkSlots<F> all_slots, uint32_t nwaves,
-                                                        uint32_t wave_mul) {
+                                                        ChunkMap cm, size_t nbuckets, xyzz<F>* __restrict__ buckets,
+                                                        ChunkSlots<F> all_slots) {
   typedef typename LN::R R;
-  constexpr uint32_t PER_WAVE = 64 / LN::N;  // chunks per wave
   msm_accumulate_priority<F>();
-  const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
-  if ((tid >> 6) >= nwaves) return;
-  const uint32_t ch = (uint32_t)((uint64_t)(tid >> 6) * wave_mul % nwaves) * PER_WAVE + (tid & 63) / LN::N;
+  const uint32_t ch = (blockIdx.x * blockDim.x + threadIdx.x) / LN::N;
   if (ch >= nchunks) return;
   const uint32_t set = blockIdx.y;
   const uint4* __restrict__ recs = sets.recs[set];
@@ -912,12 +922,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(acc_waves<L
   const uint32_t pstride = sets.pstride, tstride = sets.tstride[set];
   buckets += set * nbuckets;
   const ChunkSlots<F> slots = all_slots.at(set, nchunks);
-  const uint32_t w = ch / chunks_per_window;
-  const uint32_t total = w * n_pad + wstat[2 * w];
-  const uint32_t lo = ch * L0;
+  uint32_t w, c0;
+  cm.find(ch, w, c0);
+  const uint32_t total = w * cm.n_pad + wstat[2 * w];
+  const uint32_t lo = w * cm.n_pad + (ch - c0) * cm.L0;
   uint32_t hk = KEY_INVALID, tk = KEY_INVALID;
-  if (lo < total) {
-    const uint32_t hi = min(lo + L0, total);
+  {
+    const uint32_t hi = min(lo + cm.L0, total);
     xyzz<R> acc;
     xyzz_set_inf(acc);
     bool empty = true;  // acc is the point at infinity
@@ -960,7 +971,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(acc_waves<L
     // last run of the chunk
     if (__builtin_expect(empty, 0)) xyzz_set_inf(acc);
     const uint32_t rs = start[cur], re = end[cur];
-    if (rs >= lo && re <= lo + L0) {
+    if (rs >= lo && re <= hi) {
       LN::store(buckets[cur], acc);
     } else if (rs < lo) {
       hk = cur;
@@ -998,7 +1009,7 @@ __device__ __forceinline__ uint32_t cdiv_dev(uint32_t a, uint32_t b) { return (a
 template <class F, class LN>
 __global__ __launch_bounds__(256) void k_msm_combine_serial(ChunkSlots<F> all_slots,
                                                             const uint32_t* __restrict__ end, uint32_t nchunks,
-                                                            uint32_t L0, size_t nbuckets,
+                                                            ChunkMap cm, size_t nbuckets,
                                                             xyzz<F>* __restrict__ buckets,
                                                             uint32_t* __restrict__ fold_cnt, uint32_t tb) {
   msm_priority<F>();
@@ -1009,7 +1020,7 @@ __global__ __launch_bounds__(256) void k_msm_combine_serial(ChunkSlots<F> all_sl
   buckets += blockIdx.y * nbuckets;
   const uint32_t tk = slots.tkey[ch];
   if (tk == KEY_INVALID) return;
-  const uint32_t c1 = (end[tk] - 1) / L0;
+  const uint32_t c1 = cm.of(tk, end[tk] - 1);
   if (c1 - ch > MSM_SERIAL_SPAN) return;  // a long span: the tree combine
   auto acc = LN::load(slots.tpt[ch]);
   for (uint32_t j = ch + 1; j <= c1; j++) xyzz_add_lx(acc, LN::load(slots.hpt[j]));
@@ -1026,7 +1037,7 @@ __global__ __launch_bounds__(256) void k_msm_combine_serial(ChunkSlots<F> all_sl
 template <class F, class LN>
 __global__ __launch_bounds__(256) void k_msm_combine(ChunkSlots<F> all_slots, const uint32_t* __restrict__ start,
                                                      const uint32_t* __restrict__ end, uint32_t nchunks,
-                                                     uint32_t L0, uint32_t step, size_t nbuckets,
+                                                     ChunkMap cm, uint32_t step, size_t nbuckets,
                                                      xyzz<F>* __restrict__ buckets) {
   constexpr uint32_t S = MSM_COMBINE_S;
   msm_priority<F>();
@@ -1040,7 +1051,7 @@ __global__ __launch_bounds__(256) void k_msm_combine(ChunkSlots<F> all_slots, co
     key = slots.hkey[ch];
     if (key == KEY_INVALID) return;
   }
-  const uint32_t c0 = start[key] / L0, c1 = (end[key] - 1) / L0;
+  const uint32_t c0 = cm.of(key, start[key]), c1 = cm.of(key, end[key] - 1);
   if ((ch - c0) % (S * step) != 0 || ch + step > c1) return;  // nothing to fold here
   xyzz<F>* self = tail ? &slots.tpt[ch] : &slots.hpt[ch];
   auto acc = LN::load(*self);
@@ -1068,7 +1079,7 @@ template <class F, class LN, int TB>
 __global__ __launch_bounds__(TB * LN::N) void k_msm_combine_tree(ChunkSlots<F> all_slots,
                                                                  const uint32_t* __restrict__ start,
                                                                  const uint32_t* __restrict__ end,
-                                                                 uint32_t nchunks, uint32_t L0, size_t nbuckets,
+                                                                 uint32_t nchunks, ChunkMap cm, size_t nbuckets,
                                                                  xyzz<F>* __restrict__ buckets,
                                                                  uint32_t* __restrict__ fold_cnt,
                                                                  xyzz<F>* __restrict__ cin, xyzz<F>* __restrict__ cout) {
@@ -1095,8 +1106,8 @@ __global__ __launch_bounds__(TB * LN::N) void k_msm_combine_tree(ChunkSlots<F> a
   if (ch < b1) {
     const uint32_t k = slots.hkey[ch];
     if (k != KEY_INVALID) {
-      hc0 = start[k] / L0;
-      hc1 = (end[k] - 1) / L0;
+      hc0 = cm.of(k, start[k]);
+      hc1 = cm.of(k, end[k] - 1);
       if (hc1 - hc0 > MSM_SERIAL_SPAN) {
         hk = k;
         const uint32_t lo = max(hc0 + 1, b0), hi = min(hc1, b1 - 1);
@@ -1110,7 +1121,7 @@ __global__ __launch_bounds__(TB * LN::N) void k_msm_combine_tree(ChunkSlots<F> a
   if (ch < b1) {
     const uint32_t k = slots.tkey[ch];
     if (k != KEY_INVALID) {
-      tc1 = (end[k] - 1) / L0;
+      tc1 = cm.of(k, end[k] - 1);
       if (tc1 - ch > MSM_SERIAL_SPAN) tk = k;
     }
   }
@@ -1422,7 +1433,6 @@ static RedShape red_shape(int l, bool g2) {
 }
 
 // ------------------------------------------------------------------ workspace
-constexpr int MSM_MAX_W = 32;   // windows of the narrowest window (8 bits)
 constexpr int MSM_PARTS = 512;  // points of one MSM's reduction, all windows (or sub-windows) and sets
 
 struct MsmWorkspace {
@@ -1446,16 +1456,6 @@ void msm_workspace_free(MsmWorkspace* ws) {
   if (ws->h_parts) (void)hipHostFree(ws->h_parts);
   if (ws->stat_ready) (void)hipEventDestroy(ws->stat_ready);
   delete ws;
-}
-
-// Multiplier of the accumulation's wave scatter: coprime to nwaves (so
-// v -> v * m mod nwaves is a permutation) and near nwaves / golden ratio, so
-// that consecutive waves land far apart in the chunk space.
-static uint32_t wave_scatter(uint32_t nwaves) {
-  if (nwaves <= 2) return 1;
-  uint32_t m = (uint32_t)(nwaves * 0.6180339887) | 1u;
-  while (std::gcd(m, nwaves) != 1) m += 2;
-  return m % nwaves;
 }
 
 // Window size by input size (index: ceil(log2 n)), from measurements on
@@ -1580,7 +1580,7 @@ struct MsmShape {
   size_t n;
   int W;
   uint32_t B;
-  uint32_t n_pad;  // window region of the sorted list, padded to the longest chunk
+  uint32_t n_pad;  // window region of the sorted list, in whole cache lines
   uint32_t S;      // slices per window of the sort: about 256 blocks, each slice at least B points
 };
 
@@ -1680,23 +1680,37 @@ static int msm_sort_wide(zk_context* ctx, MsmWorkspace& ws, const MsmShape& sh, 
 
 // Accumulation shape, from the sort statistics.
 struct AccPlan {
-  uint32_t L0;        // sorted entries per chunk
-  uint32_t cpw;       // chunks per window
+  ChunkMap map;
   uint32_t nchunks;   // chunks of one set
   uint32_t max_span;  // chunks spanned by the largest bucket
+  bool one_lane;      // G2 chunks on one lane instead of a pair
 };
 
-// Entries per accumulation thread, by the entry count (G1: zero digits are
-// no entries, so skewed scalars, such as a witness of small values, count
-// for less than W*n): short chunks give small MSMs enough threads (a thread's
-// chunk is a serial chain of additions), long chunks keep the chunk-combine
-// tree of large ones shallow.  Measured on MI355X over 2^10 .. 2^20 points,
-// G1 and G2, uniform and witness-like scalars.  Inside a proof the same
-// lengths serve: halving the G1 chunks beside the other jobs once paid (2^16
-// proof 1.97 -> 1.87 ms), but with the proof's later host and placement
-// work it cost config 4's 2^16 proof 1.26 -> 1.29 ms.
+// Entries per chunk.  A chunk is a serial chain of additions and the SIMDs are
+// filled in whole waves, so the length decides how many of the 1024 SIMDs hold k
+// waves: the shortest length whose chunks (zero digits are no entries) make at
+// most 1024 k waves, for
+//   k = 1 while that is at most 28 entries (a lone wave issues slower, but half as
+//         many chunks leave half as many partials to combine),
+//   k = 2 while that is at most 48, else the first multiple of 4 (a full chip each)
+//         that asks for at most 64.
+// G2 chunks take one lane instead of a pair from 5 million entries (k = 2 then fills
+// the registers, multiples of 2 for at most 80 entries): 524,288 points in 20 windows
+// 64 entries on 2.5 waves 2998 us, in 16 on 2 waves 2312.
+// Against powers of two by the entry count (us; uniform scalars): G1 65,536 points
+// in 24 windows 32 -> 24 entries 443 -> 405, 100,000 in 20 windows 32 -> 16 455 ->
+// 448, in 24 windows 32 -> 20 563 -> 478; G2 62,779 in 24 windows 32 -> 24 842 -> 742.
+// Beside other jobs (a proof), whose waves fill the SIMDs, k = 1 and 8 to 40
+// entries: a 2^16 proof 1057 -> 1044, one of 200,001 rows 2984 -> 2840.
+// Alone, few points take chunks of 4: 1000 points 243 -> 235.  A length of up to 12
+// at which the largest bucket spans few enough chunks for the serial combine is
+// preferred to a shorter one (10,000 points: 8 entries 293, 10 280).
+constexpr uint32_t MSM_SIMDS = 1024;  // 256 CUs of 4
+constexpr uint32_t MSM_L0_ONE = 80;   // longest G2 chunk on one lane
+constexpr size_t MSM_ONE_LANE_ENTRIES = 5000000;
+
 template <class F>
-static AccPlan plan_accumulation(const MsmWorkspace& ws, const MsmShape& sh) {
+static AccPlan plan_accumulation(const MsmWorkspace& ws, const MsmShape& sh, bool beside) {
   constexpr bool G2 = sizeof(F) != sizeof(fq);
   size_t entries = 0;
   uint32_t maxrun = 1;
@@ -1704,20 +1718,43 @@ static AccPlan plan_accumulation(const MsmWorkspace& ws, const MsmShape& sh) {
     entries += ws.h_stat[2 * w];
     maxrun = std::max(maxrun, ws.h_stat[2 * w + 1]);
   }
-  entries += entries / 32;  // uniform scalars' few zero digits keep their chunk length
-  // a G2 chunk combine costs about 3x a G1 one: shorter G2 chunks for skewed
-  // scalars lost more there than they gained (2^16 witness-like G2 MSM 1.30 ->
-  // 1.35 ms), so G2 keeps the length of W*n entries
-  if (G2) entries = (size_t)sh.W * sh.n;
-  const uint32_t L0_alone = entries >= ((size_t)1 << 23)   ? MSM_L0
-                            : entries >= ((size_t)1 << 20) ? MSM_L0 / 2
-                            : entries >= ((size_t)1 << 18) ? MSM_L0 / 4
-                                                           : MSM_L0 / 8;
+  auto chunks = [&](uint32_t L) {
+    size_t c = 0;
+    for (int w = 0; w < sh.W; w++) c += cdiv(ws.h_stat[2 * w], L);
+    return c;
+  };
+  auto shortest = [&](uint32_t k, uint32_t lanes) {
+    const size_t limit = (size_t)MSM_SIMDS * k * 64 / lanes;
+    uint32_t L = (uint32_t)std::max<size_t>(1, cdiv(entries, limit));
+    while (chunks(L) > limit && L < cdiv(entries, limit) + 8) L++;
+    return L;
+  };
+  constexpr uint32_t N = Lanes<F>::N;
   AccPlan ap;
-  ap.L0 = G2 ? std::max<uint32_t>(L0_alone >> ZK_MSM_G2_L0_SHIFT, MSM_L0 / 8) : L0_alone;
-  ap.cpw = sh.n_pad / ap.L0;
-  ap.nchunks = ap.cpw * (uint32_t)sh.W;
-  ap.max_span = (maxrun + ap.L0 - 2) / ap.L0 + 1;
+  ap.one_lane = false;
+  uint32_t L0 = shortest(1, N);
+  if (beside) {
+    L0 = std::min(std::max(L0, 8u), 40u);
+  } else {
+    if (L0 > 28) L0 = shortest(2, N);
+    if (L0 > 48) L0 = shortest(4 * (uint32_t)cdiv(entries * N, (size_t)MSM_L0 * 4 * MSM_SIMDS * 64), N);
+    if (G2 && entries >= MSM_ONE_LANE_ENTRIES) {
+      ap.one_lane = true;
+      L0 = shortest(2 * (uint32_t)cdiv(entries, (size_t)MSM_L0_ONE * 2 * MSM_SIMDS * 64), 1);
+    }
+    const uint32_t serial = (maxrun + MSM_SERIAL_SPAN - 4) / (MSM_SERIAL_SPAN - 1);
+    L0 = std::max(L0, serial <= 12 ? std::max(serial, 4u) : 4u);
+  }
+  ap.map.L0 = L0;
+  ap.map.n_pad = sh.n_pad;
+  ap.map.lb = 0;
+  while ((1u << ap.map.lb) < sh.B) ap.map.lb++;
+  ap.nchunks = 0;
+  for (int w = 0; w < MSM_MAX_W; w++) {
+    ap.map.first[w] = w < sh.W ? ap.nchunks : UINT32_MAX;
+    if (w < sh.W) ap.nchunks += cdiv(ws.h_stat[2 * w], L0);
+  }
+  ap.max_span = (maxrun + L0 - 2) / L0 + 1;
   return ap;
 }
 
@@ -1732,37 +1769,31 @@ static int msm_accumulate(zk_context* ctx, MsmWorkspace& ws, const MsmShape& sh,
   const uint32_t* end = (const uint32_t*)ws.end.p;
   const uint32_t* wstat = (const uint32_t*)ws.wstat.p;
   xyzz<F>* buckets = (xyzz<F>*)ws.buckets.p;
-  const uint32_t nchunks = ap.nchunks, L0 = ap.L0;
+  const uint32_t nchunks = ap.nchunks;
+  const ChunkMap cm = ap.map;
+  if (nchunks == 0) return ZK_OK;  // all digits zero: every bucket is empty
   ZK_TRY(ctx->ensure(ws.hkey, (size_t)nsets * nchunks * 4));
   ZK_TRY(ctx->ensure(ws.tkey, (size_t)nsets * nchunks * 4));
   ZK_TRY(ctx->ensure(ws.hpt, (size_t)nsets * nchunks * sizeof(xyzz<F>)));
   ZK_TRY(ctx->ensure(ws.tpt, (size_t)nsets * nchunks * sizeof(xyzz<F>)));
   ChunkSlots<F> slots{(uint32_t*)ws.hkey.p, (uint32_t*)ws.tkey.p, (xyzz<F>*)ws.hpt.p, (xyzz<F>*)ws.tpt.p};
-  // lanes per chunk: G1 one, G2 a lane pair, or one for the longest chunks
-  // (the largest G2 MSMs, throughput-bound)
-  const bool one_lane = G2 && ZK_MSM_G2_ONE_LANE && L0 >= (uint32_t)MSM_L0;
-  const uint32_t lanes = one_lane ? 1 : Lanes<F>::N;
+  const uint32_t lanes = ap.one_lane ? 1 : Lanes<F>::N;
   const uint32_t gxl = cdiv((size_t)nchunks * lanes, 256);
-  const uint32_t nwaves = cdiv((size_t)nchunks * lanes, 64);
-  if (one_lane) {
+  if (ap.one_lane) {
     if constexpr (G2) {
       if (sets.pstride)
         ZK_LAUNCH(ctx, st, "msm_accumulate", (k_msm_accumulate<F, true, OneLane<F>>), dim3(gxl, nsets), dim3(256), 0,
-                  sorted, sets, start, end, wstat, nchunks, ap.cpw, sh.n_pad, L0, nbuckets, buckets, slots, nwaves,
-                  wave_scatter(nwaves));
+                  sorted, sets, start, end, wstat, nchunks, cm, nbuckets, buckets, slots);
       else
         ZK_LAUNCH(ctx, st, "msm_accumulate", (k_msm_accumulate<F, false, OneLane<F>>), dim3(gxl, nsets), dim3(256),
-                  0, sorted, sets, start, end, wstat, nchunks, ap.cpw, sh.n_pad, L0, nbuckets, buckets, slots, nwaves,
-                  wave_scatter(nwaves));
+                  0, sorted, sets, start, end, wstat, nchunks, cm, nbuckets, buckets, slots);
     }
   } else if (sets.pstride) {
     ZK_LAUNCH(ctx, st, "msm_accumulate", (k_msm_accumulate<F, true>), dim3(gxl, nsets), dim3(256), 0, sorted, sets,
-              start, end, wstat, nchunks, ap.cpw, sh.n_pad, L0, nbuckets, buckets, slots, nwaves,
-              wave_scatter(nwaves));
+              start, end, wstat, nchunks, cm, nbuckets, buckets, slots);
   } else {
     ZK_LAUNCH(ctx, st, "msm_accumulate", (k_msm_accumulate<F, false>), dim3(gxl, nsets), dim3(256), 0, sorted, sets,
-              start, end, wstat, nchunks, ap.cpw, sh.n_pad, L0, nbuckets, buckets, slots, nwaves,
-              wave_scatter(nwaves));
+              start, end, wstat, nchunks, cm, nbuckets, buckets, slots);
   }
   // The chunk combine and the bucket reduction are chains of dependent
   // additions.  Few of their waves are busy at once (the combine's active
@@ -1784,10 +1815,10 @@ static int msm_accumulate(zk_context* ctx, MsmWorkspace& ws, const MsmShape& sh,
     for (uint64_t step = 1; step < ap.max_span; step *= MSM_COMBINE_S) {
       if (split_combine)
         ZK_LAUNCH(ctx, st, "msm_combine", (k_msm_combine<F, SL>), dim3(gxs, nsets), dim3(256), 0, slots, start, end,
-                  nchunks, L0, (uint32_t)step, nbuckets, buckets);
+                  nchunks, cm, (uint32_t)step, nbuckets, buckets);
       else
         ZK_LAUNCH(ctx, st, "msm_combine", (k_msm_combine<F, Lanes<F>>), dim3(gxs, nsets), dim3(256), 0, slots, start,
-                  end, nchunks, L0, (uint32_t)step, nbuckets, buckets);
+                  end, nchunks, cm, (uint32_t)step, nbuckets, buckets);
     }
   } else if (ap.max_span > 1) {
     const bool tree = ap.max_span > MSM_SERIAL_SPAN + 1;
@@ -1802,19 +1833,19 @@ static int msm_accumulate(zk_context* ctx, MsmWorkspace& ws, const MsmShape& sh,
     }
     if (split_combine)
       ZK_LAUNCH(ctx, st, "msm_combine", (k_msm_combine_serial<F, SL>), dim3(gxs, nsets), dim3(256), 0, slots, end,
-                nchunks, L0, nbuckets, buckets, fcnt, (uint32_t)TB);
+                nchunks, cm, nbuckets, buckets, fcnt, (uint32_t)TB);
     else
       ZK_LAUNCH(ctx, st, "msm_combine", (k_msm_combine_serial<F, Lanes<F>>), dim3(gxs, nsets), dim3(256), 0, slots,
-                end, nchunks, L0, nbuckets, buckets, fcnt, (uint32_t)TB);
+                end, nchunks, cm, nbuckets, buckets, fcnt, (uint32_t)TB);
     if (tree) {
       xyzz<F>* fin = (xyzz<F>*)ws.fin.p;
       xyzz<F>* fout = (xyzz<F>*)ws.fout.p;
       if (split_combine)
         ZK_LAUNCH(ctx, st, "msm_combine", (k_msm_combine_tree<F, SL, TB>), dim3(nblk, nsets), dim3(TB * SL::N), 0,
-                  slots, start, end, nchunks, L0, nbuckets, buckets, fcnt, fin, fout);
+                  slots, start, end, nchunks, cm, nbuckets, buckets, fcnt, fin, fout);
       else
         ZK_LAUNCH(ctx, st, "msm_combine", (k_msm_combine_tree<F, Lanes<F>, TB>), dim3(nblk, nsets),
-                  dim3(TB * Lanes<F>::N), 0, slots, start, end, nchunks, L0, nbuckets, buckets, fcnt, fin, fout);
+                  dim3(TB * Lanes<F>::N), 0, slots, start, end, nchunks, cm, nbuckets, buckets, fcnt, fin, fout);
     }
   }
   return ZK_OK;
@@ -1943,10 +1974,7 @@ static int msm_run_sets(zk_context* ctx, MsmWorkspace& ws, const BaseSets& sets_
       return ctx->fail(ZK_ERR_INVALID, "msm: window table sub-window size");
     sets.pstride = (uint32_t)n;
   }
-  // window regions of the sorted list are padded to the longest chunk, so
-  // every chunk length divides them (the length is chosen after the sort's
-  // counts are known)
-  sh.n_pad = (uint32_t)((sh.n + MSM_L0 - 1) / MSM_L0 * MSM_L0);
+  sh.n_pad = (uint32_t)((sh.n + 63) / 64 * 64);
   // slices per window: about 256 blocks; each slice at least B points, or,
   // for the one bucket space of a window table, at least ZK_MSM_TAB_SLICE
   // (a slice's histogram of B counters is written and scanned once)
@@ -1984,7 +2012,7 @@ static int msm_run_sets(zk_context* ctx, MsmWorkspace& ws, const BaseSets& sets_
   // the windows' entry counts and largest buckets come back while the
   // scatter runs
   ZK_HIP(ctx, hipEventSynchronize(ws.stat_ready));
-  const AccPlan ap = plan_accumulation<F>(ws, sh);
+  const AccPlan ap = plan_accumulation<F>(ws, sh, beside);
   if (ws.gate) {
     int gs;
     while ((gs = ws.gate->state.load()) == 0) std::this_thread::yield();

@@ -471,3 +471,37 @@ def test_msm_wide_window_placement(ctx, g2, n, kind):
     G, gen, from_words = (Z.g2, Z.G2, Z.g2_from_words) if g2 else (Z.g1, Z.G1, Z.g1_from_words)
     got = run(dp, ctx.upload(to_mont(ds)), n)
     assert from_words(got) == G.pmul(gen, closed_form_scalar(kstd, ds))
+
+
+@pytest.mark.parametrize("g2,n", [(False, 1), (False, 300), (False, 65536), (False, 262145), (True, 300),
+                                  (True, 40000), (True, 330001)])
+def test_msm_chunk_plan(ctx, g2, n):
+    """Chunks are numbered over the windows' entries only and their length
+    follows the entry count: no entries at all, one entry, entries in the first
+    and last windows alone, a few whole chunks in every other window, and long
+    uniform lists (330,001 G2 points: one lane per chunk)."""
+    import zkml_amd
+    c, windows = zkml_amd.Context.msm_config(n, g2)
+    rng = np.random.default_rng(n + g2)
+    kstd = rand_std(n, rng)
+    dp = gpu_points(ctx, to_mont(kstd), g2=g2)
+    run = ctx.msm_g2 if g2 else ctx.msm_g1
+    G, gen, from_words = (Z.g2, Z.G2, Z.g2_from_words) if g2 else (Z.g1, Z.G1, Z.g1_from_words)
+    none = np.zeros((n, 4), dtype=np.uint64)
+    one = none.copy()
+    one[n // 2] = std_words([Z.R - 1])[0]
+    ends = none.copy()
+    top = std_words([1 << 252])[0]
+    ends[: n // 2 + 1, 0] = 1 + np.arange(n // 2 + 1, dtype=np.uint64) % np.uint64(100)
+    ends[n // 3:] = top
+    edges = none.copy()
+    for w in range(0, windows - 1, 2):  # window w: 64 (w + 1) entries
+        edges[: min(n, 64 * (w + 1))] |= std_words([1 << (c * w)])[0]
+    for name, s in (("none", none), ("one", one), ("ends", ends), ("edges", edges), ("uniform", rand_std(n, rng))):
+        print(f"[msm chunk plan {'g2' if g2 else 'g1'} {n} c={c}] {name}", flush=True)
+        got = run(dp, ctx.upload(to_mont(s)), n)
+        k = closed_form_scalar(kstd, s)
+        if k == 0:
+            assert not got.any(), name
+        else:
+            assert from_words(got) == G.pmul(gen, k), name
