@@ -1458,15 +1458,20 @@ void msm_workspace_free(MsmWorkspace* ws) {
   delete ws;
 }
 
-// Window size by input size (index: ceil(log2 n)), from measurements on
-// gfx950 with uniform scalars.  Below ~2^19 points the accumulation and the
-// bucket reduction are latency-bound, so fewer buckets pay off well beyond
-// what operation counts suggest; G2 operations are ~3x longer still.
+// Window size by input size (index: ceil(log2 n)), the least sum of the times for
+// uniform and for witness-like scalars (70% below 2^16), which want fewer buckets:
+// their few full windows leave the bucket reduction the larger part.  Measured (us,
+// uniform / witness-like): G1 1000 points 8 bits 245 / 262, 9 bits 240 / 231;
+// 32,768: 9 bits 345 / 309, 10 352 / 349, 13 324 / 439; 65,536: 11 bits 409 / 372,
+// 13 393 / 459; 131,072: 11 bits 527 / 402, 12 518 / 493; 262,144: 11 bits 768 /
+// 492, 13 704 / 570; 400,000: 14 bits 914 / 646, 16 866 / 735.  G2 1000: 8 bits
+// 431 / 454, 10 411 / 446; 65,536: 9 bits 886 / 618, 10 772 / 613, 11 754 / 613;
+// 100,000: 11 bits 921 / 675, 12 897 / 732, 13 864 / 785.
 static int choose_c(size_t n, bool g2) {
   int lg = 0;
   while (((size_t)1 << lg) < n) lg++;
-  static const int g1_table[20] = {8, 8, 8, 8, 8, 8, 8, 8, 8, 8, 8, 8, 8, 9, 9, 10, 11, 12, 13, 14};
-  static const int g2_table[20] = {8, 8, 8, 8, 8, 8, 8, 8, 8, 8, 8, 8, 8, 9, 9, 9, 10, 12, 13, 14};
+  static const int g1_table[20] = {8, 8, 8, 8, 8, 8, 8, 9, 9, 9, 9, 9, 9, 9, 9, 9, 11, 11, 13, 14};
+  static const int g2_table[20] = {8, 8, 8, 8, 8, 8, 8, 8, 8, 8, 10, 10, 10, 10, 10, 11, 11, 11, 13, 14};
   if (lg >= 20) return MSM_CMAX;
   return g2 ? g2_table[lg] : g1_table[lg];
 }
