@@ -116,3 +116,26 @@ def test_pairing_equation(ctx, srs):
     assert np.array_equal(lhs, rhs)
     wrong = g1.padd(C, g1.pneg(g1.pmul(G1, (fzv + 1) % R)))
     assert not np.array_equal(zkml_amd.pairing(_std_point_g1(wrong), _std_point_g2(G2)), rhs)
+
+
+@pytest.mark.parametrize("degree", [4, 5, 6, 1023, 1026, 2049, 4098, 1048577, 1049603])
+def test_open_division_blocks(ctx, degree):
+    """The division scans blocks of 1024 quotient coefficients, four per thread,
+    and the blocks' values the same way: ragged ends of a thread, of a block and
+    of the second level (from 2^20 + 1 coefficients on a third one)."""
+    rng = np.random.default_rng(degree)
+    tau, z = (int(rng.integers(1 << 62)) ** 4 % R for _ in range(2))
+    powers, p = [], MONT % R
+    for _ in range(degree):
+        powers.append(p.to_bytes(32, "little"))
+        p = p * tau % R
+    d_srs = ctx.alloc(degree * 64)
+    ctx.g1_generator_mul(ctx.upload(np.frombuffer(b"".join(powers), dtype=np.uint64).reshape(-1, 4)), degree, d_srs)
+    words = zkml_amd.random_fr(degree, rng)  # Montgomery words
+    raw = [int.from_bytes(w.tobytes(), "little") for w in words]
+    print(f"[kzg division] degree {degree}", flush=True)
+    proof, fz = ctx.kzg_open(d_srs, ctx.upload(words), degree, mont_words([z])[0])
+    ft, fzv = horner(raw, tau), horner(raw, z)
+    assert zkml_amd.words_int(fz) == fzv
+    qt = (ft - fzv) * pow((tau - z) * MONT % R, -1, R) % R
+    assert np.array_equal(proof, gen_points([qt])[0])
