@@ -1687,6 +1687,7 @@ static int msm_sort_wide(zk_context* ctx, MsmWorkspace& ws, const MsmShape& sh, 
 struct AccPlan {
   ChunkMap map;
   uint32_t nchunks;   // chunks of one set
+  uint32_t cap;       // chunks of one set the partials' buffers hold (chunk_bound)
   uint32_t max_span;  // chunks spanned by the largest bucket
   bool one_lane;      // G2 chunks on one lane instead of a pair
 };
@@ -1713,6 +1714,42 @@ struct AccPlan {
 constexpr uint32_t MSM_SIMDS = 1024;  // 256 CUs of 4
 constexpr uint32_t MSM_L0_ONE = 80;   // longest G2 chunk on one lane
 constexpr size_t MSM_ONE_LANE_ENTRIES = 5000000;
+constexpr uint32_t MSM_L0_K1 = 28, MSM_L0_K2 = 48;                    // longest chunks of one and two waves per SIMD
+constexpr uint32_t MSM_L0_MIN = 4;                                    // shortest chunk alone
+constexpr uint32_t MSM_L0_BESIDE_MIN = 8, MSM_L0_BESIDE_MAX = 40;     // beside other jobs
+
+// Waves per SIMD (a multiple of 4) of the lists beyond k = 2, and of the G2 lists
+// on one lane (a multiple of 2).
+static uint32_t full_waves(size_t entries, uint32_t lanes) {
+  return 4 * (uint32_t)cdiv(entries * lanes, (size_t)MSM_L0 * 4 * MSM_SIMDS * 64);
+}
+static uint32_t one_lane_waves(size_t entries) {
+  return 2 * (uint32_t)cdiv(entries, (size_t)MSM_L0_ONE * 2 * MSM_SIMDS * 64);
+}
+
+// Most chunks plan_accumulation makes of a list of this shape, whatever the
+// scalars: the chunk partials' buffers are sized by it, so that only the first
+// call of a size allocates (sized by the chunks themselves, every witness with a
+// few more nonzero digits than any before it freed and allocated four buffers in
+// the middle of a proof).  k grows with the entries, of which there are at most W
+// n, and k's chunks number at most 1024 k waves: one window's last chunk each, at
+// most 32, is made up for by one more entry per chunk (hence the + 1).
+template <class F>
+static uint32_t chunk_bound(const MsmShape& sh, bool beside) {
+  constexpr bool G2 = sizeof(F) != sizeof(fq);
+  constexpr uint32_t N = Lanes<F>::N;
+  const size_t most = (size_t)sh.W * sh.n, wave1 = (size_t)MSM_SIMDS * 64 / N;
+  if (beside)
+    return (uint32_t)std::min((size_t)sh.W * cdiv(sh.n, MSM_L0_BESIDE_MIN),
+                              std::max(wave1, (size_t)cdiv(most, MSM_L0_BESIDE_MAX) + sh.W));
+  const size_t paired = G2 ? std::min(most, MSM_ONE_LANE_ENTRIES) : most;
+  size_t k = 1;
+  if (cdiv(paired, wave1) + 1 > MSM_L0_K1) k = 2;
+  if (cdiv(paired, 2 * wave1) + 1 > MSM_L0_K2) k = full_waves(paired, N);
+  size_t c = k * wave1;
+  if (G2 && most >= MSM_ONE_LANE_ENTRIES) c = std::max(c, (size_t)one_lane_waves(most) * MSM_SIMDS * 64);
+  return (uint32_t)std::min((size_t)sh.W * cdiv(sh.n, MSM_L0_MIN), c);
+}
 
 template <class F>
 static AccPlan plan_accumulation(const MsmWorkspace& ws, const MsmShape& sh, bool beside) {
@@ -1739,16 +1776,16 @@ static AccPlan plan_accumulation(const MsmWorkspace& ws, const MsmShape& sh, boo
   ap.one_lane = false;
   uint32_t L0 = shortest(1, N);
   if (beside) {
-    L0 = std::min(std::max(L0, 8u), 40u);
+    L0 = std::min(std::max(L0, MSM_L0_BESIDE_MIN), MSM_L0_BESIDE_MAX);
   } else {
-    if (L0 > 28) L0 = shortest(2, N);
-    if (L0 > 48) L0 = shortest(4 * (uint32_t)cdiv(entries * N, (size_t)MSM_L0 * 4 * MSM_SIMDS * 64), N);
+    if (L0 > MSM_L0_K1) L0 = shortest(2, N);
+    if (L0 > MSM_L0_K2) L0 = shortest(full_waves(entries, N), N);
     if (G2 && entries >= MSM_ONE_LANE_ENTRIES) {
       ap.one_lane = true;
-      L0 = shortest(2 * (uint32_t)cdiv(entries, (size_t)MSM_L0_ONE * 2 * MSM_SIMDS * 64), 1);
+      L0 = shortest(one_lane_waves(entries), 1);
     }
     const uint32_t serial = (maxrun + MSM_SERIAL_SPAN - 4) / (MSM_SERIAL_SPAN - 1);
-    L0 = std::max(L0, serial <= 12 ? std::max(serial, 4u) : 4u);
+    L0 = std::max(L0, serial <= 12 ? std::max(serial, MSM_L0_MIN) : MSM_L0_MIN);
   }
   ap.map.L0 = L0;
   ap.map.n_pad = sh.n_pad;
@@ -1759,6 +1796,7 @@ static AccPlan plan_accumulation(const MsmWorkspace& ws, const MsmShape& sh, boo
     ap.map.first[w] = w < sh.W ? ap.nchunks : UINT32_MAX;
     if (w < sh.W) ap.nchunks += cdiv(ws.h_stat[2 * w], L0);
   }
+  ap.cap = std::max(ap.nchunks, chunk_bound<F>(sh, beside));
   ap.max_span = (maxrun + L0 - 2) / L0 + 1;
   return ap;
 }
@@ -1776,11 +1814,17 @@ static int msm_accumulate(zk_context* ctx, MsmWorkspace& ws, const MsmShape& sh,
   xyzz<F>* buckets = (xyzz<F>*)ws.buckets.p;
   const uint32_t nchunks = ap.nchunks;
   const ChunkMap cm = ap.map;
+  // chunks per tree block of the combine (36 KB of LDS points)
+  constexpr int TB = G2 ? 128 : 256;
+  const size_t slots_all = (size_t)nsets * ap.cap, blocks_all = (size_t)nsets * cdiv(ap.cap, TB);
+  ZK_TRY(ctx->ensure(ws.hkey, slots_all * 4));
+  ZK_TRY(ctx->ensure(ws.tkey, slots_all * 4));
+  ZK_TRY(ctx->ensure(ws.hpt, slots_all * sizeof(xyzz<F>)));
+  ZK_TRY(ctx->ensure(ws.tpt, slots_all * sizeof(xyzz<F>)));
+  ZK_TRY(ctx->ensure(ws.fcnt, blocks_all * 4));
+  ZK_TRY(ctx->ensure(ws.fin, blocks_all * sizeof(xyzz<F>)));
+  ZK_TRY(ctx->ensure(ws.fout, blocks_all * sizeof(xyzz<F>)));
   if (nchunks == 0) return ZK_OK;  // all digits zero: every bucket is empty
-  ZK_TRY(ctx->ensure(ws.hkey, (size_t)nsets * nchunks * 4));
-  ZK_TRY(ctx->ensure(ws.tkey, (size_t)nsets * nchunks * 4));
-  ZK_TRY(ctx->ensure(ws.hpt, (size_t)nsets * nchunks * sizeof(xyzz<F>)));
-  ZK_TRY(ctx->ensure(ws.tpt, (size_t)nsets * nchunks * sizeof(xyzz<F>)));
   ChunkSlots<F> slots{(uint32_t*)ws.hkey.p, (uint32_t*)ws.tkey.p, (xyzz<F>*)ws.hpt.p, (xyzz<F>*)ws.tpt.p};
   const uint32_t lanes = ap.one_lane ? 1 : Lanes<F>::N;
   const uint32_t gxl = cdiv((size_t)nchunks * lanes, 256);
@@ -1827,15 +1871,8 @@ static int msm_accumulate(zk_context* ctx, MsmWorkspace& ws, const MsmShape& sh,
     }
   } else if (ap.max_span > 1) {
     const bool tree = ap.max_span > MSM_SERIAL_SPAN + 1;
-    constexpr int TB = G2 ? 128 : 256;  // chunks per tree block (36 KB of LDS points)
     const uint32_t nblk = cdiv(nchunks, TB);
-    uint32_t* fcnt = nullptr;
-    if (tree) {
-      ZK_TRY(ctx->ensure(ws.fcnt, (size_t)nsets * nblk * 4));
-      ZK_TRY(ctx->ensure(ws.fin, (size_t)nsets * nblk * sizeof(xyzz<F>)));
-      ZK_TRY(ctx->ensure(ws.fout, (size_t)nsets * nblk * sizeof(xyzz<F>)));
-      fcnt = (uint32_t*)ws.fcnt.p;
-    }
+    uint32_t* fcnt = tree ? (uint32_t*)ws.fcnt.p : nullptr;
     if (split_combine)
       ZK_LAUNCH(ctx, st, "msm_combine", (k_msm_combine_serial<F, SL>), dim3(gxs, nsets), dim3(256), 0, slots, end,
                 nchunks, cm, nbuckets, buckets, fcnt, (uint32_t)TB);

@@ -104,3 +104,89 @@ def test_pk_window_table_allocation_failure_falls_back(tmp_path):
     finally:
         _fail_at(0)
         ctx.close()
+
+
+@pytest.mark.parametrize("g2,n", [(False, 1000), (False, 40000), (False, 300007), (True, 9000), (True, 70001)])
+def test_msm_allocates_only_on_the_first_call_of_a_size(g2, n):
+    """After one MSM of a size, other scalars of that size need no device
+    memory: the workspaces follow the size, not the scalars' digit counts.  No
+    entries at all first, then a few, then witness-like, uniform and equal
+    scalars (one hot bucket in every window), each with the next allocation
+    armed to fail, against the closed form."""
+    import zkml_amd
+    import zkpy as Z
+    from test_gpu_msm import closed_form_scalar, gpu_points, rand_std, to_mont, witness_like
+    ctx = zkml_amd.Context(0)
+    try:
+        rng = np.random.default_rng(n + g2)
+        kstd = rand_std(n, rng)
+        dp = gpu_points(ctx, to_mont(kstd), g2=g2)
+        run = ctx.msm_g2 if g2 else ctx.msm_g1
+        G, gen, from_words = (Z.g2, Z.G2, Z.g2_from_words) if g2 else (Z.g1, Z.G1, Z.g1_from_words)
+        none = np.zeros((n, 4), dtype=np.uint64)
+        few = none.copy()
+        few[:: max(1, n // 50)] = rand_std(len(few[:: max(1, n // 50)]), rng)
+        equal = np.repeat(rand_std(1, rng), n, axis=0)
+        assert not run(dp, ctx.upload(to_mont(none)), n).any()
+        for name, s in (("few", few), ("witness", witness_like(n, rng)), ("uniform", rand_std(n, rng)),
+                        ("equal", equal)):
+            print(f"[msm allocations {'g2' if g2 else 'g1'} {n}] {name}", flush=True)
+            ds = ctx.upload(to_mont(s))
+            _fail_at(1)
+            got = run(dp, ds, n)
+            _fail_at(0)
+            assert from_words(got) == G.pmul(gen, closed_form_scalar(kstd, s)), name
+    finally:
+        _fail_at(0)
+        ctx.close()
+
+
+@pytest.mark.parametrize("rows", [5000, 20000])
+def test_proofs_of_one_circuit_allocate_only_once(rows, tmp_path):
+    """Proofs of one circuit (x_i^2 = y_i) with other witnesses than the first
+    proof's (few entries, small values, uniform values) need no device memory
+    of their own, plain MSMs (5000 rows) and window tables (20,000): each with
+    the next allocation armed to fail gives the proof of a fresh context."""
+    import zkml_amd
+    import zkpy as Z
+    from r1cs_gen import Circuit
+    from test_gpu_groth16 import PROVE_SEED, SETUP_SEED
+    rng = np.random.default_rng(rows)
+    nv = 1 + 2 * rows  # 1, then x_i, then y_i
+    xs = [(i, 1 + i, 1) for i in range(rows)]
+    circ = Circuit(rows, nv, 1, nv - 2, xs, xs, [(i, 1 + rows + i, 1) for i in range(rows)], None)
+    mats = circ.mats()
+
+    def witness(kind):
+        x = [0] * rows
+        for i in range(0, rows, 100 if kind == "few" else 1):
+            x[i] = int(rng.integers(1, 1 << 15)) if kind == "small" else int(rng.integers(1, 1 << 62)) ** 5 % Z.R
+        circ.w = [1] + x + [v * v % Z.R for v in x]
+        return circ.witness_words()
+
+    pk_path, vk_path = str(tmp_path / "pk.bin"), str(tmp_path / "vk.bin")
+    proofs, ws = {}, {k: witness(k) for k in ("few", "small", "uniform")}
+    for fresh in (False, True):
+        for kind in (("few", "small", "uniform") if not fresh else ("small", "uniform")):
+            if fresh or kind == "few":
+                ctx = zkml_amd.Context(0)
+                r = ctx.r1cs(rows, nv, 1, *mats)
+                if not proofs:
+                    ctx.setup(r, SETUP_SEED, pk_path, vk_path)
+                pk = ctx.load_pk(pk_path)
+            print(f"[proof allocations] {rows} rows, {kind}, {'fresh context' if fresh else 'kept context'}",
+                  flush=True)
+            try:
+                _fail_at(0 if fresh or kind == "few" else 1)
+                proof, _ = ctx.prove(pk, r, ws[kind], 1, PROVE_SEED)
+            finally:
+                _fail_at(0)
+            if not fresh:
+                proofs[kind] = proof
+            else:
+                assert proof == proofs[kind], kind
+            if fresh or kind == "uniform":
+                pk.close()
+                r.close()
+                ctx.close()
+    assert len(set(proofs.values())) == 3
