@@ -1707,7 +1707,11 @@ struct AccPlan {
 // in 24 windows 32 -> 24 entries 443 -> 405, 100,000 in 20 windows 32 -> 16 455 ->
 // 448, in 24 windows 32 -> 20 563 -> 478; G2 62,779 in 24 windows 32 -> 24 842 -> 742.
 // Beside other jobs (a proof), whose waves fill the SIMDs, k = 1 and 8 to 40
-// entries: a 2^16 proof 1057 -> 1044, one of 200,001 rows 2984 -> 2840.
+// entries: a 2^16 proof 1057 -> 1044, one of 200,001 rows 2984 -> 2840.  From 10
+// million entries 64, and G2 on one lane, as long lists alone: there the partials
+// cost more than the SIMDs' last waves.  Proofs with 40 / with 64 on one lane (ms):
+// 700,001 rows (9 million entries) 7.65 / 7.73, 1,046,576 (14) 9.93 / 9.90,
+// 2,095,152 (27) 18.8 / 18.2, 4,192,304 (54) 37.8 / 35.7 (64 on a pair 36.1).
 // Alone, few points take chunks of 4: 1000 points 243 -> 235.  A length of up to 12
 // at which the largest bucket spans few enough chunks for the serial combine is
 // preferred to a shorter one (10,000 points: 8 entries 293, 10 280).
@@ -1717,6 +1721,7 @@ constexpr size_t MSM_ONE_LANE_ENTRIES = 5000000;
 constexpr uint32_t MSM_L0_K1 = 28, MSM_L0_K2 = 48;                    // longest chunks of one and two waves per SIMD
 constexpr uint32_t MSM_L0_MIN = 4;                                    // shortest chunk alone
 constexpr uint32_t MSM_L0_BESIDE_MIN = 8, MSM_L0_BESIDE_MAX = 40;     // beside other jobs
+constexpr size_t MSM_BESIDE_LONG_ENTRIES = 10000000;
 
 // Waves per SIMD (a multiple of 4) of the lists beyond k = 2, and of the G2 lists
 // on one lane (a multiple of 2).
@@ -1739,9 +1744,11 @@ static uint32_t chunk_bound(const MsmShape& sh, bool beside) {
   constexpr bool G2 = sizeof(F) != sizeof(fq);
   constexpr uint32_t N = Lanes<F>::N;
   const size_t most = (size_t)sh.W * sh.n, wave1 = (size_t)MSM_SIMDS * 64 / N;
-  if (beside)
+  if (beside) {
+    const size_t below = cdiv(std::min(most, MSM_BESIDE_LONG_ENTRIES), MSM_L0_BESIDE_MAX);
     return (uint32_t)std::min((size_t)sh.W * cdiv(sh.n, MSM_L0_BESIDE_MIN),
-                              std::max(wave1, (size_t)cdiv(most, MSM_L0_BESIDE_MAX) + sh.W));
+                              std::max(wave1, std::max<size_t>(below, cdiv(most, MSM_L0)) + sh.W));
+  }
   const size_t paired = G2 ? std::min(most, MSM_ONE_LANE_ENTRIES) : most;
   size_t k = 1;
   if (cdiv(paired, wave1) + 1 > MSM_L0_K1) k = 2;
@@ -1775,7 +1782,10 @@ static AccPlan plan_accumulation(const MsmWorkspace& ws, const MsmShape& sh, boo
   AccPlan ap;
   ap.one_lane = false;
   uint32_t L0 = shortest(1, N);
-  if (beside) {
+  if (beside && entries >= MSM_BESIDE_LONG_ENTRIES) {
+    ap.one_lane = G2;
+    L0 = MSM_L0;
+  } else if (beside) {
     L0 = std::min(std::max(L0, MSM_L0_BESIDE_MIN), MSM_L0_BESIDE_MAX);
   } else {
     if (L0 > MSM_L0_K1) L0 = shortest(2, N);

@@ -292,3 +292,27 @@ def test_prove_2_22_config5_verifies(ctx, tmp_path):
         assert ref().ref_verify_files(str(vk_path).encode(), str(pf).encode(), str(pubf).encode()) == 1
     pk.close()
     r.close()
+
+
+@pytest.mark.parametrize("nc", [769180, 769300])
+def test_prove_around_long_lists(ctx, tmp_path, nc):
+    """The witness queries' lists on both sides of 10 million entries (13 of
+    each of nc + 21 variables), from which a proof's chunks hold 64 entries and
+    take one lane over G2; H's list is above it.  The verifier accepts the
+    proof, and not another public input."""
+    import zkml_amd
+    npub = 4
+    A, B, C, w = zkml_amd.synthetic_r1cs(nc, npub, 16, 11)
+    r = ctx.r1cs(nc, w.shape[0], npub, A, B, C)
+    pk_path, vk_path = tmp_path / "pk.bin", tmp_path / "vk.bin"
+    print(f"[prove long lists] nc={nc} domain 2^{r.log_n}", flush=True)
+    ctx.setup(r, SETUP_SEED, pk_path, vk_path)
+    pk = ctx.load_pk(pk_path)
+    proof, _ = ctx.prove(pk, r, w, npub, PROVE_SEED)
+    pub = [Z.from_mont(Z.from_limbs([int(x) for x in w[1 + i]]), Z.R) for i in range(npub)]
+    pub_words = np.array([Z.limbs(v) for v in pub], dtype=np.uint64)
+    assert zkml_amd.verify(vk_path.read_bytes(), proof, pub_words)
+    pub_words[0, 0] ^= 1
+    assert not zkml_amd.verify(vk_path.read_bytes(), proof, pub_words)
+    pk.close()
+    r.close()
