@@ -131,6 +131,24 @@ static size_t tot_capacity(size_t n) {
   return t;
 }
 
+// Whether the fold may read [p, p + bytes) in place: one device allocation of
+// this context's GPU that is known to hold all of it, at an address its 16-byte
+// loads take.  (About a microsecond on the host; a copy of the coefficients is a
+// launch and a pass over them.)
+static bool readable_in_place(const zk_context* ctx, const void* p, size_t bytes) {
+  if ((uintptr_t)p % 16) return false;
+  hipPointerAttribute_t at;
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  const bool known = hipPointerGetAttributes(&at, p) == hipSuccess && at.type == hipMemoryTypeDevice &&
+                     at.device == ctx->device &&
+                     hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) == hipSuccess;
+  (void)hipGetLastError();  // an address the runtime does not know is an answer, not this call's failure
+  if (!known) return false;
+  const size_t off = (size_t)((const uint8_t*)p - (const uint8_t*)base);
+  return off <= size && bytes <= size - off;
+}
+
 static fr fr_internal(const uint64_t mont[4]) {
   uint32_t w[8];
   memcpy(w, mont, 32);
@@ -172,8 +190,14 @@ static int zk_kzg_open_impl(zk_context* ctx, const void* d_srs_g1, const void* d
   ZK_TRY(ctx->ensure(ctx->scratch_b, nq * 32));
   ZK_TRY(ctx->ensure(ctx->scratch_c, tot_capacity(nq) * 32 + 64));
   uint4* q = (uint4*)ctx->scratch_b.p;
-  // f_1 .. f_{d-1}
-  ZK_TRY(suffix_horner(ctx, (const uint4*)d_coeffs + 2, q, nq, fr_internal(zm), (uint4*)ctx->scratch_c.p, st));
+  // f_1 .. f_{d-1}: read in place, or as the runtime's copy takes them (other
+  // memory than this GPU's, other alignments) or refuses them (a buffer too short)
+  const uint4* f1 = (const uint4*)d_coeffs + 2;
+  if (!readable_in_place(ctx, d_coeffs, degree * 32)) {
+    ZK_HIP(ctx, hipMemcpyAsync(q, (const uint8_t*)d_coeffs + 32, nq * 32, hipMemcpyDeviceToDevice, st));
+    f1 = q;
+  }
+  ZK_TRY(suffix_horner(ctx, f1, q, nq, fr_internal(zm), (uint4*)ctx->scratch_c.p, st));
   if (f_z) {
     // to pinned memory, read after the MSM has waited for the stream: a copy to
     // pageable memory and a wait of its own held the MSM's launches back

@@ -139,3 +139,45 @@ def test_open_division_blocks(ctx, degree):
     assert zkml_amd.words_int(fz) == fzv
     qt = (ft - fzv) * pow((tau - z) * MONT % R, -1, R) % R
     assert np.array_equal(proof, gen_points([qt])[0])
+
+
+def _open_raw(ctx, d_srs, coeffs_ptr, degree, z):
+    """zk_kzg_open through the C ABI, the coefficients at any address."""
+    import ctypes
+    out, fz = np.zeros(8, dtype=np.uint64), np.zeros(4, dtype=np.uint64)
+    zw = mont_words([z])[0].copy()
+    rc = zkml_amd.lib().zk_kzg_open(ctx.h, ctypes.c_void_p(d_srs.ptr), ctypes.c_void_p(coeffs_ptr), degree, ptr(zw),
+                                    ptr(out), ptr(fz), None)
+    return rc, out, fz
+
+
+@pytest.mark.parametrize("degree", [2, 33, 1500])
+def test_open_takes_coefficients_where_the_copy_did(ctx, srs, degree):
+    """Coefficients that the division does not read in place go through the
+    runtime's copy: at an address that is a multiple of 8 only, and in host
+    memory.  Same proof and value as from a device buffer."""
+    _, pts = srs
+    rng = random.Random(degree)
+    f, z = [rng.randrange(R) for _ in range(degree)], rng.randrange(R)
+    d_srs = ctx.upload(pts[:degree])
+    words = mont_words(f)
+    want, fz = ctx.kzg_open(d_srs, ctx.upload(words), degree, mont_words([z])[0])
+    assert zkml_amd.words_int(fz) * pow(MONT, -1, R) % R == horner(f, z)
+    shifted = ctx.upload(np.concatenate([np.zeros(1, dtype=np.uint64), words.reshape(-1)]))
+    for name, at in (("shifted", shifted.ptr + 8), ("host", words.ctypes.data)):
+        print(f"[kzg coefficients] degree {degree} {name}", flush=True)
+        rc, out, got_fz = _open_raw(ctx, d_srs, at, degree, z)
+        assert rc == 0, name
+        assert np.array_equal(out, want) and np.array_equal(got_fz, fz), name
+
+
+def test_open_refuses_a_coefficient_buffer_shorter_than_the_degree(ctx, srs):
+    """A degree beyond the buffer's end is refused (the runtime checks the copy's
+    range), not read.  The buffer ends inside a page, so that even an unchecked
+    read of one coefficient more would stay in mapped memory."""
+    _, pts = srs
+    d_srs, d_f = ctx.upload(pts[:128]), ctx.upload(mont_words(list(range(1, 101))))
+    rc, _, _ = _open_raw(ctx, d_srs, d_f.ptr, 101, 5)
+    assert rc != 0
+    rc, _, _ = _open_raw(ctx, d_srs, d_f.ptr, 100, 5)
+    assert rc == 0
