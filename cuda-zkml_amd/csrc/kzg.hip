@@ -176,7 +176,6 @@ static int zk_kzg_open_impl(zk_context* ctx, const void* d_srs_g1, const void* d
   if (!ctx || !h_proof || !z || (degree && (!d_srs_g1 || !d_coeffs))) return ZK_ERR_INVALID;
   if (degree > MSM_MAX_N + 1) return ctx->fail(ZK_ERR_SIZE, "kzg: degree above the MSM limit");
   hipStream_t st = ctx->s(stream);
-  const uint64_t* zm = z;
   if (degree <= 1) {  // constant polynomial: the proof is the identity (groth16.cu:414-416)
     memset(h_proof, 0, 64);
     if (f_z) {
@@ -187,6 +186,7 @@ static int zk_kzg_open_impl(zk_context* ctx, const void* d_srs_g1, const void* d
     return ZK_OK;
   }
   const size_t nq = degree - 1;
+  const fr zi = fr_internal(z);  // read before anything is written: z may lie in h_proof or f_z
   ZK_TRY(ctx->ensure(ctx->scratch_b, nq * 32));
   ZK_TRY(ctx->ensure(ctx->scratch_c, tot_capacity(nq) * 32 + 64));
   uint4* q = (uint4*)ctx->scratch_b.p;
@@ -197,7 +197,7 @@ static int zk_kzg_open_impl(zk_context* ctx, const void* d_srs_g1, const void* d
     ZK_HIP(ctx, hipMemcpyAsync(q, (const uint8_t*)d_coeffs + 32, nq * 32, hipMemcpyDeviceToDevice, st));
     f1 = q;
   }
-  ZK_TRY(suffix_horner(ctx, f1, q, nq, fr_internal(zm), (uint4*)ctx->scratch_c.p, st));
+  ZK_TRY(suffix_horner(ctx, f1, q, nq, zi, (uint4*)ctx->scratch_c.p, st));
   if (f_z) {
     // to pinned memory, read after the MSM has waited for the stream: a copy to
     // pageable memory and a wait of its own held the MSM's launches back
@@ -214,7 +214,7 @@ static int zk_kzg_open_impl(zk_context* ctx, const void* d_srs_g1, const void* d
     uint32_t a[8], b[8], out[8];
     memcpy(a, ctx->h_words, 32);
     memcpy(b, ctx->h_words + 4, 32);
-    repack_out(fadd(repack_in<FrP>(a), fmul(repack_in<FrP>(b), fr_internal(zm))), out);
+    repack_out(fadd(repack_in<FrP>(a), fmul(repack_in<FrP>(b), zi)), out);
     memcpy(f_z, out, 32);
   }
   return ZK_OK;

@@ -181,3 +181,23 @@ def test_open_refuses_a_coefficient_buffer_shorter_than_the_degree(ctx, srs):
     assert rc != 0
     rc, _, _ = _open_raw(ctx, d_srs, d_f.ptr, 100, 5)
     assert rc == 0
+
+
+def test_open_with_z_in_the_result_buffers(ctx, srs):
+    """z may share its words with the proof or with f(z): it is read before
+    they are written."""
+    import ctypes
+    _, pts = srs
+    rng = random.Random(9)
+    degree = 300
+    f, z = [rng.randrange(R) for _ in range(degree)], rng.randrange(R)
+    d_srs, d_f = ctx.upload(pts[:degree]), ctx.upload(mont_words(f))
+    want, fz = ctx.kzg_open(d_srs, d_f, degree, mont_words([z])[0])
+    for shared in ("proof", "value"):
+        out, got = np.zeros(8, dtype=np.uint64), np.zeros(4, dtype=np.uint64)
+        zw = out[2:6] if shared == "proof" else got
+        zw[:] = mont_words([z])[0]
+        rc = zkml_amd.lib().zk_kzg_open(ctx.h, ctypes.c_void_p(d_srs.ptr), ctypes.c_void_p(d_f.ptr), degree, ptr(zw),
+                                        ptr(out), ptr(got), None)
+        assert rc == 0
+        assert np.array_equal(out, want) and np.array_equal(got, fz), shared
