@@ -8,21 +8,21 @@
 // and results leave the device as canonical affine points.
 //
 // All functions are generic over the coordinate field F (fq or fq2) through
-// the overloads fmul/fsqr/fadd/fsub/fis_zero/fdbl below.
+// the overloads fmul/fsqr/fis_zero and the like below.
 //
-// Two forms of each operation.  The *_lx forms, which the MSM kernels run, leave
-// X in (0, 6m) ("lazy X") instead of reducing it: X3 = R^2 - PPP - 2Q + 4m is one
-// carry pass, where the reduced form adds two conditional subtractions (about
-// 90 of a mixed addition's 2300 instructions, a third of them selects).  X is
-// only ever a product's operand or subtracted with an offset, so no other step
-// changes its cost.  Y, ZZ, ZZZ stay below 2m.  The plain forms take and give
-// coordinates below 2m.  Bounds, per coordinate and in units of m (a product
+// The *_lx forms leave X in (0, 6m) ("lazy X") instead of reducing it: X3 = R^2 -
+// PPP - 2Q + 4m is one carry pass, where a reduced X3 takes two conditional
+// subtractions more (about 90 of a mixed addition's 2300 instructions, a third of
+// them selects).  X is only ever a product's operand or subtracted with an offset,
+// so no other step changes its cost.  Y, ZZ, ZZZ stay below 2m.  xyzz_madd gives X
+// below 2m, too.  Bounds, per coordinate and in units of m (a product
 // of a and b is below ab / 169.2 + 1.0000003; an Fq2 product is one of sums
 // a0 b0 + (4 - a1) b1 with a the reduced factor; an Fq2 square (a0 + a1)(a0 -
 // a1 + 8) and (2 a0) a1):
-//   mixed addition: U2, S2 < 1.1; P = U2 - X + 6 in (0, 7), R = S2 - Y + 2 in
-//   (0, 3.3); P^2 < 2.2, R^2 < 1.5; PPP, Q < 1.2; X3 = R^2 - PPP - 2Q + 4 in (0.4,
-//   5.6); Q - X3 + 6 in (0.4, 6.9), so Y3 < 1.5; ZZ3, ZZZ3 < 1.1.
+//   mixed addition: U2, S2 < 1.1; P = U2 - X + 6 in (0, 7.1), R = S2 - Y + 2 in
+//   (0, 3.1); P^2 < 1.8, R^2 < 1.4; PPP, Q < 1.25 (Fq2: 1 + (1.73 + 4) 7.1 / 169.2);
+//   X3 = R^2 - PPP - 2Q + 4 in (0.25, 5.4); Q - X3 + 6 in (0.6, 7), so Y3 < 1.5; ZZ3,
+//   ZZZ3 < 1.1.
 //   addition: P, R in (0, 4), P^2, R^2 < 1.4, then as above.
 //   doubling: U = 2Y < 4, V = U^2 < 1.4, W, S < 1.2, X^2 < 1.99, M = 3 X^2 < 6,
 //   M^2 < 1.99, X3 = M^2 - 2S + 4 in (1.6, 6), S - X3 + 6 in (0, 5.6), Y3 < 1.6.
@@ -38,10 +38,6 @@ struct fq2 {
   fq c0, c1;
 };
 
-ZK_HD fq2 fadd(const fq2& a, const fq2& b) { return fq2{fadd(a.c0, b.c0), fadd(a.c1, b.c1)}; }
-ZK_HD fq2 fsub(const fq2& a, const fq2& b) { return fq2{fsub(a.c0, b.c0), fsub(a.c1, b.c1)}; }
-ZK_HD fq2 fdbl(const fq2& a) { return fq2{fdbl(a.c0), fdbl(a.c1)}; }
-ZK_HD fq2 fneg(const fq2& a) { return fq2{fneg(a.c0), fneg(a.c1)}; }
 ZK_HD fq fneg_canon_if(const fq& a, bool neg) { return fneg_canon_if<FqP>(a, neg); }
 ZK_HD fq2 fneg_canon_if(const fq2& a, bool neg) { return fq2{fneg_canon_if(a.c0, neg), fneg_canon_if(a.c1, neg)}; }
 // (a0 + a1 u)(b0 + b1 u) = (a0 b0 - a1 b1) + (a0 b1 + a1 b0) u, each
@@ -217,19 +213,7 @@ ZK_HD void xyzz_add_lx(xyzz<F>& p, const xyzz<F>& q) {
   p.y = fmul_sub(R, fsub_x(qq, p.x), s1, ppp);
 }
 
-// The same operations with every coordinate reduced below 2m.
-template <class F>
-ZK_HD void xyzz_mdbl(xyzz<F>& p, const F& x, const F& y) {
-  xyzz_mdbl_lx(p, x, y);
-  p.x = freduce_x(p.x);
-}
-
-template <class F>
-ZK_HD void xyzz_dbl(xyzz<F>& p) {
-  xyzz_dbl_lx(p);
-  p.x = freduce_x(p.x);
-}
-
+// p += (x2, y2) affine and finite, every coordinate below 2m.
 template <class F>
 ZK_HD void xyzz_madd(xyzz<F>& p, const F& x2, const F& y2) {
   if (xyzz_is_inf(p)) {
@@ -238,17 +222,6 @@ ZK_HD void xyzz_madd(xyzz<F>& p, const F& x2, const F& y2) {
   }
   (void)xyzz_madd_fin_lx(p, x2, y2);
   p.x = freduce_x(p.x);
-}
-
-template <class F>
-ZK_HD void xyzz_add(xyzz<F>& p, const xyzz<F>& q) {
-  xyzz_add_lx(p, q);
-  p.x = freduce_x(p.x);
-}
-
-template <class F>
-ZK_HD void xyzz_neg(xyzz<F>& p) {
-  p.y = fneg(p.y);
 }
 
 // a^-1 = a^(q-2) (Fermat); Fq2 through the norm: (c0 - c1 u) / (c0^2 + c1^2)

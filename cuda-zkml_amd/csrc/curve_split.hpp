@@ -38,10 +38,6 @@ __device__ __forceinline__ fq fsel(bool odd, const fq& a, const fq& b) {
   return r;
 }
 
-__device__ __forceinline__ fq2h fadd(const fq2h& a, const fq2h& b) { return fq2h{fadd(a.c, b.c)}; }
-__device__ __forceinline__ fq2h fsub(const fq2h& a, const fq2h& b) { return fq2h{fsub(a.c, b.c)}; }
-__device__ __forceinline__ fq2h fdbl(const fq2h& a) { return fq2h{fdbl(a.c)}; }
-__device__ __forceinline__ fq2h fneg(const fq2h& a) { return fq2h{fneg(a.c)}; }
 __device__ __forceinline__ fq2h fneg_canon_if(const fq2h& a, bool neg) { return fq2h{fneg_canon_if(a.c, neg)}; }
 __device__ __forceinline__ fq2h fsub_m(const fq2h& a, const fq2h& b) { return fq2h{fsub_lazy(a.c, b.c)}; }
 __device__ __forceinline__ fq2h fsub_x(const fq2h& a, const fq2h& b) { return fq2h{fsub_off<6>(a.c, b.c)}; }
@@ -64,7 +60,11 @@ __device__ __forceinline__ void fset_one(fq2h& a) { a.c = lane_odd() ? fe_zero<F
 
 // The even / odd lane's coordinate on both lanes of the pair (DPP quad_perm
 // [0, 0, 2, 2] and [1, 1, 3, 3]).  The operations below take their operands by
-// these moves and by negations under a lane mask instead of selects.
+// these moves and by negations under a lane mask instead of selects.  (A move may
+// read a register two wait states after its write at the earliest, and the
+// compiler does not see the writes inside a product's assembly block: the limbs go
+// in order, the block writes the last ones last.  A test looks at every move of
+// the built library.)
 template <int CTRL>
 __device__ __forceinline__ fq dpp_fq(const fq& a) {
   fq r;
@@ -221,11 +221,6 @@ __device__ __forceinline__ void xyzz_set_inf(xyzz_half<E>& p) {
 template <class E>
 __device__ __forceinline__ bool xyzz_is_inf(const xyzz_half<E>& p) {
   return fis_zero(p.b);
-}
-
-template <class E>
-__device__ __forceinline__ void xyzz_neg(xyzz_half<E>& p) {
-  if (split_role1<E>()) p.a = fneg(p.a);
 }
 
 // p = 2p (dbl-2008-s-1): X^2 | V = U^2, S = X V | W = U V, M^2 and X3 on both,

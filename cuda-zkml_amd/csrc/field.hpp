@@ -7,7 +7,7 @@
 // radix inside kernels is R' = 2^261 (= 2^(29*9)), not the reference's 2^256:
 // with 29-bit limbs every limb product is one v_mad_u64_u32 into a 64-bit
 // column accumulator and no carry has to be propagated until the column is
-// finished (18 products of < 2^60 plus a 2^35 carry stay below 2^64).  On
+// finished (mont_columns_fit below: at most 61 of 2^64's 64 units of 2^58).  On
 // gfx950 the 32x32->64 mad issues at full rate, so the instruction count of
 // the multiply is what matters; this layout needs 169 mads and 22 other ops
 // (a square 133 and 30) against ~560 instructions for a compiler-lowered
@@ -500,11 +500,6 @@ ZK_HD fe<P> fneg(const fe<P>& a) {
   return fsub(fe_zero<P>(), a);
 }
 
-template <class P>
-ZK_HD fe<P> fdbl(const fe<P>& a) {
-  return fadd(a, a);
-}
-
 // a + b with carries and no reduction: normalized limbs, value in [0, 4m) for
 // a, b in [0, 2m).
 template <class P>
@@ -584,21 +579,6 @@ ZK_HD fe<P> fcsub(const fe<P>& t, const uint32_t (&K)[NL]) {
   return fselect(br != 0, t, u);
 }
 
-// (a - b - 2c) mod m into [0, 2m) for a, b, c in [0, 2m): one pass forms
-// a + 6m - b - 2c in (0, 8m), then two conditional subtractions of 4m, 2m.
-template <class P>
-ZK_HD fe<P> fsub3(const fe<P>& a, const fe<P>& b, const fe<P>& c) {
-  fe<P> t;
-  int32_t cy = 0;
-#pragma unroll
-  for (int i = 0; i < NL; i++) {
-    int32_t v = (int32_t)a.l[i] + (int32_t)P::MOD6[i] - (int32_t)b.l[i] - 2 * (int32_t)c.l[i] + cy;
-    cy = v >> 29;
-    t.l[i] = (uint32_t)v & LMASK;
-  }
-  return fcsub(fcsub(t, P::MOD4), P::MOD2);
-}
-
 // a - b - 2c + 4m, exact (normalized limbs), for a value that stays positive:
 // b + 2c < 4m.
 template <class P>
@@ -642,21 +622,6 @@ ZK_HD fe<P> fneg_lazy6(const fe<P>& a) {
   return d;
 }
 
-// a - b + 4m for a in [0, 4m), b in [0, 4m]: value in (0, 8m), normalized
-// limbs.  Valid only as an fmul / fsqr input.
-template <class P>
-ZK_HD fe<P> fsub_lazy4(const fe<P>& a, const fe<P>& b) {
-  fe<P> d;
-  int32_t c = 0;
-#pragma unroll
-  for (int i = 0; i < NL; i++) {
-    int32_t v = (int32_t)a.l[i] + (int32_t)P::MOD4[i] - (int32_t)b.l[i] + c;
-    c = v >> 29;
-    d.l[i] = (uint32_t)v & LMASK;
-  }
-  return d;
-}
-
 // mask ? KM*m - a : a with carries (mask all ones or zero; KM = 2 or 6, a <= KM*m).
 template <int KM, class P>
 ZK_HD fe<P> fneg_mask(const fe<P>& a, uint32_t mask) {
@@ -667,20 +632,6 @@ ZK_HD fe<P> fneg_mask(const fe<P>& a, uint32_t mask) {
 #pragma unroll
   for (int i = 0; i < NL; i++) {
     int32_t v = (int32_t)((a.l[i] ^ mask) + (mask & (K[i] + 1u))) + c;
-    c = v >> 29;
-    d.l[i] = (uint32_t)v & LMASK;
-  }
-  return d;
-}
-
-// 4m - a for a in [0, 4m]: value in [0, 4m], normalized limbs.
-template <class P>
-ZK_HD fe<P> fneg_lazy4(const fe<P>& a) {
-  fe<P> d;
-  int32_t c = 0;
-#pragma unroll
-  for (int i = 0; i < NL; i++) {
-    int32_t v = (int32_t)P::MOD4[i] - (int32_t)a.l[i] + c;
     c = v >> 29;
     d.l[i] = (uint32_t)v & LMASK;
   }

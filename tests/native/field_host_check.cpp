@@ -34,9 +34,9 @@ int fh_op(int op, const uint32_t* a, const uint32_t* b, const uint32_t* c, const
     case 5: r = fadd(A, B); break;
     case 6: r = fsub(A, B); break;
     case 7: r = fmul_sub(A, B, C, D); break;
-    case 9: r = fsub3<FqP>(A, B, C); break;
-    case 10: r = fsub_lazy4<FqP>(A, B); break;
-    case 11: r = fneg_lazy4<FqP>(A); break;
+    case 9: r = freduce_x(fsub_off<4>(fsub_lazy(A, B), fadd_wide(C, C))); break;  // a - b - 2c
+    case 10: r = fsub_off<4>(A, B); break;
+    case 11: r = fsub_off<4>(fe_zero<FqP>(), A); break;
     case 12: r = fe_zero<FqP>(); r.l[0] = fis_zero<FqP>(A) ? 1u : 0u; break;
     case 13: r = fe_zero<FqP>(); r.l[0] = fis_zero4<FqP>(A) ? 1u : 0u; break;
     case 14: r = fadd_wide(A, B); break;
@@ -74,19 +74,20 @@ int fh_fr_op(int op, const uint32_t* a, const uint32_t* b, uint32_t* out) {
   return 0;
 }
 
-// XYZZ operations; G1 points are 36 words (x, y, zz, zzz), G2 points 72.
+// XYZZ operations, X reduced below 2q afterwards; G1 points are 36 words (x, y,
+// zz, zzz), G2 points 72.
 // op 0: p += (qx, qy) affine   1: p += q   2: p = 2p   3: p = 2 (qx, qy)
 int fh_xyzz(int g2, int op, const uint32_t* p, const uint32_t* q, uint32_t* out) {
   if (!g2) {
     xyzz<fq> P{ld(p), ld(p + 9), ld(p + 18), ld(p + 27)}, Q{ld(q), ld(q + 9), ld(q + 18), ld(q + 27)};
     switch (op) {
       case 0: xyzz_madd(P, Q.x, Q.y); break;
-      case 1: xyzz_add(P, Q); break;
-      case 2: xyzz_dbl(P); break;
-      case 3: xyzz_mdbl(P, Q.x, Q.y); break;
+      case 1: xyzz_add_lx(P, Q); break;
+      case 2: xyzz_dbl_lx(P); break;
+      case 3: xyzz_mdbl_lx(P, Q.x, Q.y); break;
       default: return -1;
     }
-    st(out, P.x);
+    st(out, freduce_x(P.x));
     st(out + 9, P.y);
     st(out + 18, P.zz);
     st(out + 27, P.zzz);
@@ -94,12 +95,12 @@ int fh_xyzz(int g2, int op, const uint32_t* p, const uint32_t* q, uint32_t* out)
     xyzz<fq2> P{ld2(p), ld2(p + 18), ld2(p + 36), ld2(p + 54)}, Q{ld2(q), ld2(q + 18), ld2(q + 36), ld2(q + 54)};
     switch (op) {
       case 0: xyzz_madd(P, Q.x, Q.y); break;
-      case 1: xyzz_add(P, Q); break;
-      case 2: xyzz_dbl(P); break;
-      case 3: xyzz_mdbl(P, Q.x, Q.y); break;
+      case 1: xyzz_add_lx(P, Q); break;
+      case 2: xyzz_dbl_lx(P); break;
+      case 3: xyzz_mdbl_lx(P, Q.x, Q.y); break;
       default: return -1;
     }
-    st2(out, P.x);
+    st2(out, freduce_x(P.x));
     st2(out + 18, P.y);
     st2(out + 36, P.zz);
     st2(out + 54, P.zzz);

@@ -7,14 +7,16 @@ limb, carry or range assumption fails here before any kernel runs:
 
   fmul / fsqr / fmul_sum  a*b*2^-261 (sums of 2 and 4 products) mod q, result < 2q, limbs < 2^29,
                           at the edges of the documented input ranges
-  fsub_lazy / fneg_lazy   exact a - b + 2q and 2q - a (and the 4q forms)
-  fsub3, fis_zero(4)      a - b - 2c into [0, 2q); zero tests over [0, 2q) / [0, 4q)
+  fsub_lazy / fneg_lazy   exact a - b + 2q and 2q - a; a - b + 4q (fsub_off)
+  freduce_x, fis_zero(4)  a - b - 2c into [0, 2q); zero tests over [0, 2q) / [0, 4q)
   fadd / fsub / fmul_sub  congruence and the [0, 2q) output range
   fadd_wide / fcsub       exact a + b below 4q; a - 2q when a >= 2q
-  NTT lazy butterfly      over Fr: X, Y in [0, 4r) give X' +- Y*w in [0, 4r)
+  NTT                     over Fr: the offset subtractions and reductions, products
+                          by constants, three-stage steps without carry passes
   XYZZ madd/add/dbl/mdbl  G1 and G2 against affine formulas, with coordinates
                           given in non-canonical [q, 2q) representatives and
-                          random Z, plus the doubling / inverse / infinity cases
+                          random Z, plus the doubling / inverse / infinity cases;
+                          the lazy-X forms at the edges of their ranges
 """
 import ctypes
 import os
@@ -148,9 +150,10 @@ def fr_op(fh, code, a, b=0):
 
 
 def test_ntt_lazy_butterfly_bounds(fh):
-    """The NTT's lazy radix-2 step: inputs X, Y in [0, 4r), a canonical
-    twiddle w; T = Y*w (Montgomery), X' = X mod 2r, outputs X' + T and
-    X' - T + 2r must stay in [0, 4r) and be congruent to X +- Y*w/R'."""
+    """A lazy radix-2 step from the helpers over Fr: inputs X, Y in [0, 4r), a
+    canonical w; T = Y*w (Montgomery), X' = X mod 2r, outputs X' + T and
+    X' - T + 2r must stay in [0, 4r) and be congruent to X +- Y*w/R'.  (The
+    passes' own steps: test_ntt_step_without_carries.)"""
     rng = random.Random(12)
     r = ORDER
     rinv = pow(RP, -1, r)
@@ -190,10 +193,11 @@ def test_ntt_offset_subtract_and_reduce(fh):
 
 
 def test_ntt_grow_butterfly_chain(fh):
-    """The pass kernel's arithmetic on one element path: a first radix-8 step
-    with twiddle-free butterflies (offsets 2r, 4r, 8r) and five twiddled
-    stages (u + w v, u - w v + 2r, no reduction) keep normalized limbs and
-    values below 26r, congruent to the exact result; freduce finishes."""
+    """A first radix-8 step with the pass kernel's twiddle-free butterflies
+    (offsets 2r, 4r, 8r), then five stages by Montgomery products (u + w v,
+    u - w v + 2r, no reduction), keep normalized limbs and values below 26r,
+    congruent to the exact result; freduce finishes.  (The passes' twiddled
+    stages: test_ntt_step_without_carries.)"""
     rng = random.Random(22)
     r = ORDER
     rinv = pow(RP, -1, r)
