@@ -557,8 +557,8 @@ int zk_quotient_h(zk_context* ctx, const zk_r1cs* c, const void* d_witness, size
 // 2^ZK_PK_TAB_MIN_LOG .. 2^ZK_PK_TAB_MAX_LOG scalars.  The digit windows of a
 // table MSM share one bucket space, so wider windows cost no reduction per
 // window: 16 windows of 16 bits (or 20 of 13), against 24-26 windows of 10-11
-// bits in the plain MSMs at 2^16 points, reduced in sub-windows of 2^SUB
-// buckets.  A table holds W copies of its query.  Measured on the 2^16 proof
+// bits in the plain MSMs at 2^16 points, reduced as one window of up to 2^15
+// buckets (more of them above 2^18 scalars).  A table holds W copies of its query.  Measured on the 2^16 proof
 // (config 4): 1.63 -> 1.45 ms with W = 16 for the witness G1 sets (A, B1, L
 // share one sort) and W = 20 for B2 and H (a 16-bit single window sorts
 // slower, and H's sort runs beside the other MSMs' accumulations); 2^13

@@ -47,7 +47,7 @@ namespace zk {
 
 constexpr uint32_t KEY_INVALID = 0xffffffffu;
 constexpr int MSM_MAX_W = 32;   // windows of the narrowest window (8 bits)
-constexpr int MSM_L0 = 64;         // sorted entries per accumulation thread (largest)
+constexpr int MSM_L0 = 64;         // longest chunk of sorted entries (G2 on one lane: MSM_L0_ONE)
 constexpr int MSM_CMAX = 16;       // widest window: 2^15 LDS counters (128 KB)
 constexpr uint32_t MSM_LDS_B = 32768;  // most buckets a window's slice histogram holds in LDS
 constexpr int SORT_T = 1024;       // threads of the histogram / scatter blocks
@@ -163,8 +163,6 @@ __device__ __forceinline__ void std_to_coord(const uint32_t* e, fq2& a) {
   a.c1 = from_std<FqP>(e + 8);
 }
 
-// External points (zk_g1_affine / zk_g2_affine: Montgomery R = 2^256, x = y =
-// 0 for infinity) -> records.
 // Issue priority of the MSM's waves.  Inside a proof several MSMs and the
 // quotient share the GPU.  The accumulation is throughput-bound and always
 // ready to issue; the digit sort and the chunk combine are short or
@@ -178,9 +176,9 @@ template <class F>
 __device__ __forceinline__ void msm_priority() {
   msm_short_priority();
 }
-// The bucket reduction stays at priority 0: its kernels take 100 registers a
-// lane on split lanes, so another job's accumulation waves fit beside them on a
-// SIMD, and at priority 2 they starved there (a 2^13 proof's H accumulation took
+// The bucket reduction stays at priority 0: its kernels take 95 to 127 registers
+// a lane (k_msm_rowcol over G2 137 to 149), so another job's accumulation waves
+// fit beside them on a SIMD, and at priority 2 they starved there (a 2^13 proof's H accumulation took
 // 135 us instead of 43; the proof 0.54 instead of 0.49 ms).
 __device__ __forceinline__ void msm_reduce_priority() { __builtin_amdgcn_s_setprio(0); }
 // The G2 accumulation is the longest throughput phase of a proof and starts
@@ -190,6 +188,8 @@ __device__ __forceinline__ void msm_accumulate_priority() {
   if constexpr (sizeof(F) == sizeof(fq2)) __builtin_amdgcn_s_setprio(1);
 }
 
+// External points (zk_g1_affine / zk_g2_affine: Montgomery R = 2^256, x = y =
+// 0 for infinity) -> records.
 template <class F>
 __global__ void k_msm_convert(uint4* __restrict__ recs, const uint32_t* __restrict__ ext, size_t n) {
   size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;

@@ -364,8 +364,8 @@ __device__ __forceinline__ void tile_copy_out(const TileCtx& tc, const PassGeo& 
 
 // ---- fixed-geometry tiles: the elements stay in registers between steps
 // and move through LDS in two halves (limbs 0-4, then 5-8) over five planes,
-// so a 2048-element tile takes 50 KB of LDS instead of 83 KB and three
-// blocks fit on a CU where one would.
+// so a 2048-element tile takes 50 KB of LDS instead of 83 KB: room for three
+// blocks on a CU (two run, by registers) where one would fit.
 constexpr int NTT_XPLANES = 5;
 
 // LDS rows of a step of K stages starting at stage s: group gi of the
@@ -855,8 +855,8 @@ struct NttCall {
   NttTile tile;
 };
 
-// Tiles of 2048 elements take 78 KB of LDS: above the 64 KB a launch may
-// request by default.
+// Tiles of 2048 elements in nine planes take 83 KB of LDS: above the 64 KB a
+// launch may request by default.
 static void ntt_lds_limits() {
   static std::once_flag once;
   std::call_once(once, [] {

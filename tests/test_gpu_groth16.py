@@ -194,8 +194,8 @@ def test_prove_window_table_shapes(ctx, tmp_path, nc):
     """Proofs whose MSMs run on the proving key's window tables at each shape
     boundary (m = nc + 21 variables): 2^14..2^15 (20 windows of 13 bits for
     every query, a 2^14 domain),
-    up to 2^18 (16-bit windows for the witness sets, 13-bit for B2 and H;
-    sub-windows of 2^10 and 2^8 buckets) and just above 2^18 (13 windows of
+    up to 2^18 (16-bit windows for the witness sets, 13-bit for B2 and H; one
+    window of 2^15 or 2^12 buckets to reduce) and just above 2^18 (13 windows of
     19-20 bits through the two-level wide sort, 2^15-bucket sub-windows).
     Byte-identical to the oracle's prove on the same key and seed."""
     import zkml_amd

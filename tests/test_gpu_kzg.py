@@ -9,7 +9,8 @@ Pins (closed forms over an SRS built from a known tau, [tau^i]_1 = tau^i G1):
   the pairing equation e(C - f(z) G1, G2) = e(proof, [tau]_2 - z G2) holds
   (host pairing), and fails for a wrong f(z);
   degrees 0 and 1 give the identity proof (the reference's rule); the sizes
-  cross the blocked scan's chunk (32) and recursion (32^2, 32^3) edges.
+  cross the edges of the blocked scan's threads (4 values), blocks (1024) and
+  levels (2^20).
 The expected points come from the oracle's CPU fixed-base multiply.
 """
 import random

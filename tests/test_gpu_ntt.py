@@ -131,7 +131,7 @@ def test_ntt_rejects_bad_sizes(ctx):
                                          (18, 1), (18, 2), (18, 3), (12, 256), (8, 4096), (19, 3)])
 def test_ntt_tile_rule(ctx, log_n, batch):
     """Transforms on both sides of every limit of the tile rule (elements of the
-    call: 2^16, 2^18, 2^20), and batches that reach them with small transforms:
+    call: 2^16, 2^17, 2^20), and batches that reach them with small transforms:
     the first, a middle and the last transform of the batch, forward, inverse
     and inverse coset, against the oracle."""
     n = 1 << log_n
