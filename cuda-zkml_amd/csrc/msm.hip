@@ -1467,9 +1467,14 @@ void msm_workspace_free(MsmWorkspace* ws) {
 // 492, 13 704 / 570; 400,000: 14 bits 914 / 646, 16 866 / 735.  G2 1000: 8 bits
 // 431 / 454, 10 411 / 446; 65,536: 9 bits 886 / 618, 10 772 / 613, 11 754 / 613;
 // 100,000: 11 bits 921 / 675, 12 897 / 732, 13 864 / 785.
-static int choose_c(size_t n, bool g2) {
+// Beside other jobs (a proof) a G2 product below 2^14 points takes 8 bits: its
+// windows then reduce in one launch, and those chains end the proof (uniform
+// witnesses, 10 bits / 8: 700 rows 525 / 465, 2000 542 / 492, 6000 603 / 539, 12,000
+// 642 / 635; a quantized MLP of 1993 rows 421 / 419, 5965 468 / 455, 7933 472 / 462).
+static int choose_c(size_t n, bool g2, bool beside = false) {
   int lg = 0;
   while (((size_t)1 << lg) < n) lg++;
+  if (beside && g2 && n < ((size_t)1 << 14)) return 8;
   static const int g1_table[20] = {8, 8, 8, 8, 8, 8, 8, 9, 9, 9, 9, 9, 9, 9, 9, 9, 11, 11, 13, 14};
   static const int g2_table[20] = {8, 8, 8, 8, 8, 8, 8, 8, 8, 8, 10, 10, 10, 10, 10, 11, 11, 11, 13, 14};
   if (lg >= 20) return MSM_CMAX;
@@ -2008,7 +2013,7 @@ static int msm_run_sets(zk_context* ctx, MsmWorkspace& ws, const BaseSets& sets_
   MsmShape sh;
   int Wd;  // digit windows
   if (!tab) {
-    const int c = choose_c(n, G2);
+    const int c = choose_c(n, G2, beside);
     Wd = (MSM_BITS + c - 1) / c;
     sh.n = n;
     sh.W = Wd;

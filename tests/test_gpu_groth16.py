@@ -189,10 +189,11 @@ def test_prove_2_16_matches_oracle(ctx, tmp_path):
         assert ref().ref_verify_files(str(vk_path).encode(), str(pf).encode(), str(pub).encode()) == 1
 
 
-@pytest.mark.parametrize("nc", [(1 << 14) - 8, (1 << 18) - 64, (1 << 18) + 64])
+@pytest.mark.parametrize("nc", [(1 << 14) - 22, (1 << 14) - 8, (1 << 18) - 64, (1 << 18) + 64])
 def test_prove_window_table_shapes(ctx, tmp_path, nc):
     """Proofs whose MSMs run on the proving key's window tables at each shape
-    boundary (m = nc + 21 variables): 2^14..2^15 (20 windows of 13 bits for
+    boundary (m = nc + 21 variables): just below 2^14 (no tables but H's, B2 in
+    windows of 8 bits), 2^14..2^15 (20 windows of 13 bits for
     every query, a 2^14 domain),
     up to 2^18 (16-bit windows for the witness sets, 13-bit for B2 and H; one
     window of 2^15 or 2^12 buckets to reduce) and just above 2^18 (13 windows of
