@@ -1465,7 +1465,7 @@ void msm_workspace_free(MsmWorkspace* ws) {
 // 32,768: 9 bits 345 / 309, 10 352 / 349, 13 324 / 439; 65,536: 11 bits 409 / 372,
 // 13 393 / 459; 131,072: 11 bits 527 / 402, 12 518 / 493; 262,144: 11 bits 768 /
 // 492, 13 704 / 570; 400,000: 14 bits 914 / 646, 16 866 / 735.  G2 1000: 8 bits
-// 431 / 454, 10 411 / 446; 65,536: 9 bits 886 / 618, 10 772 / 613, 11 754 / 613;
+// 431 / 454, 10 411 / 446 (2000 points of 12 bits: 8 bits 370, 10 432); 65,536: 9 bits 886 / 618, 10 772 / 613, 11 754 / 613;
 // 100,000: 11 bits 921 / 675, 12 897 / 732, 13 864 / 785.
 // Beside other jobs (a proof) a G2 product below 2^14 points takes 8 bits: its
 // windows then reduce in one launch, and those chains end the proof (uniform
@@ -1719,12 +1719,18 @@ struct AccPlan {
 // 2,095,152 (27) 18.8 / 18.2, 4,192,304 (54) 37.8 / 35.7 (64 on a pair 36.1).
 // Alone, few points take chunks of 4: 1000 points 243 -> 235.  A length of up to 12
 // at which the largest bucket spans few enough chunks for the serial combine is
-// preferred to a shorter one (10,000 points: 8 entries 293, 10 280).
+// preferred to a shorter one (10,000 points: 8 entries 293, 10 280).  So is one at
+// which it takes the level combine instead of the tree, or, where that is longer
+// than 12, one at which a full window's ordinary buckets take the serial one: among
+// other entries (a bucket of more than half of them is what the tree is for) short
+// chunks hand hundreds of ordinary buckets to the tree, too.  Chunks of 4 / by this
+// rule: G2 10,000 points of 12 bits 575 / 462, 16,000 746 / 486, 32,000 756 / 583,
+// 8000 points, half of them 1, 697 / 619; G1 16,000 of 12 bits 334 / 249.
 constexpr uint32_t MSM_SIMDS = 1024;  // 256 CUs of 4
 constexpr uint32_t MSM_L0_ONE = 80;   // longest G2 chunk on one lane
 constexpr size_t MSM_ONE_LANE_ENTRIES = 5000000;
 constexpr uint32_t MSM_L0_K1 = 28, MSM_L0_K2 = 48;                    // longest chunks of one and two waves per SIMD
-constexpr uint32_t MSM_L0_MIN = 4;                                    // shortest chunk alone
+constexpr uint32_t MSM_L0_MIN = 4, MSM_L0_SERIAL = 12;                 // shortest chunk alone; longest one chosen for the combine
 constexpr uint32_t MSM_L0_BESIDE_MIN = 8, MSM_L0_BESIDE_MAX = 40;     // beside other jobs
 constexpr size_t MSM_BESIDE_LONG_ENTRIES = 10000000;
 
@@ -1800,7 +1806,14 @@ static AccPlan plan_accumulation(const MsmWorkspace& ws, const MsmShape& sh, boo
       L0 = shortest(one_lane_waves(entries), 1);
     }
     const uint32_t serial = (maxrun + MSM_SERIAL_SPAN - 4) / (MSM_SERIAL_SPAN - 1);
-    L0 = std::max(L0, serial <= 12 ? std::max(serial, MSM_L0_MIN) : MSM_L0_MIN);
+    L0 = std::max(L0, serial <= MSM_L0_SERIAL ? std::max(serial, MSM_L0_MIN) : MSM_L0_MIN);
+    // the tree combine, and more to combine than one bucket
+    if (maxrun > 1 + L0 * (MSM_TREE_SPAN - 1) && entries > 2 * (size_t)maxrun) {
+      const uint32_t levels = cdiv(maxrun - 1, MSM_TREE_SPAN - 1);  // the level combine's longest span
+      const uint32_t mean = (uint32_t)(sh.n / sh.B);                // a full window's buckets: up to about 2 mean
+      const uint32_t full = cdiv(2 * mean + 4, MSM_SERIAL_SPAN - 1);
+      L0 = std::max(L0, levels <= MSM_L0_SERIAL ? levels : std::min(full, MSM_L0_SERIAL));
+    }
   }
   ap.map.L0 = L0;
   ap.map.n_pad = sh.n_pad;

@@ -505,3 +505,25 @@ def test_msm_chunk_plan(ctx, g2, n):
             assert not got.any(), name
         else:
             assert from_words(got) == G.pmul(gen, k), name
+
+
+@pytest.mark.parametrize("g2,n,kind", [(False, 6000, "half"), (False, 24000, "12 bits"), (False, 24000, "half"),
+                                       (True, 4500, "half"), (True, 16000, "12 bits"), (True, 32000, "12 bits")])
+def test_msm_long_buckets_among_others(ctx, g2, n, kind):
+    """Few entries, and a largest bucket that chunks of 4 would make span more
+    than 512 of them, among ordinary buckets: the chunk length is the level
+    combine's, or the serial combine's for the ordinary buckets with the tree for
+    the long ones (G1 24,000 points, half of them 1; G2 32,000 of 12 bits)."""
+    rng = np.random.default_rng(n + g2)
+    kstd = rand_std(n, rng)
+    dp = gpu_points(ctx, to_mont(kstd), g2=g2)
+    s = rand_std(n, rng)
+    if kind == "half":
+        s[: n // 2] = 0
+        s[: n // 2, 0] = 1
+    else:
+        s[:] = 0
+        s[:, 0] = rng.integers(0, 1 << 12, n, dtype=np.uint64)
+    run = ctx.msm_g2 if g2 else ctx.msm_g1
+    G, gen, from_words = (Z.g2, Z.G2, Z.g2_from_words) if g2 else (Z.g1, Z.G1, Z.g1_from_words)
+    assert from_words(run(dp, ctx.upload(to_mont(s)), n)) == G.pmul(gen, closed_form_scalar(kstd, s))
